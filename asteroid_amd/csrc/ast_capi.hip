@@ -1144,7 +1144,7 @@ int class_batch_update(ast_ctx* c, int k, const std::vector<DevJob*>& members) {
 }
 
 // One fit-kernel launch of class k over the class batch, on its stream.
-hipError_t launch_class(ast_ctx* c, int k, const DevJob& j0) {
+hipError_t launch_class(ast_ctx* c, int k, const DevJob& j0, int lanes) {
   LaunchArgs a{};
   a.op = 1;
   a.stream = c->streams[stream_of(k)];
@@ -1157,13 +1157,14 @@ hipError_t launch_class(ast_ctx* c, int k, const DevJob& j0) {
   a.group_size = c->pool.G;
   a.n_filters = j0.n_filters;
   a.waves = c->waves[k];
+  a.lanes = lanes;
   return dispatch(j0.space.v, a);
 }
 
 // The cycle as a HIP graph: every class launch, forked from stream 0 onto
 // the classes' streams and joined back.  Valid while the class batches, the
 // pool and the register budgets are unchanged (the key).
-int cycle_graph(ast_ctx* c, std::vector<DevJob*>* members, const bool* used_s) {
+int cycle_graph(ast_ctx* c, std::vector<DevJob*>* members, const bool* used_s, int lanes) {
   std::vector<uint64_t> key{(uint64_t)(uintptr_t)c->pool.X, (uint64_t)c->pool.nf, (uint64_t)c->pool.G};
   for (int k = 0; k < MAX_CLASSES; ++k) {
     if (members[k].empty()) continue;
@@ -1183,7 +1184,7 @@ int cycle_graph(ast_ctx* c, std::vector<DevJob*>* members, const bool* used_s) {
   for (int k = 1; k < NSTREAMS && e == hipSuccess; ++k)
     if (used_s[k]) e = hipStreamWaitEvent(c->streams[k], c->ev_fork, 0);
   for (int k = 0; k < MAX_CLASSES && e == hipSuccess; ++k)
-    if (!members[k].empty()) e = launch_class(c, k, *members[k][0]);
+    if (!members[k].empty()) e = launch_class(c, k, *members[k][0], lanes);
   for (int k = 1; k < NSTREAMS && e == hipSuccess; ++k)
     if (used_s[k]) {
       e = hipEventRecord(c->ev_join[k], c->streams[k]);
@@ -1206,6 +1207,7 @@ int cycle_graph(ast_ctx* c, std::vector<DevJob*>* members, const bool* used_s) {
 int run_cycle_once(ast_ctx* c, std::vector<DevJob*>& jobs, double* kernel_ms, int* launches, bool graphs) {
   std::vector<DevJob*> members[MAX_CLASSES];
   bool used_s[NSTREAMS] = {false};
+  int64_t fits = 0;
   for (DevJob* j : jobs) {
     if (job_complete(*j)) continue;
     if (!job_fits_pool(*j, c->pool)) {
@@ -1214,7 +1216,9 @@ int run_cycle_once(ast_ctx* c, std::vector<DevJob*>& jobs, double* kernel_ms, in
     }
     members[j->cls].push_back(j);
     used_s[stream_of(j->cls)] = true;
+    fits += (int64_t)j->n_workers * c->pool.G;
   }
+  const int lanes = lanes_per_model(fits);  // the classes of a cycle run side by side
   int n_cls = 0;
   for (int k = 0; k < MAX_CLASSES; ++k)
     if (!members[k].empty()) {
@@ -1225,7 +1229,7 @@ int run_cycle_once(ast_ctx* c, std::vector<DevJob*>& jobs, double* kernel_ms, in
   std::vector<int32_t> done(jobs.size());
   if (graphs && n_cls > 0) {
     // one graph launch on stream 0; every class stream joins back into it
-    RETIF(cycle_graph(c, members, used_s));
+    RETIF(cycle_graph(c, members, used_s, lanes));
     const hipStream_t s0 = c->streams[0];
     // The graph runs on stream 0, but a job's init kernel and clears were
     // queued on its class's stream: stream 0 waits for them, or the first
@@ -1248,7 +1252,7 @@ int run_cycle_once(ast_ctx* c, std::vector<DevJob*>& jobs, double* kernel_ms, in
       if (used_s[k]) HIPCHK(hipEventRecord(c->ev0[k], c->streams[k]));
     for (int k = 0; k < MAX_CLASSES; ++k) {
       if (members[k].empty()) continue;
-      HIPCHK(launch_class(c, k, *members[k][0]));
+      HIPCHK(launch_class(c, k, *members[k][0], lanes));
       (*launches)++;
     }
     for (int k = 0; k < NSTREAMS; ++k)

@@ -779,6 +779,35 @@ AST_AI void begin_rotation(const double* params, int k, double Is_inv, double Ii
   }
 }
 
+enum { FORM_CHI2 = 0, FORM_PLOT = 1, FORM_RMSD = 2 };
+
+// A model's score from its per-filter sums, and delta_V (cuda.c:884-910; with
+// NUDGE the merit of its minima, cuda.c:912-992).
+template <class CF, int VC, int NF, int FORM>
+AST_AI CF model_score(const double* sy2, const double* sy, int n_filters, int dof, const double* sum_w, CF* dV,
+                      const NudgeState* nu, TailPtr mr) {
+  CF chi2a = 0.0;
+  CF sum_all = 0.0;
+#pragma unroll
+  for (int m = 0; m < NF; ++m) {
+    if (m < n_filters) {
+      CF chi2m = sy2[m] - sy[m] * sy[m] / sum_w[m];
+      chi2a = chi2a + chi2m;
+      dV[m] = sy[m] / sum_w[m];
+      if constexpr (FORM == FORM_RMSD) sum_all = sum_all + sum_w[m];
+    }
+  }
+  if constexpr (FORM == FORM_RMSD) {
+    // the root is taken in double: rounded to float it is the correctly
+    // rounded float root
+    chi2a = (CF)__builtin_sqrt((double)(chi2a / sum_all));
+  } else {
+    chi2a = chi2a / dof;
+  }
+  if constexpr (VarF<VC>::NU) chi2a = nu->merit<CF>(chi2a, dV[0], mr);
+  return chi2a;
+}
+
 // chi^2 of one model (chi2one, cuda.c:81-1011, in-scope branches), summed
 // per filter; NF is the compile-time filter capacity (>= n_filters).  With MX
 // (the mixed-precision form) the Euler angles and angular velocity are
@@ -790,7 +819,6 @@ AST_AI void begin_rotation(const double* params, int k, double Is_inv, double Ii
 // point's Vmod + dv0 goes to vplot[i * vstride], nothing is summed and the
 // result is 0; FORM_RMSD (the RMSD build, cuda.c:890-906), the root of the
 // summed filter chi^2 over the summed weights.
-enum { FORM_CHI2 = 0, FORM_PLOT = 1, FORM_RMSD = 2 };
 template <class CF, int VC, int NF, bool MX = false, int FORM = FORM_CHI2>
 __device__ CF chi2_model(const double* params, PointPtr pts, int n_data, int n_filters, int dof,
                          const double* sum_w, CF* dV, double* vplot = nullptr, size_t vstride = 0,
@@ -998,26 +1026,7 @@ __device__ CF chi2_model(const double* params, PointPtr pts, int n_data, int n_f
   // A failed NUDGE model returns before delta_V is written (cuda.c:737).
   if constexpr (NU)
     if (nu.failed) return CF(1e30);
-  CF chi2a = 0.0;  // cuda.c:884-910
-  CF sum_all = 0.0;
-#pragma unroll
-  for (int m = 0; m < NF; ++m) {
-    if (m < n_filters) {
-      CF chi2m = sy2[m] - sy[m] * sy[m] / sum_w[m];
-      chi2a = chi2a + chi2m;
-      dV[m] = sy[m] / sum_w[m];
-      if constexpr (FORM == FORM_RMSD) sum_all = sum_all + sum_w[m];
-    }
-  }
-  if constexpr (FORM == FORM_RMSD) {
-    // the root is taken in double: rounded to float it is the correctly
-    // rounded float root
-    chi2a = (CF)__builtin_sqrt((double)(chi2a / sum_all));
-  } else {
-    chi2a = chi2a / dof;
-  }
-  if constexpr (NU) chi2a = nu.merit<CF>(chi2a, dV[0], mr);
-  return chi2a;
+  return model_score<CF, VC, NF, FORM>(sy2, sy, n_filters, dof, sum_w, dV, NU ? &nu : nullptr, mr);
 }
 
 }  // namespace ast

@@ -22,6 +22,7 @@
 // HBM between launches.
 #pragma once
 #include "ast_device.h"
+#include "ast_rows.h"
 
 namespace ast {
 
@@ -593,6 +594,116 @@ __global__ __launch_bounds__(64) void group_best_kernel(const CF* fit_f, const d
   }
 }
 
+// ----------------------------------------------------------------- stage end
+// The end of a stage, by the whole workgroup (one thread per simplex of the
+// group, all of which finished the stage; cuda.c:1739-1823): the block argmin,
+// then either the next stage's reseed (the lanes are left at PH_START, true)
+// or the best-per-group write and the fits' own results (false).
+template <class CF, int VC>
+__device__ bool group_stage_end(const GroupDesc<CF>& D, const Machine<CF, VC>& M, LaneRegs<CF>& R, int t, int G,
+                                int& stage, int& reopt) {
+  constexpr int N = Pos<VC>::N;
+  __shared__ CF s_f[1024];
+  __shared__ CF s_x0[MAXP];
+  __shared__ int s_tm;
+  __shared__ CF s_smin;
+  const Space<CF>& sp = M.sp;
+  s_f[t] = R.sf;
+  __syncthreads();
+  if (t == 0) {
+    int tm = 0;
+    CF smin = (CF)1e30;
+    for (int k = 0; k < G; ++k)
+      if (s_f[k] < smin) { smin = s_f[k]; tm = k; }
+    s_tm = tm;
+    s_smin = smin;
+  }
+  __syncthreads();
+  const int tm = s_tm;
+  const CF smin = s_smin;
+  if (D.nstages > 1 && stage < D.nstages - 1) {
+    if (t == tm) {
+      CF xb[N];
+      const int b = M.IND(0);
+#pragma unroll
+      for (int i = 0; i < N; ++i) xb[i] = M.X(b, i);
+      if (sp.p_psi && reopt == 0) {  // cuda.c:1791-1798
+        double prm[N];
+#pragma unroll
+        for (int i = 0; i < N; ++i) prm[i] = M.PRM(i);
+        x2params_at<CF, VC>(xb, prm, sp, reopt);
+        params2x<CF, VC>(xb, prm, sp);
+#pragma unroll
+        for (int i = 0; i < N; ++i) { M.PRM(i) = prm[i]; M.X(b, i) = xb[i]; }
+      }
+#pragma unroll
+      for (int i = 0; i < N; ++i) s_x0[i] = xb[i];
+    }
+    __syncthreads();
+    reopt = 1;
+    stage++;
+#pragma unroll
+    for (int i = 0; i < N; ++i) M.X(0, i) = s_x0[i];
+    R.phase = PH_START;
+    return true;
+  }
+  const int g = D.group_in_job;
+  if (t == tm && smin < D.best_f[g]) {  // cuda.c:1810-1823
+    D.best_f[g] = smin;
+    CF xb[N];
+    double prm[N];
+    const int b = M.IND(0);
+#pragma unroll
+    for (int i = 0; i < N; ++i) { xb[i] = M.X(b, i); prm[i] = M.PRM(i); }
+    x2params_at<CF, VC>(xb, prm, sp, reopt);
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+      M.PRM(i) = prm[i];
+      D.best_params[(size_t)g * N + i] = prm[i];
+    }
+    for (int m = 0; m < D.n_filters; ++m)
+      D.best_dV[(size_t)g * D.n_filters + m] = M.B.DV[(size_t)m * M.rs + M.fo];
+  }
+  D.fit_f[M.jfit] = R.sf;
+  D.fit_nev[M.jfit] = R.nev_tot;
+  D.fit_steps[M.jfit] = R.steps_tot;
+  stage++;
+  R.phase = PH_FIT_DONE;
+  return false;
+}
+
+// A lane's machine state, from and to its slot.
+template <class CF>
+__device__ inline LaneRegs<CF> load_lane(const SlotBufs<CF>& B, size_t fit, size_t fo, uint32_t rng) {
+  LaneRegs<CF> R;
+  const int ctl = B.ctl[fit];
+  R.phase = ctl & 15;
+  R.j = (ctl >> 4) & 63;
+  R.failed = (ctl >> 10) & 1;
+  R.bad = (ctl >> 11) & 1;
+  R.l = B.lstep[fit];
+  R.nev = B.nev[fit];
+  R.nev_tot = B.nev_tot[fit];
+  R.steps_tot = B.steps_tot[fit];
+  R.work = B.work[fit];
+  R.rng = rng;
+  R.fr = B.fr[fo];
+  R.sf = B.sf[fo];
+  return R;
+}
+template <class CF>
+__device__ inline void store_lane(const SlotBufs<CF>& B, size_t fit, size_t fo, const LaneRegs<CF>& R, uint64_t jfit) {
+  B.ctl[fit] = R.phase | (R.j << 4) | (R.failed << 10) | (R.bad << 11);
+  B.lstep[fit] = R.l;
+  B.nev[fit] = R.nev;
+  B.nev_tot[fit] = R.nev_tot;
+  B.steps_tot[fit] = R.steps_tot;
+  B.work[fit] = R.work;
+  B.fitid[fit] = (int32_t)jfit;
+  B.fr[fo] = R.fr;
+  B.sf[fo] = R.sf;
+}
+
 // ---------------------------------------------------------------- fit kernel
 // One workgroup = one group (the reference's block); it runs D.ticks rounds
 // of "evaluate the pending points, advance every lane", then saves its state.
@@ -607,10 +718,6 @@ void fit_kernel(const GroupDesc<CF>* descs, SlotBufs<CF> B) {
   using P = Pos<VC>;
   AST_VFLAGS(VC);
   constexpr int N = P::N;
-  __shared__ CF s_f[1024];
-  __shared__ CF s_x0[MAXP];
-  __shared__ int s_tm;
-  __shared__ CF s_smin;
   constexpr int KC = 8 / sizeof(CF);
   const GroupDesc<CF>& D = descs[blockIdx.x];
   const int t = threadIdx.x;
@@ -623,23 +730,10 @@ void fit_kernel(const GroupDesc<CF>* descs, SlotBufs<CF> B) {
   uint64_t jfit = (uint64_t)B.fitid[fit];  // group_in_job * G + t unless the lane has refilled
   const Space<CF>& sp = *D.sp;
   const StageCfg<CF> SC{D.seed, D.size2_min, D.n_steps, D.eval_budget};
-  const int nstages = D.nstages, ticks = D.ticks;
+  const int ticks = D.ticks;
   int reopt = B.g_reopt[slot];
   int stage = B.g_stage[slot];
-  LaneRegs<CF> R;
-  const int ctl = B.ctl[fit];
-  R.phase = ctl & 15;
-  R.j = (ctl >> 4) & 63;
-  R.failed = (ctl >> 10) & 1;
-  R.bad = (ctl >> 11) & 1;
-  R.l = B.lstep[fit];
-  R.nev = B.nev[fit];
-  R.nev_tot = B.nev_tot[fit];
-  R.steps_tot = B.steps_tot[fit];
-  R.work = B.work[fit];
-  R.rng = D.rng[jfit];
-  R.fr = B.fr[fo];
-  R.sf = B.sf[fo];
+  LaneRegs<CF> R = load_lane(B, fit, fo, D.rng[jfit]);
   const bool refill = D.refill != 0;
   bool done = false;
   {
@@ -678,82 +772,196 @@ void fit_kernel(const GroupDesc<CF>* descs, SlotBufs<CF> B) {
     }
     const int running = __syncthreads_count(phase_pending(R.phase));
     if (running) continue;
-    // Every simplex of the group finished the stage (cuda.c:1739-1823).
-    s_f[t] = R.sf;
-    __syncthreads();
-    if (t == 0) {
-      int tm = 0;
-      CF smin = (CF)1e30;
-      for (int k = 0; k < G; ++k)
-        if (s_f[k] < smin) { smin = s_f[k]; tm = k; }
-      s_tm = tm;
-      s_smin = smin;
-    }
-    __syncthreads();
-    const int tm = s_tm;
-    const CF smin = s_smin;
-    if (nstages > 1 && stage < nstages - 1) {
-      if (t == tm) {
-        CF xb[N];
-        const int b = M.IND(0);
-#pragma unroll
-        for (int i = 0; i < N; ++i) xb[i] = M.X(b, i);
-        if (sp.p_psi && reopt == 0) {  // cuda.c:1791-1798
-          double prm[N];
-#pragma unroll
-          for (int i = 0; i < N; ++i) prm[i] = M.PRM(i);
-          x2params_at<CF, VC>(xb, prm, sp, reopt);
-          params2x<CF, VC>(xb, prm, sp);
-#pragma unroll
-          for (int i = 0; i < N; ++i) { M.PRM(i) = prm[i]; M.X(b, i) = xb[i]; }
-        }
-#pragma unroll
-        for (int i = 0; i < N; ++i) s_x0[i] = xb[i];
-      }
-      __syncthreads();
-      reopt = 1;
-      stage++;
-#pragma unroll
-      for (int i = 0; i < N; ++i) M.X(0, i) = s_x0[i];
-      R.phase = PH_START;
+    // Every simplex of the group finished the stage.
+    if (group_stage_end<CF, VC>(D, M, R, t, G, stage, reopt)) {
       Machine<CF, VC> M2{sp, B, SC, fit, nf, fo, rs, jfit, reopt};
       M2.advance(R, (CF)0, false);
     } else {
-      const int g = D.group_in_job;
-      if (t == tm && smin < D.best_f[g]) {  // cuda.c:1810-1823
-        D.best_f[g] = smin;
-        CF xb[N];
-        double prm[N];
-        const int b = M.IND(0);
-#pragma unroll
-        for (int i = 0; i < N; ++i) { xb[i] = M.X(b, i); prm[i] = M.PRM(i); }
-        x2params_at<CF, VC>(xb, prm, sp, reopt);
-#pragma unroll
-        for (int i = 0; i < N; ++i) {
-          M.PRM(i) = prm[i];
-          D.best_params[(size_t)g * N + i] = prm[i];
-        }
-        for (int m = 0; m < D.n_filters; ++m)
-          D.best_dV[(size_t)g * D.n_filters + m] = B.DV[(size_t)m * rs + fo];
-      }
-      D.fit_f[jfit] = R.sf;
-      D.fit_nev[jfit] = R.nev_tot;
-      D.fit_steps[jfit] = R.steps_tot;
-      stage++;
-      R.phase = PH_FIT_DONE;
       done = true;
     }
   }
-  B.ctl[fit] = R.phase | (R.j << 4) | (R.failed << 10) | (R.bad << 11);
-  B.lstep[fit] = R.l;
-  B.nev[fit] = R.nev;
-  B.nev_tot[fit] = R.nev_tot;
-  B.steps_tot[fit] = R.steps_tot;
-  B.work[fit] = R.work;
-  B.fitid[fit] = (int32_t)jfit;
+  store_lane(B, fit, fo, R, jfit);
   D.rng[jfit] = R.rng;
-  B.fr[fo] = R.fr;
-  B.sf[fo] = R.sf;
+  if (t == 0) {
+    B.g_reopt[slot] = reopt;
+    B.g_stage[slot] = stage;
+    B.g_done[slot] = done ? 1 : 0;
+    if (done) atomicAdd(D.job_done, 1);
+  }
+}
+
+// ---------------------------------------------------- several lanes per model
+// One evaluation with LP lanes per model (chi2_model_rows), for the kernels
+// below: parameters at PRM[i * stride], delta_V to DV[m * dv_stride].  Out of
+// line, so that a kernel class has one copy of it for its kernels.
+template <class CF, int VC, int NF, bool MX, int LP>
+__device__ __attribute__((noinline)) CF eval_rows(const double* PRM, size_t stride, CF* DV, size_t dv_stride,
+                                                   const PointRec* pts_g, int n_data, int n_filters, int dof,
+                                                   const double* sum_w) {
+  constexpr int N = Pos<VC>::N;
+  const uint64_t pu = (uint64_t)(uintptr_t)pts_g;
+  const uint64_t plo = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)pu);
+  const uint64_t phi = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(pu >> 32));
+  const uintptr_t pa = (uintptr_t)((phi << 32) | plo);
+  n_data = __builtin_amdgcn_readfirstlane(n_data);
+  n_filters = __builtin_amdgcn_readfirstlane(n_filters);
+  dof = __builtin_amdgcn_readfirstlane(dof);
+  double prm[N];
+#pragma unroll
+  for (int i = 0; i < N; ++i) prm[i] = PRM[(size_t)i * stride];
+  CF dv[NF];
+#pragma unroll
+  for (int m = 0; m < NF; ++m)  // a failed NUDGE model leaves delta_V as it was
+    dv[m] = VarF<VC>::NU && m < n_filters ? DV[(size_t)m * dv_stride] : CF(0);
+  CF fv = chi2_model_rows<CF, VC, NF, MX, FORM_CHI2, LP>(prm, (PointPtr)pa, (const PointRec*)pa, n_data, n_filters,
+                                                         dof, sum_w, dv);
+#pragma unroll
+  for (int m = 0; m < NF; ++m)
+    if (m < n_filters) DV[(size_t)m * dv_stride] = dv[m];
+  return fv;
+}
+
+// Registers for one or two waves per SIMD: these kernels run where the chip
+// is not full.
+#define AST_ROWS_BOUNDS __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 2)))
+
+// chi2_batch_kernel with LP lanes per model, 64 / LP models per workgroup (of
+// one wavefront, so that few models spread over the CUs).
+template <class CF, int VC, int NF, bool MX, int LP>
+__global__ AST_ROWS_BOUNDS void chi2_rows_kernel(const PointRec* pts_g, const double* sum_w, int n_data,
+                                                 int n_filters, int dof, const double* params, int n, double* chi2,
+                                                 double* dV) {
+  astm::sincos_table_load();
+  constexpr int N = Pos<VC>::N, M = 64 / LP;
+  __shared__ CF s_dv[M][NF];
+  const int row = threadIdx.x / LP;
+  const int k = blockIdx.x * M + row;
+  if (k >= n) return;
+  for (int m = 0; m < NF; ++m) s_dv[row][m] = VarF<VC>::NU ? CF(__builtin_nan("")) : CF(0);
+  const CF c = eval_rows<CF, VC, NF, MX, LP>(params + (size_t)k * N, 1, s_dv[row], 1, pts_g, n_data, n_filters, dof,
+                                             sum_w);
+  chi2[k] = c;
+  for (int m = 0; m < n_filters; ++m) dV[(size_t)k * n_filters + m] = s_dv[row][m];
+}
+
+// The grid walk of model_curve_kernel with LP lanes per model: delta_V of the
+// first filter from dV, written by chi2_rows_kernel before it.
+template <class CF, int VC, int NF, bool MX, int LP>
+__global__ AST_ROWS_BOUNDS void curve_rows_kernel(const double* sum_w, int n_filters, int dof,
+                                                  const PointRec* grid_g, int n_plot, const double* params, int n,
+                                                  const double* dV, double* vmod) {
+  astm::sincos_table_load();
+  constexpr int N = Pos<VC>::N, M = 64 / LP;
+  const int k = blockIdx.x * M + threadIdx.x / LP;
+  if (k >= n) return;
+  double prm[N];
+#pragma unroll
+  for (int i = 0; i < N; ++i) prm[i] = params[(size_t)k * N + i];
+  CF dv[NF];
+  chi2_model_rows<CF, VC, NF, MX, FORM_PLOT, LP>(prm, (PointPtr)(uintptr_t)grid_g, grid_g, n_plot, n_filters, dof,
+                                                 sum_w, dv, vmod + (size_t)k * n_plot, dV[(size_t)k * n_filters]);
+}
+
+// take_fit for LP lanes per model: one fit per asking model.
+template <int LP>
+__device__ inline int take_fit_rows(int32_t* queue) {
+  constexpr uint64_t firsts = LP == 16 ? 0x0001000100010001ull : 0x1111111111111111ull;
+  const uint64_t mask = __ballot(1) & firsts;
+  const int lane = (int)__lane_id();
+  const int leader = __ffsll((unsigned long long)mask) - 1;
+  const int rank = __popcll(mask & ((1ull << (lane & ~(LP - 1))) - 1ull));
+  int base = 0;
+  if (lane == leader) {
+    const int cnt = __popcll(mask);
+    base = atomicAdd(&queue[0], cnt);
+    atomicAdd(&queue[1], cnt);
+  }
+  base = __shfl(base, leader);
+  return base + rank;
+}
+
+// The fitting kernel with LP lanes per model: a workgroup is one wavefront
+// that runs 64 / LP of a group's simplexes, so that the simplexes of a few
+// groups spread over the whole chip.  Every lane of a model holds and stores
+// the model's state (equal values to the same addresses).  A wavefront ends
+// its launch when none of its simplexes has a pending point; the end of the
+// group's stage, which needs them all, is group_step_kernel's, launched
+// after it.
+template <class CF, int VC, int NF, bool MX, int LP>
+__global__ AST_ROWS_BOUNDS void fit_rows_kernel(const GroupDesc<CF>* descs, SlotBufs<CF> B, int G) {
+  astm::sincos_table_load();
+  constexpr int KC = 8 / sizeof(CF), M = 64 / LP;
+  const int per_group = G / M;
+  const GroupDesc<CF>& D = descs[blockIdx.x / per_group];
+  const int t = (int)(blockIdx.x % per_group) * M + (int)threadIdx.x / LP;
+  const int slot = D.slot;
+  const size_t nf = B.nf, rs = KC * nf;
+  const size_t fit = (size_t)slot * G + t;
+  const size_t fo = (size_t)slot * G * KC + t;
+  if (B.g_done[slot]) return;
+  uint64_t jfit = (uint64_t)B.fitid[fit];
+  const Space<CF>& sp = *D.sp;
+  const StageCfg<CF> SC{D.seed, D.size2_min, D.n_steps, D.eval_budget};
+  const int ticks = D.ticks;
+  const int reopt = B.g_reopt[slot];
+  LaneRegs<CF> R = load_lane(B, fit, fo, D.rng[jfit]);
+  const bool refill = D.refill != 0;
+  if (R.phase == PH_START) {
+    Machine<CF, VC> Ms{sp, B, SC, fit, nf, fo, rs, jfit, reopt};
+    Ms.advance(R, (CF)0, false);
+  }
+  for (int tick = 0; tick < ticks; ++tick) {
+    if (phase_pending(R.phase)) {
+      CF fv = eval_rows<CF, VC, NF, MX, LP>(B.PRM + fit, nf, B.DV + fo, rs, D.pts, D.n_data, D.n_filters, D.dof,
+                                            D.sum_w);
+      R.nev++;
+      R.nev_tot++;
+      R.work++;
+      Machine<CF, VC> Mt{sp, B, SC, fit, nf, fo, rs, jfit, reopt};
+      Mt.advance(R, fv, true);
+    }
+    if (refill) {  // as in fit_kernel
+      while (R.phase == PH_STAGE_DONE) {
+        Machine<CF, VC> Me{sp, B, SC, fit, nf, fo, rs, jfit, reopt};
+        Me.end_fit(R, D);
+        const int nj = take_fit_rows<LP>(D.queue);
+        if (nj >= D.n_fits) {
+          R.phase = PH_FIT_DONE;
+          break;
+        }
+        jfit = (uint64_t)nj;
+        Machine<CF, VC> Mb{sp, B, SC, fit, nf, fo, rs, jfit, reopt};
+        Mb.begin_fit(R, D);
+      }
+    }
+    if (__ballot(phase_pending(R.phase)) == 0) break;
+  }
+  store_lane(B, fit, fo, R, jfit);
+  D.rng[jfit] = R.rng;
+}
+
+// After fit_rows_kernel: one workgroup per group ends the group's stage once
+// all of its simplexes have (fit_kernel does this in place).
+template <class CF, int VC>
+__global__ __launch_bounds__(1024) void group_step_kernel(const GroupDesc<CF>* descs, SlotBufs<CF> B) {
+  constexpr int KC = 8 / sizeof(CF);
+  const GroupDesc<CF>& D = descs[blockIdx.x];
+  const int t = threadIdx.x, G = blockDim.x, slot = D.slot;
+  if (B.g_done[slot]) return;
+  const size_t nf = B.nf, rs = KC * nf;
+  const size_t fit = (size_t)slot * G + t, fo = (size_t)slot * G * KC + t;
+  const int phase = B.ctl[fit] & 15;
+  if (__syncthreads_count(phase != (D.refill ? PH_FIT_DONE : PH_STAGE_DONE))) return;
+  bool done = true;
+  int stage = B.g_stage[slot], reopt = B.g_reopt[slot];
+  if (!D.refill) {
+    const uint64_t jfit = (uint64_t)B.fitid[fit];
+    const StageCfg<CF> SC{D.seed, D.size2_min, D.n_steps, D.eval_budget};
+    LaneRegs<CF> R = load_lane(B, fit, fo, D.rng[jfit]);
+    Machine<CF, VC> M{*D.sp, B, SC, fit, nf, fo, rs, jfit, reopt};
+    done = !group_stage_end<CF, VC>(D, M, R, t, G, stage, reopt);
+    store_lane(B, fit, fo, R, jfit);
+  }
   if (t == 0) {
     B.g_reopt[slot] = reopt;
     B.g_stage[slot] = stage;
@@ -849,19 +1057,20 @@ struct RmsdArgs {
 };
 
 template <class CF, int VC, int NF, bool MX>
-__global__ __launch_bounds__(64) void rmsd_ref_kernel(RmsdArgs<CF> A) {
+__global__ AST_ROWS_BOUNDS void rmsd_ref_kernel(RmsdArgs<CF> A) {
   astm::sincos_table_load();  // the evaluator's sin/cos table into LDS (whole workgroup)
   using P = Pos<VC>;
   AST_VFLAGS(VC);
   constexpr int N = P::N;
-  if (threadIdx.x != 0) return;
+  if (threadIdx.x >= 16) return;  // one model, a row of lanes
   double prm[N];
   for (int i = 0; i < N; ++i) prm[i] = A.params0[i];
   CF x[N];
   params2x<CF, VC>(x, prm, *A.sp);
   CF dv[NF];
-  const CF f0 = chi2_model<CF, VC, NF, MX, FORM_RMSD>(prm, (PointPtr)(uintptr_t)A.pts, A.n_data,
-                                                              A.n_filters, A.dof, A.sum_w, dv);
+  const CF f0 = chi2_model_rows<CF, VC, NF, MX, FORM_RMSD, 16>(prm, (PointPtr)(uintptr_t)A.pts, A.pts, A.n_data,
+                                                               A.n_filters, A.dof, A.sum_w, dv);
+  if (threadIdx.x != 0) return;
   RmsdRef<CF>& R = *A.ref;
   for (int i = 0; i < N; ++i) R.x0[i] = x[i];
   R.f0 = f0;
@@ -983,6 +1192,7 @@ struct LaunchArgs {
   const void* bufs;    // SlotBufs<CF>*
   int n_groups, group_size, n_filters;
   int waves;           // fit kernel register budget: 4, 3 or 2 waves per SIMD
+  int lanes;           // fit: lanes per model (lanes_per_model)
   // batch
   const PointRec* pts;
   const double* sum_w;
@@ -999,11 +1209,42 @@ struct LaunchArgs {
   const void* rmsd;
 };
 
+// Lanes per model for n models evaluated side by side: as many as leave each
+// of the 1024 SIMDs one wavefront, since a wavefront alone takes its own time
+// whatever its lanes hold.  Kernel time at 16 / 4 / 1 lanes, LS + torque,
+// 400 points over 3 days, FP64 -- chi^2: 64 models 292 / 363 / 530 us, 4096
+// 356 / 376 / 533, 6144 588 / 389 / 533, 16384 1132 / 418 / 533, 24576
+// - / 679 / 539; fits of 30 evaluations: 4096 17.2 / 17.9 / 38.4 ms, 16384
+// 54.6 / 24.9 / 39.7, 24576 - / 37.3 / 39.8.  The mixed form and the form
+// without torque cross at the same sizes.
+constexpr int ROWS16_MAX = 4096, ROWS4_MAX = 16384;
+inline int lanes_per_model(int64_t n) { return n <= ROWS16_MAX ? 16 : n <= ROWS4_MAX ? 4 : 1; }
+
+template <class CF, int VC, int NF, bool MX, int LP>
+void launch_chi2_rows(const LaunchArgs& a) {
+  constexpr int M = 64 / LP;
+  hipLaunchKernelGGL((chi2_rows_kernel<CF, VC, NF, MX, LP>), dim3((a.n + M - 1) / M), dim3(64), 0, a.stream, a.pts,
+                     a.sum_w, a.n_data, a.n_filters, a.dof, a.params, a.n, a.chi2, a.dV);
+}
+template <class CF, int VC, int NF, bool MX, int LP>
+void launch_fit_rows(const LaunchArgs& a) {
+  constexpr int M = 64 / LP;
+  const GroupDesc<CF>* d = (const GroupDesc<CF>*)a.descs;
+  const SlotBufs<CF>& B = *(const SlotBufs<CF>*)a.bufs;
+  hipLaunchKernelGGL((fit_rows_kernel<CF, VC, NF, MX, LP>), dim3(a.n_groups * (a.group_size / M)), dim3(64), 0,
+                     a.stream, d, B, a.group_size);
+  hipLaunchKernelGGL((group_step_kernel<CF, VC>), dim3(a.n_groups), dim3(a.group_size), 0, a.stream, d, B);
+}
+
 template <class CF, int VC, int NF, bool MX>
 hipError_t launch_nf(const LaunchArgs& a) {
   if (a.op == 0) {
     hipLaunchKernelGGL((fit_init_kernel<CF, VC>), dim3(a.n_groups), dim3(a.group_size), 0, a.stream,
                        (const GroupDesc<CF>*)a.descs, *(const SlotBufs<CF>*)a.bufs);
+  } else if (a.op == 1 && a.lanes == 16) {
+    launch_fit_rows<CF, VC, NF, MX, 16>(a);
+  } else if (a.op == 1 && a.lanes == 4) {
+    launch_fit_rows<CF, VC, NF, MX, 4>(a);
   } else if (a.op == 1) {
     const GroupDesc<CF>* d = (const GroupDesc<CF>*)a.descs;
     const SlotBufs<CF>& B = *(const SlotBufs<CF>*)a.bufs;
@@ -1017,10 +1258,18 @@ hipError_t launch_nf(const LaunchArgs& a) {
     else
       hipLaunchKernelGGL((fit_kernel<CF, VC, NF, MX, 4>), dim3(a.n_groups), dim3(a.group_size), 0, a.stream,
                          d, B);
+  } else if (a.op == 2 && lanes_per_model(a.n) == 16) {
+    launch_chi2_rows<CF, VC, NF, MX, 16>(a);
+  } else if (a.op == 2 && lanes_per_model(a.n) == 4) {
+    launch_chi2_rows<CF, VC, NF, MX, 4>(a);
   } else if (a.op == 2) {
     int blocks = (a.n + 255) / 256;
     hipLaunchKernelGGL((chi2_batch_kernel<CF, VC, NF, MX>), dim3(blocks), dim3(256), 0, a.stream, a.pts,
                        a.sum_w, a.n_data, a.n_filters, a.dof, a.params, a.n, a.chi2, a.dV);
+  } else if (a.op == 3 && lanes_per_model(a.n) == 16) {
+    launch_chi2_rows<CF, VC, NF, MX, 16>(a);
+    hipLaunchKernelGGL((curve_rows_kernel<CF, VC, NF, MX, 16>), dim3((a.n + 3) / 4), dim3(64), 0, a.stream, a.sum_w,
+                       a.n_filters, a.dof, a.grid, a.n_plot, a.params, a.n, a.dV, a.vmod);
   } else if (a.op == 3) {
     int blocks = (a.n + 255) / 256;
     hipLaunchKernelGGL((model_curve_kernel<CF, VC, NF, MX>), dim3(blocks), dim3(256), 0, a.stream, a.pts,

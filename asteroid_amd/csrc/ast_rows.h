@@ -1,0 +1,330 @@
+// ast_rows.h -- the evaluator with several lanes per model.
+//
+// With one lane per model a launch of few models leaves the chip idle: 4096
+// models are 64 wavefronts on 1024 SIMDs, and a wavefront alone on its SIMD
+// issues one FP64 instruction every 4.3 cycles whatever its lanes hold, so
+// its time is its instruction count (620 per point of the torque form: 1.35
+// RK4 steps of 252 and 280 of brightness, 1.3 us).  Here LP = 16 or 4
+// neighbouring lanes (a DPP row or quad) share one model and the count per
+// point falls to about 300 or 390:
+//
+//   * the two sine/cosine pairs of an RK4 stage (theta and psi; without
+//     torque theta and 2 psi) are one call, even lanes taking the first angle
+//     and odd lanes the second, the results handed round by DPP moves;
+//   * the brightness, which needs only the Euler angles at its point, runs
+//     once per LP points, lane j doing point j of the batch;
+//   * the chi^2 sums then take the batch's residuals in the points' order.
+//
+// Every value comes from the same operations on the same operands as in
+// chi2_model, in the same order where order matters (the integration and the
+// sums), so the results are bitwise those of one lane per model.  The
+// lanes of a model hold equal values of everything but the shared angle and
+// the brightness.
+#pragma once
+#include "ast_device.h"
+
+namespace ast {
+
+// The intrinsic behind the DPP builtins, which take 32-bit values only: a
+// 64-bit row broadcast is one v_mov_b64 on gfx950.
+__device__ long long dpp_mov_b64(long long old, long long src, int ctrl, int row_mask, int bank_mask,
+                                 bool bound_ctrl) __asm("llvm.amdgcn.update.dpp.i64");
+
+// Value of lane K of the caller's LP-lane group.
+template <int LP, int K>
+AST_AI double lane_of(double x) {
+  static_assert(LP == 16 || LP == 4, "a DPP row or a quad");
+  const long long b = __builtin_bit_cast(long long, x);
+  if constexpr (LP == 16) {
+    return __builtin_bit_cast(double, dpp_mov_b64(0, b, 0x150 + K, 0xf, 0xf, true));  // row_newbcast:K
+  } else {
+    constexpr int ctrl = K * 0x55;  // quad_perm:[K,K,K,K]
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)b, ctrl, 0xf, 0xf, true);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(b >> 32), ctrl, 0xf, 0xf, true);
+    return __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
+  }
+}
+
+// f(integral_constant<int, 0>), ..., f(integral_constant<int, N - 1>).
+template <int K>
+struct IntC {
+  static constexpr int value = K;
+};
+template <int N, int K = 0, class F>
+AST_AI void unroll_lanes(const F& f) {
+  if constexpr (K < N) {
+    f(IntC<K>{});
+    unroll_lanes<N, K + 1>(f);
+  }
+}
+
+// sin and cos of the two angles of a stage: the lane's own argument in x
+// (even lanes the first angle, odd lanes the second), both pairs out.
+template <int LP>
+AST_AI void sincos_pair(double x, double* sc) {
+  double s, c;
+  astm::sincos_t(x, &s, &c);
+  sc[0] = lane_of<LP, 0>(s);
+  sc[1] = lane_of<LP, 0>(c);
+  sc[2] = lane_of<LP, 1>(s);
+  sc[3] = lane_of<LP, 1>(c);
+}
+
+// One RK4 step of the shared integration (cuda.c:348-372).  w holds the
+// angular velocity (torque form only), phi the first Euler angle and p the
+// lane's angle (theta or psi); sc the sine/cosine pairs at the step's start
+// (theta and psi, without torque theta and 2 psi), replaced by those at its
+// end.  The same operations as ode() and chi2_model's step.
+template <bool TQ, int LP>
+AST_AI void rk4_shared(double* w, double& phi, double& p, double* sc, const double* mu, double mu02, bool odd,
+                       double h, double hh, double h6) {
+  const double twice = odd ? 2.0 : 1.0;  // without torque the odd lanes' argument is 2 psi
+  double sw[3] = {0, 0, 0}, fw[3], sphi, sp;
+  if (TQ) { fw[0] = w[0]; fw[1] = w[1]; fw[2] = w[2]; }
+#pragma unroll
+  for (int stage = 0; stage < 4; ++stage) {
+    double k[3] = {0, 0, 0}, kphi, kp;
+    if (TQ) {
+      k[0] = __builtin_fma(mu[0] * fw[1], fw[2], mu[3]);
+      k[1] = __builtin_fma(mu[1] * fw[2], fw[0], mu[4]);
+      k[2] = __builtin_fma(mu[2] * fw[0], fw[1], mu[5]);
+      kphi = astm::div_rn(__builtin_fma(fw[1], sc[3], fw[0] * sc[2]), sc[0]);
+      const double kth = __builtin_fma(-fw[1], sc[2], fw[0] * sc[3]);
+      const double kps = __builtin_fma(-kphi, sc[1], fw[2]);
+      kp = odd ? kps : kth;
+    } else {
+      kphi = mu[0] * __builtin_fma(-mu[2], sc[3], mu[1]);
+      const double kth = (mu02 * sc[0]) * sc[2];
+      const double kps = sc[1] * (mu[0] - kphi);
+      kp = odd ? kps : kth;
+    }
+    if (stage == 0) {
+      sw[0] = k[0]; sw[1] = k[1]; sw[2] = k[2];
+      sphi = kphi;
+      sp = kp;
+    } else if (stage < 3) {
+      if (TQ) {
+#pragma unroll
+        for (int j = 0; j < 3; ++j) sw[j] = __builtin_fma(2.0, k[j], sw[j]);
+      }
+      sphi = __builtin_fma(2.0, kphi, sphi);
+      sp = __builtin_fma(2.0, kp, sp);
+    } else {
+      if (TQ) {
+#pragma unroll
+        for (int j = 0; j < 3; ++j) w[j] = __builtin_fma(h6, sw[j] + k[j], w[j]);
+      }
+      phi = __builtin_fma(h6, sphi + kphi, phi);
+      p = __builtin_fma(h6, sp + kp, p);
+    }
+    double a = p;
+    if (stage < 3) {
+      const double hs = stage < 2 ? hh : h;
+      if (TQ) {
+#pragma unroll
+        for (int j = 0; j < 3; ++j) fw[j] = __builtin_fma(hs, k[j], w[j]);
+      }
+      a = __builtin_fma(hs, kp, p);
+    }
+    sincos_pair<LP>(TQ ? a : twice * a, sc);
+  }
+}
+
+// chi2_model with LP lanes per model (same arguments, same results in every
+// lane of a model).  All lanes of a model must be active together.  With
+// FORM_PLOT vplot is the model's own curve (stride 1).
+template <class CF, int VC, int NF, bool MX, int FORM, int LP>
+__device__ CF chi2_model_rows(const double* params, PointPtr pts, const PointRec* pts_g, int n_data, int n_filters,
+                              int dof, const double* sum_w, CF* dV, double* vplot = nullptr, double dv0 = 0.0) {
+  using P = Pos<VC>;
+  AST_VFLAGS(VC);
+  static_assert(!(TR && (T2 || NU)), "PointRec.aux is the phase angle under TREND and the time otherwise");
+  const int lane = (int)__lane_id() & (LP - 1);
+  const bool odd = lane & 1;
+  double sy2[NF], sy[NF];
+#pragma unroll
+  for (int m = 0; m < NF; ++m) { sy2[m] = 0.0; sy[m] = 0.0; }
+  const double bt = params[P::b_tumb], ct = params[P::c_tumb];
+  const double den = __builtin_fma(ct, ct, bt * bt);
+  const double Is = __builtin_fma(bt, bt, 1.0) / den;
+  const double Ii = __builtin_fma(ct, ct, 1.0) / den;
+  const double Is_inv = 1.0 / Is;
+  const double Ii_inv = 1.0 / Ii;
+  SpinFrame<double> Fd;
+  double mu[6];
+  double mu02 = 0.0;
+  double w[3] = {0, 0, 0}, phi, p, sc[4];
+  // The rotation's start (or a segment's): the state as begin_rotation gives
+  // it, the lane's angle picked out, and without torque the sine and cosine
+  // of 2 psi beside those of theta.
+  auto begin = [&](int k) {
+    double y[6];
+    begin_rotation<VC>(params, k, Is_inv, Ii_inv, Is, Ii, Fd, y, mu, mu02, sc);
+    if (TQ) {
+      w[0] = y[0]; w[1] = y[1]; w[2] = y[2];
+      phi = y[3];
+      p = odd ? y[5] : y[4];
+    } else {
+      phi = y[0];
+      p = odd ? y[2] : y[1];
+      astm::sincos_t(2.0 * y[2], &sc[2], &sc[3]);
+    }
+  };
+  begin(0);
+  ModelConsts K{0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
+  if constexpr (RO) {
+    astm::sincos_t(params[P::phi_R], &K.sR, &K.cR);
+    astm::sincos_t(params[P::theta_R], &K.stR, &K.ctR);
+    astm::sincos_t(params[P::psi_R], &K.sPR, &K.cPR);
+  }
+  if (BW) {
+    astm::sincos_t(params[P::phi_R], &K.sR, &K.cR);
+    astm::sincos_t(params[P::theta_R], &K.stR, &K.ctR);
+    K.kappa = params[P::kappa];
+  } else {
+    const double b = BC ? params[P::b] : bt;
+    const double c = BC ? params[P::c] : ct;
+    K.ib = 1.0 / b;
+    K.ic = 1.0 / c;
+    K.bcp = b * c;
+  }
+  const float bcpf = (float)K.bcp;  // mixed form
+  float nu_t[NU ? NU_M_MAX : 1], nu_V[NU ? NU_M_MAX : 1];
+  NudgeState nu;
+  nu.t_mod = nu_t;
+  nu.V_mod = nu_V;
+  TailPtr mr = (TailPtr)(pts + n_data);
+  double trendA = 0.0, t_split = 0.0;
+  if constexpr (TR) trendA = params[P::A];
+  bool switched = false;
+  if constexpr (T2)  // cuda.c:291
+    t_split = __builtin_fma(params[P::Tt], pts[n_data - 1].aux - pts[0].aux, pts[0].aux);
+  // The next interval's constants are read one point ahead (pts[n_data] is
+  // the tail record), as in chi2_model.
+  int nx_steps = pts[0].nsteps;
+  double nx_h = pts[0].h, nx_hh = pts[0].hh, nx_h6 = pts[0].h6;
+  for (int i0 = 0; i0 < n_data; i0 += LP) {
+    const int m = n_data - i0 < LP ? n_data - i0 : LP;
+    // The lane's own point of the batch (the last one, for lanes beyond it,
+    // whose results are left out): read before the integration covers the
+    // loads' latency.
+    const PointRec* pr = pts_g + (i0 + (lane < m ? lane : m - 1));
+    const double E[3] = {pr->E[0], pr->E[1], pr->E[2]};
+    const double S[3] = {pr->S[0], pr->S[1], pr->S[2]};
+    const float pV = pr->V, pw = pr->w;
+    double aux = 0.0;
+    if constexpr (TR) aux = pr->aux;
+    double cphi = 0.0, cth = 0.0, cps = 0.0;  // the Euler angles at the lane's point
+    SpinFrame<double> Fl = Fd;                // and, with segments, its spin frame
+    for (int j = 0; j < m; ++j) {
+      const int i = i0 + j;
+      int nsteps = nx_steps;
+      double h = nx_h, hh = nx_hh, h6 = nx_h6;
+      nx_steps = pts[i + 1].nsteps;
+      nx_h = pts[i + 1].h;
+      nx_hh = pts[i + 1].hh;
+      nx_h6 = pts[i + 1].h6;
+      if constexpr (SG) {
+        if (nsteps < 0) begin(-1 - nsteps);
+      }
+      int nsub = 1;
+      double t2_end = 0.0;
+      if constexpr (T2) {  // cuda.c:288-317
+        if (i > 0 && !switched && t_split >= pts[i - 1].aux && t_split < pts[i].aux) {
+          const double t1 = pts[i - 1].aux;
+          nsub = 2;
+          t2_end = pts[i].aux;
+          nsteps = (int)((t_split - t1) / mr->ts + 1);
+          h = (t_split - t1) / nsteps;
+          hh = 0.5 * h;
+          h6 = 1 / 6.0 * h;
+        }
+      }
+      for (int isub = 0; isub < nsub; ++isub) {
+        if constexpr (T2) {
+          if (isub == 1) {
+            nsteps = (int)((t2_end - t_split) / mr->ts + 1);
+            h = (t2_end - t_split) / nsteps;
+            hh = 0.5 * h;
+            h6 = 1 / 6.0 * h;
+            mu[3] = params[P::T2i];
+            mu[4] = params[P::T2s];
+            mu[5] = params[P::T2l];
+            switched = true;
+          }
+        }
+        for (int l = 0; l < nsteps; ++l) rk4_shared<TQ, LP>(w, phi, p, sc, mu, mu02, odd, h, hh, h6);
+      }
+      const double th = lane_of<LP, 0>(p), ps = lane_of<LP, 1>(p);
+      const bool mine = lane == j;
+      cphi = mine ? phi : cphi;
+      cth = mine ? th : cth;
+      cps = mine ? ps : cps;
+      if constexpr (SG) {
+        if (mine) Fl = Fd;
+      }
+    }
+    // Brightness of the lane's point.
+    double asc[4], a[3], b[3], c[3];
+    astm::sincos_t(cth, &asc[0], &asc[1]);
+    if (TQ) astm::sincos_t(cps, &asc[2], &asc[3]);
+    axes_at<TQ>(SG ? Fl : Fd, cphi, cps, asc, a, b, c);
+    if constexpr (RO) rotate_axes(a, b, c, K);
+    double Vmod;
+    if constexpr (RC) {
+      Vmod = rect_mag(a, b, c, E, params[P::b], params[P::c]);
+    } else if (BW) {
+      const double arg = bw_arg_f64(a, b, c, E, K);
+      Vmod = MX ? M2P5_LOG10_2 * log2_f32x((float)arg) : -2.5 * astm::log10(arg);
+    } else {
+      const ScaledDirs u = scaled_dirs(a, b, c, E, S, K);
+      if (MX) Vmod = ls_tail_mx(u, bcpf);
+      else Vmod = ls_tail_f64(u, K.bcp);
+    }
+    if constexpr (TR) Vmod = __builtin_fma(-trendA, aux, Vmod);  // cuda.c:692-697
+    if constexpr (NU) {
+      // The minima are found point by point, by every lane alike.
+      const int base = (int)__lane_id() & ~(LP - 1);
+      for (int j = 0; j < m; ++j) {
+        const double Vj = __shfl(Vmod, base + j);
+        if constexpr (FORM == FORM_PLOT)
+          if (lane == j) vplot[i0 + j] = nu.failed ? __builtin_nan("") : Vj + dv0;
+        nu.point(i0 + j, pts[i0 + j].aux, Vj, mr);
+      }
+    }
+    if constexpr (FORM == FORM_PLOT) {
+      if constexpr (!NU)
+        if (lane < m) vplot[i0 + lane] = Vmod + dv0;
+      continue;
+    }
+    // The sums, in the points' order.  Lanes past the curve's end give a
+    // residual and a weight of 0, which leave the sums as they are (a sum
+    // that is an exact zero is +0).
+    const bool in = lane < m;
+    const double wl = in ? (double)pw : 0.0;
+    const double yv = in ? (double)pV - Vmod : 0.0;
+    const double yq = yv * yv;
+    unroll_lanes<LP>([&](auto jc) {
+      constexpr int j = decltype(jc)::value;
+      const double yj = lane_of<LP, j>(yv), qj = lane_of<LP, j>(yq), wj = lane_of<LP, j>(wl);
+      if constexpr (NF == 1) {
+        sy2[0] = __builtin_fma(qj, wj, sy2[0]);
+        sy[0] = __builtin_fma(yj, wj, sy[0]);
+      } else {
+        const int f = pts[i0 + (j < m ? j : m - 1)].filter;
+#pragma unroll
+        for (int k = 0; k < NF; ++k)
+          if (f == k) {
+            sy2[k] = __builtin_fma(qj, wj, sy2[k]);
+            sy[k] = __builtin_fma(yj, wj, sy[k]);
+          }
+      }
+    });
+  }
+  if constexpr (FORM == FORM_PLOT) return CF(0.0);
+  if constexpr (NU)
+    if (nu.failed) return CF(1e30);
+  return model_score<CF, VC, NF, FORM>(sy2, sy, n_filters, dof, sum_w, dV, NU ? &nu : nullptr, mr);
+}
+
+}  // namespace ast

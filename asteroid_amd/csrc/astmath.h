@@ -223,10 +223,34 @@ template <class R> AST_HD void sincos(R x, R* s, R* c) {
 // (it ends with a barrier); until then the copy holds garbage.
 #if defined(__HIP_DEVICE_COMPILE__)
 static __shared__ double2 g_sctab[AST_SCTAB_N];
-__device__ inline void sincos_table_load() {
+struct SinCosTab {
+  double v[2 * AST_SCTAB_N];  // sin, cos of entry k at 2k, 2k + 1
+};
+constexpr SinCosTab sincos_tab() {
   constexpr double ts[AST_SCTAB_N] = AST_SCTAB_SIN;
   constexpr double tc[AST_SCTAB_N] = AST_SCTAB_COS;
-  for (int i = threadIdx.x; i < AST_SCTAB_N; i += blockDim.x) g_sctab[i] = make_double2(ts[i], tc[i]);
+  SinCosTab t{};
+  for (int k = 0; k < AST_SCTAB_N; ++k) {
+    t.v[2 * k] = ts[k];
+    t.v[2 * k + 1] = tc[k];
+  }
+  return t;
+}
+static __device__ const SinCosTab g_sctab_src alignas(16) = sincos_tab();
+// A workgroup of one wavefront has 16 entries per thread to fetch, all in
+// flight together.
+__device__ inline void sincos_table_load() {
+  const double2* src = (const double2*)g_sctab_src.v;
+  const int nt = blockDim.x;
+  for (int base = threadIdx.x; base < AST_SCTAB_N; base += 16 * nt) {
+    double2 r[16];
+#pragma unroll
+    for (int j = 0; j < 16; ++j)
+      if (base + j * nt < AST_SCTAB_N) r[j] = src[base + j * nt];
+#pragma unroll
+    for (int j = 0; j < 16; ++j)
+      if (base + j * nt < AST_SCTAB_N) g_sctab[base + j * nt] = r[j];
+  }
   __syncthreads();
 }
 __device__ inline void sctab_get(uint32_t i, double* s, double* c) {
