@@ -813,7 +813,7 @@ __device__ __attribute__((noinline)) CF eval_rows(const double* PRM, size_t stri
 #pragma unroll
   for (int m = 0; m < NF; ++m)  // a failed NUDGE model leaves delta_V as it was
     dv[m] = VarF<VC>::NU && m < n_filters ? DV[(size_t)m * dv_stride] : CF(0);
-  CF fv = chi2_model_rows<CF, VC, NF, MX, FORM_CHI2, LP>(prm, (PointPtr)pa, (const PointRec*)pa, n_data, n_filters,
+  CF fv = chi2_model_rows<CF, VC, NF, MX, FORM_CHI2, LP>(prm, (PointPtr)pa, (LanePtr)pa, n_data, n_filters,
                                                          dof, sum_w, dv);
 #pragma unroll
   for (int m = 0; m < NF; ++m)
@@ -858,7 +858,7 @@ __global__ AST_ROWS_BOUNDS void curve_rows_kernel(const double* sum_w, int n_fil
 #pragma unroll
   for (int i = 0; i < N; ++i) prm[i] = params[(size_t)k * N + i];
   CF dv[NF];
-  chi2_model_rows<CF, VC, NF, MX, FORM_PLOT, LP>(prm, (PointPtr)(uintptr_t)grid_g, grid_g, n_plot, n_filters, dof,
+  chi2_model_rows<CF, VC, NF, MX, FORM_PLOT, LP>(prm, (PointPtr)(uintptr_t)grid_g, (LanePtr)(uintptr_t)grid_g, n_plot, n_filters, dof,
                                                  sum_w, dv, vmod + (size_t)k * n_plot, dV[(size_t)k * n_filters]);
 }
 
@@ -1068,7 +1068,7 @@ __global__ AST_ROWS_BOUNDS void rmsd_ref_kernel(RmsdArgs<CF> A) {
   CF x[N];
   params2x<CF, VC>(x, prm, *A.sp);
   CF dv[NF];
-  const CF f0 = chi2_model_rows<CF, VC, NF, MX, FORM_RMSD, 16>(prm, (PointPtr)(uintptr_t)A.pts, A.pts, A.n_data,
+  const CF f0 = chi2_model_rows<CF, VC, NF, MX, FORM_RMSD, 16>(prm, (PointPtr)(uintptr_t)A.pts, (LanePtr)(uintptr_t)A.pts, A.n_data,
                                                                A.n_filters, A.dof, A.sum_w, dv);
   if (threadIdx.x != 0) return;
   RmsdRef<CF>& R = *A.ref;

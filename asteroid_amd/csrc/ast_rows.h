@@ -30,6 +30,14 @@ namespace ast {
 __device__ long long dpp_mov_b64(long long old, long long src, int ctrl, int row_mask, int bank_mask,
                                  bool bound_ctrl) __asm("llvm.amdgcn.update.dpp.i64");
 
+// The table as vector loads read it (a generic pointer would make them FLAT
+// loads, which the table reads in LDS have to wait for).
+typedef __attribute__((address_space(1))) const PointRec* LanePtr;
+
+// As pin_sgpr, for a value a vector load gives: what was loaded before this
+// point is waited for here and not, over and over, at its uses in a loop.
+template <class T> __device__ inline void pin_vgpr(T& v) { asm volatile("" : "+v"(v)); }
+
 // Value of lane K of the caller's LP-lane group.
 template <int LP, int K>
 AST_AI double lane_of(double x) {
@@ -58,36 +66,24 @@ AST_AI void unroll_lanes(const F& f) {
   }
 }
 
-// sin and cos of the two angles of a stage: the lane's own argument in x
-// (even lanes the first angle, odd lanes the second), both pairs out.
-template <int LP>
-AST_AI void sincos_pair(double x, double* sc) {
-  double s, c;
-  astm::sincos_t(x, &s, &c);
-  sc[0] = lane_of<LP, 0>(s);
-  sc[1] = lane_of<LP, 0>(c);
-  sc[2] = lane_of<LP, 1>(s);
-  sc[3] = lane_of<LP, 1>(c);
-}
-
 // One RK4 step of the shared integration (cuda.c:348-372).  w holds the
 // angular velocity (torque form only), phi the first Euler angle and p the
-// lane's angle (theta or psi); sc the sine/cosine pairs at the step's start
-// (theta and psi, without torque theta and 2 psi), replaced by those at its
-// end.  The same operations as ode() and chi2_model's step.
+// lane's angle (theta on even lanes, psi on odd ones); sc the sine/cosine
+// pairs at the step's start (theta and psi, without torque theta and 2 psi),
+// replaced by those at its end.  The same operations as ode() and
+// chi2_model's step; their order puts the next stage's table read as early as
+// its angle is known (the barrier keeps it there) and the angular velocity's
+// part of the stage behind it, so that a wavefront alone on its SIMD does not
+// wait for the read.
 template <bool TQ, int LP>
 AST_AI void rk4_shared(double* w, double& phi, double& p, double* sc, const double* mu, double mu02, bool odd,
                        double h, double hh, double h6) {
   const double twice = odd ? 2.0 : 1.0;  // without torque the odd lanes' argument is 2 psi
-  double sw[3] = {0, 0, 0}, fw[3], sphi, sp;
-  if (TQ) { fw[0] = w[0]; fw[1] = w[1]; fw[2] = w[2]; }
+  double sw[3] = {0, 0, 0}, fw[3] = {w[0], w[1], w[2]}, sphi, sp;
 #pragma unroll
   for (int stage = 0; stage < 4; ++stage) {
-    double k[3] = {0, 0, 0}, kphi, kp;
+    double kphi, kp;
     if (TQ) {
-      k[0] = __builtin_fma(mu[0] * fw[1], fw[2], mu[3]);
-      k[1] = __builtin_fma(mu[1] * fw[2], fw[0], mu[4]);
-      k[2] = __builtin_fma(mu[2] * fw[0], fw[1], mu[5]);
       kphi = astm::div_rn(__builtin_fma(fw[1], sc[3], fw[0] * sc[2]), sc[0]);
       const double kth = __builtin_fma(-fw[1], sc[2], fw[0] * sc[3]);
       const double kps = __builtin_fma(-kphi, sc[1], fw[2]);
@@ -98,35 +94,43 @@ AST_AI void rk4_shared(double* w, double& phi, double& p, double* sc, const doub
       const double kps = sc[1] * (mu[0] - kphi);
       kp = odd ? kps : kth;
     }
+    const double hs = stage < 2 ? hh : h;
+    double a;
+    if (stage < 3) {
+      a = __builtin_fma(hs, kp, p);
+    } else {
+      p = __builtin_fma(h6, sp + kp, p);
+      a = p;
+    }
+    if (!TQ) a = twice * a;
+    const double kb = astm::sincos_t_k(a);
+    double ts, tc, s, c;
+    astm::sctab_get(astm::sctab_index(kb), &ts, &tc);
+    __builtin_amdgcn_sched_barrier(0);
+    if (TQ) {
+      const double k[3] = {__builtin_fma(mu[0] * fw[1], fw[2], mu[3]), __builtin_fma(mu[1] * fw[2], fw[0], mu[4]),
+                           __builtin_fma(mu[2] * fw[0], fw[1], mu[5])};
+#pragma unroll
+      for (int j = 0; j < 3; ++j) {
+        sw[j] = stage == 0 ? k[j] : stage < 3 ? __builtin_fma(2.0, k[j], sw[j]) : sw[j] + k[j];
+        if (stage < 3) fw[j] = __builtin_fma(hs, k[j], w[j]);
+        else w[j] = __builtin_fma(h6, sw[j], w[j]);
+      }
+    }
     if (stage == 0) {
-      sw[0] = k[0]; sw[1] = k[1]; sw[2] = k[2];
       sphi = kphi;
       sp = kp;
     } else if (stage < 3) {
-      if (TQ) {
-#pragma unroll
-        for (int j = 0; j < 3; ++j) sw[j] = __builtin_fma(2.0, k[j], sw[j]);
-      }
       sphi = __builtin_fma(2.0, kphi, sphi);
       sp = __builtin_fma(2.0, kp, sp);
     } else {
-      if (TQ) {
-#pragma unroll
-        for (int j = 0; j < 3; ++j) w[j] = __builtin_fma(h6, sw[j] + k[j], w[j]);
-      }
       phi = __builtin_fma(h6, sphi + kphi, phi);
-      p = __builtin_fma(h6, sp + kp, p);
     }
-    double a = p;
-    if (stage < 3) {
-      const double hs = stage < 2 ? hh : h;
-      if (TQ) {
-#pragma unroll
-        for (int j = 0; j < 3; ++j) fw[j] = __builtin_fma(hs, k[j], w[j]);
-      }
-      a = __builtin_fma(hs, kp, p);
-    }
-    sincos_pair<LP>(TQ ? a : twice * a, sc);
+    astm::sincos_t_end(a, kb, ts, tc, &s, &c);
+    sc[0] = lane_of<LP, 0>(s);
+    sc[1] = lane_of<LP, 0>(c);
+    sc[2] = lane_of<LP, 1>(s);
+    sc[3] = lane_of<LP, 1>(c);
   }
 }
 
@@ -134,8 +138,8 @@ AST_AI void rk4_shared(double* w, double& phi, double& p, double* sc, const doub
 // lane of a model).  All lanes of a model must be active together.  With
 // FORM_PLOT vplot is the model's own curve (stride 1).
 template <class CF, int VC, int NF, bool MX, int FORM, int LP>
-__device__ CF chi2_model_rows(const double* params, PointPtr pts, const PointRec* pts_g, int n_data, int n_filters,
-                              int dof, const double* sum_w, CF* dV, double* vplot = nullptr, double dv0 = 0.0) {
+__device__ CF chi2_model_rows(const double* params, PointPtr pts, LanePtr pts_g, int n_data, int n_filters, int dof,
+                              const double* sum_w, CF* dV, double* vplot = nullptr, double dv0 = 0.0) {
   using P = Pos<VC>;
   AST_VFLAGS(VC);
   static_assert(!(TR && (T2 || NU)), "PointRec.aux is the phase angle under TREND and the time otherwise");
@@ -199,16 +203,28 @@ __device__ CF chi2_model_rows(const double* params, PointPtr pts, const PointRec
   bool switched = false;
   if constexpr (T2)  // cuda.c:291
     t_split = __builtin_fma(params[P::Tt], pts[n_data - 1].aux - pts[0].aux, pts[0].aux);
-  // The next interval's constants are read one point ahead (pts[n_data] is
-  // the tail record), as in chi2_model.
-  int nx_steps = pts[0].nsteps;
-  double nx_h = pts[0].h, nx_hh = pts[0].hh, nx_h6 = pts[0].h6;
+  // Each lane reads the record of its own point of a batch (the curve's last
+  // one, for lanes beyond it, whose results are left out) with vector loads:
+  // the step count and size a batch ahead, handed out point by point with
+  // readlane, the rest while the batch is integrated.  Scalar loads of the
+  // records one point ahead were waited for at every point, since they share
+  // their counter with the table reads: 0.62 us per point of a one-model
+  // plot.
+  const int row0 = __builtin_amdgcn_readfirstlane((int)__lane_id()) & ~(LP - 1);
+  int nx_steps = pts_g[lane < n_data ? lane : n_data - 1].nsteps;
+  double nx_h = pts_g[lane < n_data ? lane : n_data - 1].h;
+  pin_vgpr(nx_steps);
+  pin_vgpr(nx_h);
   for (int i0 = 0; i0 < n_data; i0 += LP) {
     const int m = n_data - i0 < LP ? n_data - i0 : LP;
-    // The lane's own point of the batch (the last one, for lanes beyond it,
-    // whose results are left out): read before the integration covers the
-    // loads' latency.
-    const PointRec* pr = pts_g + (i0 + (lane < m ? lane : m - 1));
+    const int lane_steps = nx_steps;
+    const uint64_t lane_h = astm::bits_of(nx_h);
+    {
+      const int nx = i0 + LP + lane;
+      nx_steps = pts_g[nx < n_data ? nx : n_data - 1].nsteps;
+      nx_h = pts_g[nx < n_data ? nx : n_data - 1].h;
+    }
+    const LanePtr pr = pts_g + (i0 + (lane < m ? lane : m - 1));
     const double E[3] = {pr->E[0], pr->E[1], pr->E[2]};
     const double S[3] = {pr->S[0], pr->S[1], pr->S[2]};
     const float pV = pr->V, pw = pr->w;
@@ -218,12 +234,11 @@ __device__ CF chi2_model_rows(const double* params, PointPtr pts, const PointRec
     SpinFrame<double> Fl = Fd;                // and, with segments, its spin frame
     for (int j = 0; j < m; ++j) {
       const int i = i0 + j;
-      int nsteps = nx_steps;
-      double h = nx_h, hh = nx_hh, h6 = nx_h6;
-      nx_steps = pts[i + 1].nsteps;
-      nx_h = pts[i + 1].h;
-      nx_hh = pts[i + 1].hh;
-      nx_h6 = pts[i + 1].h6;
+      int nsteps = __builtin_amdgcn_readlane(lane_steps, row0 + j);
+      const uint32_t h_lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)lane_h, row0 + j);
+      const uint32_t h_hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(lane_h >> 32), row0 + j);
+      double h = astm::of_bits(((uint64_t)h_hi << 32) | h_lo);
+      double hh = 0.5 * h, h6 = 1 / 6.0 * h;  // as the table's
       if constexpr (SG) {
         if (nsteps < 0) begin(-1 - nsteps);
       }
@@ -264,6 +279,8 @@ __device__ CF chi2_model_rows(const double* params, PointPtr pts, const PointRec
         if (mine) Fl = Fd;
       }
     }
+    pin_vgpr(nx_steps);
+    pin_vgpr(nx_h);
     // Brightness of the lane's point.
     double asc[4], a[3], b[3], c[3];
     astm::sincos_t(cth, &asc[0], &asc[1]);

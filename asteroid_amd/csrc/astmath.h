@@ -280,20 +280,28 @@ inline void sctab_get(uint32_t i, double* s, double* c) {
 // About 1 ulp for |x| < 2^51 pi/512, with no quadrant logic: 17 instructions
 // and one table read on the GPU against 39 for sincos.  Non-finite x gives
 // NaN for both.
-template <class R> AST_HD void sincos_t(R x, R* s, R* c) {
-  const R kb = p_fma(x, R(AST_SCTAB_INV_STEP), R(RINT_SHIFT));
+// In two parts, for a caller that has other work for the time of the table
+// read: sincos_t_k gives k (in RINT_SHIFT's low word), sctab_index its entry,
+// sincos_t_end the rest.
+template <class R> AST_HD R sincos_t_k(R x) { return p_fma(x, R(AST_SCTAB_INV_STEP), R(RINT_SHIFT)); }
+AST_HD uint32_t sctab_index(double kb) { return (uint32_t)bits_of(kb) & (AST_SCTAB_N - 1); }
+template <class R> AST_HD void sincos_t_end(R x, R kb, double tsv, double tcv, R* s, R* c) {
   const R k = kb - R(RINT_SHIFT);
   R r = p_fma(-k, R(AST_SCTAB_STEP_1), x);
   r = p_fma(-k, R(AST_SCTAB_STEP_2), r);
   r = p_fma(-k, R(AST_SCTAB_STEP_3), r);
-  double tsv, tcv;
-  sctab_get((uint32_t)bits_of(p_val(kb)) & (AST_SCTAB_N - 1), &tsv, &tcv);
   const R S(tsv), C(tcv);
   R z = r * r;
   R sr = p_fma(r * z, p_fma(z, R(AST_SINT_1), R(AST_SINT_0)), r);
   R cm = z * p_fma(z, R(AST_COST_0), R(-0.5));
   *s = p_fma(S, cm, p_fma(C, sr, S));
   *c = p_fma(C, cm, p_fma(-S, sr, C));
+}
+template <class R> AST_HD void sincos_t(R x, R* s, R* c) {
+  const R kb = sincos_t_k(x);
+  double tsv, tcv;
+  sctab_get(sctab_index(p_val(kb)), &tsv, &tcv);
+  sincos_t_end(x, kb, tsv, tcv, s, c);
 }
 
 template <class R> AST_HD R sin(R x) { R s, c; sincos(x, &s, &c); return s; }
