@@ -157,8 +157,13 @@ __device__ inline float cf_floor(float x) { return __builtin_floorf(x); }
 // ------------------------------------------------------------------ x2params
 // cuda.c:1120-1319 (P_PSI branch of the L mapping).  Same operation order
 // and types as the oracle.  Returns nonzero on a hard-limit crossing.
-template <class CF, int VC>
-__device__ int x2params(const CF* x, double* params, const Space<CF>& sp, int reopt) {
+// The model space is wave-uniform; through an address-space-4 pointer its
+// fields come by scalar loads.  The maps below take either form (SP).
+template <class CF>
+using SpacePtr = __attribute__((address_space(4))) const Space<CF>*;
+
+template <class CF, int VC, class SP>
+__device__ int x2params(const CF* x, double* params, const SP& sp, int reopt) {
   using P = Pos<VC>;
   AST_VFLAGS(VC);
   constexpr int N = P::N;
@@ -238,20 +243,20 @@ __device__ int x2params(const CF* x, double* params, const Space<CF>& sp, int re
 // restatement's at some lanes (hipcc of ROCm 7.2 for gfx950, at -O1, -O2 and
 // -O3 alike), while the same map evaluated on its own matched it bitwise; the
 // out-of-line copy matches bit for bit.  Other builds keep it inlined.
-template <class CF, int VC>
-__device__ __attribute__((noinline)) int x2params_ool(const CF* x, double* params, const Space<CF>& sp, int reopt) {
+template <class CF, int VC, class SP>
+__device__ __attribute__((noinline)) int x2params_ool(const CF* x, double* params, const SP& sp, int reopt) {
   return x2params<CF, VC>(x, params, sp, reopt);
 }
-template <class CF, int VC>
-__device__ inline int x2params_at(const CF* x, double* params, const Space<CF>& sp, int reopt) {
+template <class CF, int VC, class SP>
+__device__ inline int x2params_at(const CF* x, double* params, const SP& sp, int reopt) {
   if constexpr (VarF<VC>::SG) return x2params_ool<CF, VC>(x, params, sp, reopt);
   else return x2params<CF, VC>(x, params, sp, reopt);
 }
 
 // ------------------------------------------------------------------ params2x
 // cuda.c:1016-1115.
-template <class CF, int VC>
-__device__ void params2x(CF* x, const double* params, const Space<CF>& sp) {
+template <class CF, int VC, class SP>
+__device__ void params2x(CF* x, const double* params, const SP& sp) {
   using P = Pos<VC>;
   AST_VFLAGS(VC);
   constexpr int N = P::N;

@@ -132,64 +132,125 @@ struct StageCfg {
   int n_steps, eval_budget;
 };
 
+// A wave-uniform value (pointer or 64-bit size) that arrived in vector
+// registers or memory, moved to scalar registers.
+__device__ inline uint64_t uniform64(uint64_t v) {
+  const uint32_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)v);
+  const uint32_t hi = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(v >> 32));
+  return ((uint64_t)hi << 32) | lo;
+}
+// Pointers into device memory by global (not FLAT) accesses.
+template <class T>
+using GlobalPtr = __attribute__((address_space(1))) T*;
+template <class T>
+using GlobalRef = __attribute__((address_space(1))) T&;
+
+// One lane's simplex and its control flow.  Uniform members are the same for
+// the wavefront; the lane's own are its slot fit index and offsets.
 template <class CF, int VC>
 struct Machine {
   using P = Pos<VC>;
   static constexpr int N = P::N;
   static constexpr bool BC = VarF<VC>::BC;
-  const Space<CF>& sp;
-  const SlotBufs<CF>& B;
-  const StageCfg<CF>& C;
-  size_t fit, nf;   // slot fit index and slot capacity (fixed-type arrays)
-  size_t fo, rs;    // the same element in the CF arrays: offset and row stride
+  // uniform
+  SpacePtr<CF> sp;
+  GlobalPtr<CF> bX, bF, bX0, bXR, bXP, bDV;
+  GlobalPtr<uint8_t> bIND;
+  GlobalPtr<double> bPRM;
+  StageCfg<CF> C;
+  uint64_t nf, rs;  // row strides: fixed-type arrays and CF arrays
+  // the lane's
+  uint32_t fit;     // slot fit index
+  uint32_t fo;      // the same element in the CF arrays
   uint64_t jfit;    // fit index within the job (random stream)
   int reopt;
 
-  __device__ CF& X(int v, int i) const { return B.X[((size_t)v * N + i) * rs + fo]; }
-  __device__ CF& F(int v) const { return B.F[(size_t)v * rs + fo]; }
-  __device__ uint8_t& IND(int v) const { return B.IND[(size_t)v * nf + fit]; }
-  __device__ CF& X0(int i) const { return B.X0[(size_t)i * rs + fo]; }
-  __device__ CF& XR(int i) const { return B.XR[(size_t)i * rs + fo]; }
-  __device__ CF& XP(int i) const { return B.XP[(size_t)i * rs + fo]; }
-  __device__ double& PRM(int i) const { return B.PRM[(size_t)i * nf + fit]; }
+  __device__ static Machine of(const GroupDesc<CF>& D, const SlotBufs<CF>& B, size_t fit, size_t fo, uint64_t jfit,
+                               int reopt) {
+    Machine m;
+    m.sp = (SpacePtr<CF>)(uintptr_t)D.sp;
+    m.bX = (GlobalPtr<CF>)B.X;
+    m.bF = (GlobalPtr<CF>)B.F;
+    m.bX0 = (GlobalPtr<CF>)B.X0;
+    m.bXR = (GlobalPtr<CF>)B.XR;
+    m.bXP = (GlobalPtr<CF>)B.XP;
+    m.bDV = (GlobalPtr<CF>)B.DV;
+    m.bIND = (GlobalPtr<uint8_t>)B.IND;
+    m.bPRM = (GlobalPtr<double>)B.PRM;
+    m.C = StageCfg<CF>{D.seed, D.size2_min, D.n_steps, D.eval_budget};
+    m.nf = B.nf;
+    m.rs = (8 / sizeof(CF)) * B.nf;
+    m.fit = (uint32_t)fit;
+    m.fo = (uint32_t)fo;
+    m.jfit = jfit;
+    m.reopt = reopt;
+    return m;
+  }
+  // The uniform members in scalar registers.
+  __device__ void to_scalar() {
+    sp = (SpacePtr<CF>)(uintptr_t)uniform64((uint64_t)(uintptr_t)sp);
+    bX = (GlobalPtr<CF>)uniform64((uint64_t)bX);
+    bF = (GlobalPtr<CF>)uniform64((uint64_t)bF);
+    bX0 = (GlobalPtr<CF>)uniform64((uint64_t)bX0);
+    bXR = (GlobalPtr<CF>)uniform64((uint64_t)bXR);
+    bXP = (GlobalPtr<CF>)uniform64((uint64_t)bXP);
+    bDV = (GlobalPtr<CF>)uniform64((uint64_t)bDV);
+    bIND = (GlobalPtr<uint8_t>)uniform64((uint64_t)bIND);
+    bPRM = (GlobalPtr<double>)uniform64((uint64_t)bPRM);
+    nf = uniform64(nf);
+    rs = uniform64(rs);
+    C.seed = uniform64(C.seed);
+    C.n_steps = __builtin_amdgcn_readfirstlane(C.n_steps);
+    C.eval_budget = __builtin_amdgcn_readfirstlane(C.eval_budget);
+    reopt = __builtin_amdgcn_readfirstlane(reopt);
+  }
+
+  // Makes the row addresses unknown to the compiler at this point.  Else it
+  // computes those of every row of every array once, ahead of the loop they
+  // are used in, and keeps the 200 of them in scratch memory.
+  __device__ void renew() {
+    pin_sgpr(bX);
+    pin_sgpr(bF);
+    pin_sgpr(bX0);
+    pin_sgpr(bXR);
+    pin_sgpr(bXP);
+    pin_sgpr(bIND);
+    pin_sgpr(bPRM);
+  }
+
+  // Element of a row: a scalar row address and the lane's 32-bit byte offset
+  // (at least 1 KB of state per fit keeps 8 * nf far below 2^32).
+  template <class T>
+  __device__ static GlobalRef<T> at(GlobalPtr<T> base, uint64_t row_stride, int row, uint32_t lane_index) {
+    return *(GlobalPtr<T>)((GlobalPtr<char>)(base + (uint64_t)row * row_stride) + lane_index * (uint32_t)sizeof(T));
+  }
+  __device__ GlobalRef<CF> X(int v, int i) const { return at(bX, rs, v * N + i, fo); }
+  __device__ GlobalRef<CF> F(int v) const { return at(bF, rs, v, fo); }
+  __device__ GlobalRef<uint8_t> IND(int v) const { return at(bIND, nf, v, fit); }
+  __device__ GlobalRef<CF> X0(int i) const { return at(bX0, rs, i, fo); }
+  __device__ GlobalRef<CF> XR(int i) const { return at(bXR, rs, i, fo); }
+  __device__ GlobalRef<CF> XP(int i) const { return at(bXP, rs, i, fo); }
+  __device__ GlobalRef<CF> DVL(int m) const { return at(bDV, rs, m, fo); }
+  __device__ GlobalRef<double> PRM(int i) const { return at(bPRM, nf, i, fit); }
 
   // x2params on a point, through the persistent params[] buffer.
   __device__ bool propose(const CF* xv) const {
     double prm[N];
 #pragma unroll
     for (int i = 0; i < N; ++i) prm[i] = PRM(i);
-    int rc = x2params_at<CF, VC>(xv, prm, sp, reopt);
+    int rc = x2params_at<CF, VC>(xv, prm, *sp, reopt);
 #pragma unroll
     for (int i = 0; i < N; ++i) PRM(i) = prm[i];
     return rc == 0;
-  }
-  __device__ bool propose_row(int v) const {
-    CF xv[N];
-#pragma unroll
-    for (int i = 0; i < N; ++i) xv[i] = X(v, i);
-    return propose(xv);
-  }
-  __device__ bool propose_xr() const {
-    CF xv[N];
-#pragma unroll
-    for (int i = 0; i < N; ++i) xv[i] = XR(i);
-    return propose(xv);
-  }
-  __device__ bool propose_xp() const {
-    CF xv[N];
-#pragma unroll
-    for (int i = 0; i < N; ++i) xv[i] = XP(i);
-    return propose(xv);
   }
 
   __device__ float rnd(LaneRegs<CF>& R) const { return astrng::uniform01(C.seed, jfit, R.rng++); }
 
   // Stage start (cuda.c:1456-1546): x[0] random or around the reoptimised
   // point, then the N displaced vertices.
-  __device__ void start(LaneRegs<CF>& R) const {
+  __device__ void start(LaneRegs<CF>& R, CF* x0v) const {
     const CF DX_INI = (CF)0.001, D2X_INI = (CF)-1.2, DX_RAND = (CF)0.0001;  // asteroid.h:205-209
     int LAM = 0;
-    CF x0v[N];
 #pragma unroll
     for (int i = 0; i < N; ++i) x0v[i] = X(0, i);
     for (int i = 0; i < N; ++i) {
@@ -198,9 +259,9 @@ struct Machine {
         if (i == P::c) { x0v[i] = x0v[P::c_tumb]; continue; }
         if (i == P::b) { x0v[i] = x0v[P::b_tumb]; continue; }
       }
-      int per = sp.periodic[i];
+      int per = sp->periodic[i];
       CF xi;
-      if (!reopt || (reopt && sp.frozen[i] == -1)) {
+      if (!reopt || (reopt && sp->frozen[i] == -1)) {
         xi = DX_INI + SMALL + r * (1.0 - 2 * (SMALL + DX_INI));
       } else {
         CF xmin = x0v[i] - DX_RAND;
@@ -217,7 +278,7 @@ struct Machine {
     for (int jj = 1; jj < N + 1; ++jj) {
       for (int i = 0; i < N; ++i) {
         if (i == jj - 1) {
-          int per = sp.periodic[i];
+          int per = sp->periodic[i];
           float d2x = rnd(R);
           CF dx = DX_INI * cf_exp((CF)(D2X_INI * d2x));
           if (rnd(R) < 0.5) {
@@ -255,15 +316,15 @@ struct Machine {
       const int b = IND(0);
 #pragma unroll
       for (int i = 0; i < N; ++i) { xb[i] = X(b, i); prm[i] = PRM(i); }
-      x2params_at<CF, VC>(xb, prm, sp, reopt);
+      x2params_at<CF, VC>(xb, prm, *sp, reopt);
 #pragma unroll
       for (int i = 0; i < N; ++i) D.fit_params[jfit * N + i] = prm[i];
     }
-    for (int m = 0; m < D.n_filters; ++m) D.fit_dV[jfit * D.n_filters + m] = B.DV[(size_t)m * rs + fo];
+    for (int m = 0; m < D.n_filters; ++m) D.fit_dV[jfit * D.n_filters + m] = DVL(m);
   }
 
   // The lane's state for a new fit (as fit_init_kernel leaves a group's
-  // lanes), then its stage start.
+  // lanes): PH_START.
   __device__ void begin_fit(LaneRegs<CF>& R, const GroupDesc<CF>& D) const {
 #pragma unroll
     for (int v = 0; v <= N; ++v) IND(v) = (uint8_t)v;
@@ -273,203 +334,281 @@ struct Machine {
 #pragma unroll
     for (int i = 0; i < N; ++i) PRM(i) = prm[i];
     CF x[N];
-    if (reopt) params2x<CF, VC>(x, prm, sp);
+    if (reopt) params2x<CF, VC>(x, prm, *sp);
     else
       for (int i = 0; i < N; ++i) x[i] = 0;
 #pragma unroll
     for (int i = 0; i < N; ++i) X(0, i) = x[i];
-    for (int m = 0; m < MAXF; ++m) B.DV[(size_t)m * rs + fo] = 0;
+    for (int m = 0; m < MAXF; ++m) DVL(m) = 0;
     R.phase = PH_START;
     R.nev_tot = 0;
     R.steps_tot = 0;
     R.rng = D.rng[jfit];
     R.fr = 0;
     R.sf = (CF)1e30;
-    advance(R, (CF)0, false);
   }
 
-  __device__ void replace_worst_with_xr(CF fv) const {
+  __device__ void replace_worst(GlobalPtr<CF> point, CF fv) const {
     const int w = IND(N);
+    CF xn[N];
 #pragma unroll
-    for (int i = 0; i < N; ++i) X(w, i) = XR(i);
+    for (int i = 0; i < N; ++i) xn[i] = at(point, rs, i, fo);
+#pragma unroll
+    for (int i = 0; i < N; ++i) X(w, i) = xn[i];
     F(w) = fv;
   }
-  __device__ void replace_worst_with_xp(CF fv) const {
-    const int w = IND(N);
+
+  // The vertices in order of chi^2 (cuda.c:1570-1600), and the worst one: the
+  // reference takes the lowest value left, the last vertex of equal ones.
+  __device__ int sort_vertices() const {
+    CF f[N + 1];
 #pragma unroll
-    for (int i = 0; i < N; ++i) X(w, i) = XP(i);
-    F(w) = fv;
+    for (int v = 0; v <= N; ++v) f[v] = F(v);
+    bool plain = true;  // every value can be taken (none is NaN or above 1e30)
+#pragma unroll
+    for (int v = 0; v <= N; ++v) plain = plain && f[v] <= (CF)1e30;
+    if (plain) {
+      // A vertex's place is the number of those before it: one comparison
+      // per pair.
+      int place[N + 1];
+#pragma unroll
+      for (int v = 0; v <= N; ++v) place[v] = v;
+#pragma unroll
+      for (int v = 1; v <= N; ++v)
+#pragma unroll
+        for (int u = 0; u < v; ++u) {
+          const int after = f[v] <= f[u] ? 1 : 0;  // v comes before u
+          place[u] += after;
+          place[v] -= after;
+        }
+      int w = 0;
+#pragma unroll
+      for (int v = 0; v <= N; ++v) {
+        IND(place[v]) = (uint8_t)v;
+        if (place[v] == N) w = v;
+      }
+      return w;
+    }
+    uint64_t taken = 0;
+#pragma unroll 1
+    for (int v = 0; v <= N; ++v) {
+      CF fmin = 1e30;
+      int jmin = -1;
+#pragma unroll 1
+      for (int u = 0; u <= N; ++u) {
+        const CF fu = F(u);
+        if (!((taken >> u) & 1) && fu <= fmin) { fmin = fu; jmin = u; }
+      }
+      if (jmin < 0) {  // NaN values left (cuda.c:1592-1598)
+        IND(0) = 0;
+        F(0) = 1e30;
+        break;
+      }
+      IND(v) = (uint8_t)jmin;
+      taken |= 1ull << jmin;
+    }
+    return IND(N);
+  }
+
+  // K elements of the simplex, from row `first` on every `stride` rows.
+  template <int K>
+  __device__ void fetch(CF* out, int first, int stride) const {
+    const uint64_t step = (uint64_t)stride * rs * sizeof(CF);
+    uint64_t p = (uint64_t)bX + (uint64_t)first * rs * sizeof(CF);
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+      pin_sgpr(p);
+      out[k] = *(GlobalPtr<CF>)((GlobalPtr<char>)p + fo * (uint32_t)sizeof(CF));
+      p += step;
+    }
+  }
+
+  // The top of the simplex loop (cuda.c:1568-1645): sort, centroid, size and
+  // the stopping tests; false if the stage is over, else the reflected point
+  // in xv.
+  __device__ bool begin_step(LaneRegs<CF>& R, CF* xv) const {
+    const CF ALPHA = 1.0;  // asteroid.h:239
+    constexpr int UN = N <= 16 ? N : 1;  // whole rows in registers for the smaller simplexes
+    R.l++;
+    const int w = sort_vertices();
+    // Column by column for the centroid, then row by row for the size, each
+    // fetched while the one before it is summed.
+    CF x0[N];
+    CF cur[N + 1], nxt[N + 1];
+    fetch<N + 1>(cur, 0, N);
+#pragma unroll(UN)
+    for (int i = 0; i < N; ++i) {
+      if (i + 1 < N) fetch<N + 1>(nxt, i + 1, N);
+      else fetch<N>(nxt, 0, 1);
+      __builtin_amdgcn_sched_barrier(0);
+      CF sum = 0.0;
+#pragma unroll
+      for (int v = 0; v < N + 1; ++v) sum = sum + cur[v];
+      x0[i] = sum / (N + 1);
+#pragma unroll
+      for (int v = 0; v < N + 1; ++v) cur[v] = nxt[v];
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    CF size2 = 0.0;
+#pragma unroll(UN)
+    for (int v = 0; v < N + 1; ++v) {
+      if (v < N) fetch<N>(nxt, (v + 1) * N, 1);
+      __builtin_amdgcn_sched_barrier(0);
+      CF sum = 0.0;
+#pragma unroll
+      for (int i = 0; i < N; ++i) {
+        CF dx = cur[i] - x0[i];
+        sum = sum + dx * dx;
+      }
+      size2 = size2 + sum;
+#pragma unroll
+      for (int i = 0; i < N; ++i) cur[i] = nxt[i];
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    size2 = size2 / N;
+    if (size2 < C.size2_min || R.l > C.n_steps || (C.eval_budget > 0 && R.nev >= C.eval_budget)) return false;
+    CF xw[N];
+#pragma unroll
+    for (int i = 0; i < N; ++i) xw[i] = X(w, i);
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+      xv[i] = (sp->frozen[i] != 1) ? (CF)(x0[i] + ALPHA * (x0[i] - xw[i])) : xw[i];
+      X0(i) = x0[i];
+      XR(i) = xv[i];
+    }
+    return true;
   }
 
   // Advance the lane until it has a pending point or its stage is over.
-  // `val` is the chi^2 of the pending point when has_result.
-  __device__ __attribute__((noinline)) void advance(LaneRegs<CF>& R, CF val, bool has_result) const {
-    const CF ALPHA = 1.0, GAMMA = 2.0, RHO = 0.5, SIGMA = 0.5;  // asteroid.h:239-242
+  // `val` is the chi^2 of the pending point when has_result.  The lanes of a
+  // wavefront are in different phases, so each part of the control flow
+  // stands once in a pass and what follows from it behind it: the decision
+  // about the value, the next vertex of a shrink, the top of the simplex
+  // loop, and one proposal for whatever point came out of them.  (With a
+  // proposal per phase a pass ran the parameter map up to four times, and
+  // with pointers read through memory every load of the simplex was waited
+  // for by itself: 110 us per round of 64-lane FP64 fits of 11 parameters,
+  // 370 us with the chip full, of 580 and 2900 us.)
+  __device__ void advance(LaneRegs<CF>& R, CF val, bool has_result) {
+    const CF GAMMA = 2.0, RHO = 0.5, SIGMA = 0.5;  // asteroid.h:240-242
     if (!has_result && R.phase != PH_START) return;
+    CF xv[N];
     for (;;) {
-      switch (R.phase) {
-        case PH_START: {
-          start(R);
-          R.l = 0;
-          R.nev = 0;
-          R.failed = 0;
-          R.bad = 0;
-          R.j = 0;
-          R.phase = PH_INIT;
-          if (propose_row(0)) return;
-          R.failed = 1;
+      renew();
+      if (R.phase == PH_START) {
+        start(R, xv);
+        R.l = 0;
+        R.nev = 0;
+        R.failed = 0;
+        R.bad = 0;
+        R.j = 0;
+        R.phase = PH_INIT;
+      } else if (R.phase == PH_INIT) {  // cuda.c:1550-1559
+        F(R.j) = val;
+        R.j++;
+        if (R.j <= N) {
+#pragma unroll
+          for (int i = 0; i < N; ++i) xv[i] = X(R.j, i);
+        } else {
           R.phase = PH_BEGIN;
-          break;
         }
-        case PH_INIT: {  // cuda.c:1550-1559
-          F(R.j) = val;
-          R.j++;
-          if (R.j <= N) {
-            if (propose_row(R.j)) return;
-            R.failed = 1;
-          }
+      } else if (R.phase == PH_REFLECT) {  // cuda.c:1646-1712 (decisions after the reflection)
+        R.fr = val;
+        const CF fb = F(IND(0));
+        if (val >= fb && val < F(IND(N - 1))) {
+          replace_worst(bXR, val);
           R.phase = PH_BEGIN;
-          break;
-        }
-        case PH_BEGIN: {  // cuda.c:1568-1645
-          if (R.failed) { finish(R); return; }
-          R.l++;
-          CF f[N + 1];
-          int ind[N + 1];
-#pragma unroll
-          for (int v = 0; v <= N; ++v) { f[v] = F(v); ind[v] = IND(v); }
-          bool taken[N + 1];
-#pragma unroll
-          for (int v = 0; v <= N; ++v) taken[v] = false;
-          for (int v = 0; v <= N; ++v) {
-            CF fmin = 1e30;
-            int jmin = -1;
-#pragma unroll
-            for (int v2 = 0; v2 <= N; ++v2)
-              if (!taken[v2] && f[v2] <= fmin) { fmin = f[v2]; jmin = v2; }
-            if (jmin < 0) {  // NaN values left (cuda.c:1592-1598)
-              ind[0] = 0;
-              F(0) = 1e30;
-              break;
-            }
-            ind[v] = jmin;
-#pragma unroll
-            for (int v2 = 0; v2 <= N; ++v2)
-              if (v2 == jmin) taken[v2] = true;
-          }
-#pragma unroll
-          for (int v = 0; v <= N; ++v) IND(v) = (uint8_t)ind[v];
-          CF x0[N];
-          for (int i = 0; i < N; ++i) {
-            CF sum = 0.0;
-            for (int v = 0; v < N + 1; ++v) sum = sum + X(v, i);
-            x0[i] = sum / (N + 1);
-          }
-          CF size2 = 0.0;
-          for (int v = 0; v < N + 1; ++v) {
-            CF sum = 0.0;
-#pragma unroll
-            for (int i = 0; i < N; ++i) {
-              CF dx = X(v, i) - x0[i];
-              sum = sum + dx * dx;
-            }
-            size2 = size2 + sum;
-          }
-          size2 = size2 / N;
-          if (size2 < C.size2_min || R.l > C.n_steps || (C.eval_budget > 0 && R.nev >= C.eval_budget)) {
-            finish(R);
-            return;
-          }
-          const int w = ind[N];
-#pragma unroll
-          for (int i = 0; i < N; ++i) {
-            X0(i) = x0[i];
-            CF xw = X(w, i);
-            XR(i) = (sp.frozen[i] != 1) ? (CF)(x0[i] + ALPHA * (x0[i] - xw)) : xw;
-          }
-          R.phase = PH_REFLECT;
-          if (propose_xr()) return;
-          val = 1e30;
-          break;
-        }
-        case PH_REFLECT: {  // cuda.c:1646-1712 (decisions after the reflection)
-          R.fr = val;
-          const CF fb = F(IND(0));
-          if (val >= fb && val < F(IND(N - 1))) {
-            replace_worst_with_xr(val);
-            R.phase = PH_BEGIN;
-            break;
-          }
-          if (val < fb) {
-#pragma unroll
-            for (int i = 0; i < N; ++i) {
-              CF xr = XR(i);
-              XP(i) = (sp.frozen[i] != 1) ? (CF)(X0(i) + GAMMA * (xr - X0(i))) : xr;
-            }
-            R.phase = PH_EXPAND;
-            if (propose_xp()) return;
-            val = 1e30;
-            break;
-          }
+        } else {
+          // expansion (from the reflected point) or contraction (from the worst)
+          const bool expand = val < fb;
+          const CF k = expand ? GAMMA : RHO;
           const int w = IND(N);
+          CF xf[N], x0[N];
 #pragma unroll
           for (int i = 0; i < N; ++i) {
-            CF xw = X(w, i);
-            XP(i) = (sp.frozen[i] != 1) ? (CF)(X0(i) + RHO * (xw - X0(i))) : xw;
+            xf[i] = expand ? XR(i) : X(w, i);
+            x0[i] = X0(i);
           }
-          R.phase = PH_CONTRACT;
-          if (propose_xp()) return;
-          val = 1e30;
-          break;
+#pragma unroll
+          for (int i = 0; i < N; ++i) {
+            xv[i] = (sp->frozen[i] != 1) ? (CF)(x0[i] + k * (xf[i] - x0[i])) : xf[i];
+            XP(i) = xv[i];
+          }
+          R.phase = expand ? PH_EXPAND : PH_CONTRACT;
         }
-        case PH_EXPAND: {  // cuda.c:1671-1689
-          if (val < R.fr) replace_worst_with_xp(val);
-          else replace_worst_with_xr(R.fr);
+      } else if (R.phase == PH_EXPAND) {  // cuda.c:1671-1689
+        const bool better = val < R.fr;
+        replace_worst(better ? bXP : bXR, better ? val : R.fr);
+        R.phase = PH_BEGIN;
+      } else if (R.phase == PH_CONTRACT) {  // cuda.c:1703-1712
+        if (val < F(IND(N))) {
+          replace_worst(bXP, val);
           R.phase = PH_BEGIN;
-          break;
-        }
-        case PH_CONTRACT: {  // cuda.c:1703-1712
-          if (val < F(IND(N))) {
-            replace_worst_with_xp(val);
-            R.phase = PH_BEGIN;
-            break;
-          }
+        } else {
           R.bad = 0;
           R.j = 1;
           R.phase = PH_SHRINK_NEXT;
-          break;
         }
-        case PH_SHRINK: {  // cuda.c:1726
-          F(IND(R.j)) = val;
-          R.j++;
-          R.phase = PH_SHRINK_NEXT;
-          break;
-        }
-        case PH_SHRINK_NEXT: {  // cuda.c:1716-1733
-          while (R.j <= N) {
-            const int v = IND(R.j), b = IND(0);
-            CF xv[N];
+      } else if (R.phase == PH_SHRINK) {  // cuda.c:1726
+        F(IND(R.j)) = val;
+        R.j++;
+        R.phase = PH_SHRINK_NEXT;
+      }
+      if (R.phase == PH_SHRINK_NEXT) {  // cuda.c:1716-1733
+        if (R.j <= N) {
+          const int v = IND(R.j), b = IND(0);
+          CF xb[N];
 #pragma unroll
-            for (int i = 0; i < N; ++i) {
-              CF xi = X(v, i);
-              if (sp.frozen[i] != 1) xi = X(b, i) + SIGMA * (xi - X(b, i));
-              xv[i] = xi;
-              X(v, i) = xi;
-            }
-            if (propose(xv)) { R.phase = PH_SHRINK; return; }
-            R.bad = 1;
-            R.j++;
+          for (int i = 0; i < N; ++i) {
+            xv[i] = X(v, i);
+            xb[i] = X(b, i);
           }
+#pragma unroll
+          for (int i = 0; i < N; ++i) {
+            if (sp->frozen[i] != 1) xv[i] = xb[i] + SIGMA * (xv[i] - xb[i]);
+            X(v, i) = xv[i];
+          }
+        } else {
           if (R.bad) R.failed = 1;
           R.phase = PH_BEGIN;
-          break;
         }
-        default:
+      }
+      if (R.phase == PH_BEGIN) {
+        if (R.failed || !begin_step(R, xv)) {
+          finish(R);
           return;
+        }
+        R.phase = PH_REFLECT;
+      }
+      if (propose(xv)) {
+        if (R.phase == PH_SHRINK_NEXT) R.phase = PH_SHRINK;
+        return;
+      }
+      // outside the hard limits
+      if (R.phase == PH_INIT) {
+        R.failed = 1;
+        R.phase = PH_BEGIN;
+      } else if (R.phase == PH_SHRINK_NEXT) {
+        R.bad = 1;
+        R.j++;
+      } else {
+        val = 1e30;
       }
     }
   }
 };
+
+// advance() out of line, one copy for the kernels of a simplex type: its
+// registers do not compete with the evaluator's.
+template <class CF, int VC>
+__device__ __attribute__((noinline)) void advance_lane(const Machine<CF, VC>& machine, LaneRegs<CF>& regs, CF val,
+                                                       bool has_result) {
+  Machine<CF, VC> m = machine;
+  m.to_scalar();
+  LaneRegs<CF> R = regs;
+  m.advance(R, val, has_result);
+  regs = R;
+}
 
 // --------------------------------------------------------------- init kernel
 // A group's start (one workgroup of G threads per new group): identity sort
@@ -607,7 +746,7 @@ __device__ bool group_stage_end(const GroupDesc<CF>& D, const Machine<CF, VC>& M
   __shared__ CF s_x0[MAXP];
   __shared__ int s_tm;
   __shared__ CF s_smin;
-  const Space<CF>& sp = M.sp;
+  const SpacePtr<CF> sp = M.sp;
   s_f[t] = R.sf;
   __syncthreads();
   if (t == 0) {
@@ -627,12 +766,12 @@ __device__ bool group_stage_end(const GroupDesc<CF>& D, const Machine<CF, VC>& M
       const int b = M.IND(0);
 #pragma unroll
       for (int i = 0; i < N; ++i) xb[i] = M.X(b, i);
-      if (sp.p_psi && reopt == 0) {  // cuda.c:1791-1798
+      if (sp->p_psi && reopt == 0) {  // cuda.c:1791-1798
         double prm[N];
 #pragma unroll
         for (int i = 0; i < N; ++i) prm[i] = M.PRM(i);
-        x2params_at<CF, VC>(xb, prm, sp, reopt);
-        params2x<CF, VC>(xb, prm, sp);
+        x2params_at<CF, VC>(xb, prm, *sp, reopt);
+        params2x<CF, VC>(xb, prm, *sp);
 #pragma unroll
         for (int i = 0; i < N; ++i) { M.PRM(i) = prm[i]; M.X(b, i) = xb[i]; }
       }
@@ -655,14 +794,14 @@ __device__ bool group_stage_end(const GroupDesc<CF>& D, const Machine<CF, VC>& M
     const int b = M.IND(0);
 #pragma unroll
     for (int i = 0; i < N; ++i) { xb[i] = M.X(b, i); prm[i] = M.PRM(i); }
-    x2params_at<CF, VC>(xb, prm, sp, reopt);
+    x2params_at<CF, VC>(xb, prm, *sp, reopt);
 #pragma unroll
     for (int i = 0; i < N; ++i) {
       M.PRM(i) = prm[i];
       D.best_params[(size_t)g * N + i] = prm[i];
     }
     for (int m = 0; m < D.n_filters; ++m)
-      D.best_dV[(size_t)g * D.n_filters + m] = M.B.DV[(size_t)m * M.rs + M.fo];
+      D.best_dV[(size_t)g * D.n_filters + m] = M.DVL(m);
   }
   D.fit_f[M.jfit] = R.sf;
   D.fit_nev[M.jfit] = R.nev_tot;
@@ -727,59 +866,55 @@ void fit_kernel(const GroupDesc<CF>* descs, SlotBufs<CF> B) {
   const size_t fit = (size_t)slot * G + t;
   const size_t fo = (size_t)slot * G * KC + t;
   if (B.g_done[slot]) return;  // same value for every thread of the group
-  uint64_t jfit = (uint64_t)B.fitid[fit];  // group_in_job * G + t unless the lane has refilled
-  const Space<CF>& sp = *D.sp;
-  const StageCfg<CF> SC{D.seed, D.size2_min, D.n_steps, D.eval_budget};
+  // group_in_job * G + t unless the lane has refilled
+  Machine<CF, VC> M = Machine<CF, VC>::of(D, B, fit, fo, (uint64_t)B.fitid[fit], B.g_reopt[slot]);
   const int ticks = D.ticks;
-  int reopt = B.g_reopt[slot];
   int stage = B.g_stage[slot];
-  LaneRegs<CF> R = load_lane(B, fit, fo, D.rng[jfit]);
+  LaneRegs<CF> R = load_lane(B, fit, fo, D.rng[M.jfit]);
   const bool refill = D.refill != 0;
   bool done = false;
-  {
-    Machine<CF, VC> M{sp, B, SC, fit, nf, fo, rs, jfit, reopt};
-    M.advance(R, (CF)0, false);  // a lane at a stage start draws its simplex first
-  }
-  for (int tick = 0; tick < ticks && !done; ++tick) {
-    Machine<CF, VC> M{sp, B, SC, fit, nf, fo, rs, jfit, reopt};
-    if (phase_pending(R.phase)) {
-      CF fv = eval_lane<CF, VC, NF, MX, MX ? 4 : W>(B.PRM, B.DV, nf, fit, rs, fo, D.pts, D.n_data, D.n_filters, D.dof,
-                                            D.sum_w);
-      R.nev++;
-      R.nev_tot++;
-      R.work++;
-      M.advance(R, fv, true);
-    }
+  CF fv = 0;
+  bool have = false;
+  for (int tick = 0;;) {
+    advance_lane<CF, VC>(M, R, fv, have);  // a lane at a stage start draws its simplex
     if (refill) {
       // A lane whose fit ended keeps its results and starts the job's next
       // unstarted fit (one that fails at its start ends at once and the lane
       // takes another); with the queue empty it idles.  The group is done
       // when every lane idles.
       while (R.phase == PH_STAGE_DONE) {
-        Machine<CF, VC> Me{sp, B, SC, fit, nf, fo, rs, jfit, reopt};
-        Me.end_fit(R, D);
+        M.end_fit(R, D);
         const int nj = take_fit(D.queue);
         if (nj >= D.n_fits) {
           R.phase = PH_FIT_DONE;
           break;
         }
-        jfit = (uint64_t)nj;
-        Machine<CF, VC> Mb{sp, B, SC, fit, nf, fo, rs, jfit, reopt};
-        Mb.begin_fit(R, D);
+        M.jfit = (uint64_t)nj;
+        M.begin_fit(R, D);
+        advance_lane<CF, VC>(M, R, (CF)0, false);
       }
       if (__syncthreads_count(R.phase != PH_FIT_DONE) == 0) done = true;
-      continue;
-    }
-    const int running = __syncthreads_count(phase_pending(R.phase));
-    if (running) continue;
-    // Every simplex of the group finished the stage.
-    if (group_stage_end<CF, VC>(D, M, R, t, G, stage, reopt)) {
-      Machine<CF, VC> M2{sp, B, SC, fit, nf, fo, rs, jfit, reopt};
-      M2.advance(R, (CF)0, false);
-    } else {
+    } else if (!__syncthreads_count(phase_pending(R.phase))) {
+      // Every simplex of the group finished the stage.
+      if (group_stage_end<CF, VC>(D, M, R, t, G, stage, M.reopt)) {
+        have = false;
+        continue;
+      }
       done = true;
     }
+    if (done || tick == ticks) break;
+    ++tick;
+    have = phase_pending(R.phase);
+    if (have) {
+      fv = eval_lane<CF, VC, NF, MX, MX ? 4 : W>(B.PRM, B.DV, nf, fit, rs, fo, D.pts, D.n_data, D.n_filters, D.dof,
+                                                 D.sum_w);
+      R.nev++;
+      R.nev_tot++;
+      R.work++;
+    }
   }
+  const uint64_t jfit = M.jfit;
+  const int reopt = M.reopt;
   store_lane(B, fit, fo, R, jfit);
   D.rng[jfit] = R.rng;
   if (t == 0) {
@@ -890,52 +1025,47 @@ __device__ inline int take_fit_rows(int32_t* queue) {
 template <class CF, int VC, int NF, bool MX, int LP>
 __global__ AST_ROWS_BOUNDS void fit_rows_kernel(const GroupDesc<CF>* descs, SlotBufs<CF> B, int G) {
   astm::sincos_table_load();
-  constexpr int KC = 8 / sizeof(CF), M = 64 / LP;
-  const int per_group = G / M;
+  constexpr int KC = 8 / sizeof(CF), MODELS = 64 / LP;
+  const int per_group = G / MODELS;
   const GroupDesc<CF>& D = descs[blockIdx.x / per_group];
-  const int t = (int)(blockIdx.x % per_group) * M + (int)threadIdx.x / LP;
+  const int t = (int)(blockIdx.x % per_group) * MODELS + (int)threadIdx.x / LP;
   const int slot = D.slot;
   const size_t nf = B.nf, rs = KC * nf;
   const size_t fit = (size_t)slot * G + t;
   const size_t fo = (size_t)slot * G * KC + t;
   if (B.g_done[slot]) return;
-  uint64_t jfit = (uint64_t)B.fitid[fit];
-  const Space<CF>& sp = *D.sp;
-  const StageCfg<CF> SC{D.seed, D.size2_min, D.n_steps, D.eval_budget};
+  Machine<CF, VC> M = Machine<CF, VC>::of(D, B, fit, fo, (uint64_t)B.fitid[fit], B.g_reopt[slot]);
   const int ticks = D.ticks;
-  const int reopt = B.g_reopt[slot];
-  LaneRegs<CF> R = load_lane(B, fit, fo, D.rng[jfit]);
+  LaneRegs<CF> R = load_lane(B, fit, fo, D.rng[M.jfit]);
   const bool refill = D.refill != 0;
-  if (R.phase == PH_START) {
-    Machine<CF, VC> Ms{sp, B, SC, fit, nf, fo, rs, jfit, reopt};
-    Ms.advance(R, (CF)0, false);
-  }
-  for (int tick = 0; tick < ticks; ++tick) {
-    if (phase_pending(R.phase)) {
-      CF fv = eval_rows<CF, VC, NF, MX, LP>(B.PRM + fit, nf, B.DV + fo, rs, D.pts, D.n_data, D.n_filters, D.dof,
-                                            D.sum_w);
-      R.nev++;
-      R.nev_tot++;
-      R.work++;
-      Machine<CF, VC> Mt{sp, B, SC, fit, nf, fo, rs, jfit, reopt};
-      Mt.advance(R, fv, true);
-    }
+  CF fv = 0;
+  bool have = false;
+  for (int tick = 0;; ++tick) {
+    advance_lane<CF, VC>(M, R, fv, have);
     if (refill) {  // as in fit_kernel
       while (R.phase == PH_STAGE_DONE) {
-        Machine<CF, VC> Me{sp, B, SC, fit, nf, fo, rs, jfit, reopt};
-        Me.end_fit(R, D);
+        M.end_fit(R, D);
         const int nj = take_fit_rows<LP>(D.queue);
         if (nj >= D.n_fits) {
           R.phase = PH_FIT_DONE;
           break;
         }
-        jfit = (uint64_t)nj;
-        Machine<CF, VC> Mb{sp, B, SC, fit, nf, fo, rs, jfit, reopt};
-        Mb.begin_fit(R, D);
+        M.jfit = (uint64_t)nj;
+        M.begin_fit(R, D);
+        advance_lane<CF, VC>(M, R, (CF)0, false);
       }
     }
-    if (__ballot(phase_pending(R.phase)) == 0) break;
+    have = phase_pending(R.phase);
+    if (tick == ticks || __ballot(have) == 0) break;
+    if (have) {
+      fv = eval_rows<CF, VC, NF, MX, LP>(B.PRM + fit, nf, B.DV + fo, rs, D.pts, D.n_data, D.n_filters, D.dof,
+                                         D.sum_w);
+      R.nev++;
+      R.nev_tot++;
+      R.work++;
+    }
   }
+  const uint64_t jfit = M.jfit;
   store_lane(B, fit, fo, R, jfit);
   D.rng[jfit] = R.rng;
 }
@@ -956,9 +1086,8 @@ __global__ __launch_bounds__(1024) void group_step_kernel(const GroupDesc<CF>* d
   int stage = B.g_stage[slot], reopt = B.g_reopt[slot];
   if (!D.refill) {
     const uint64_t jfit = (uint64_t)B.fitid[fit];
-    const StageCfg<CF> SC{D.seed, D.size2_min, D.n_steps, D.eval_budget};
     LaneRegs<CF> R = load_lane(B, fit, fo, D.rng[jfit]);
-    Machine<CF, VC> M{*D.sp, B, SC, fit, nf, fo, rs, jfit, reopt};
+    const Machine<CF, VC> M = Machine<CF, VC>::of(D, B, fit, fo, jfit, reopt);
     done = !group_stage_end<CF, VC>(D, M, R, t, G, stage, reopt);
     store_lane(B, fit, fo, R, jfit);
   }
@@ -1102,7 +1231,7 @@ __global__ __launch_bounds__(W == 4 ? 1024 : 256) __attribute__((amdgpu_waves_pe
   __shared__ int32_t s_cnt[2][1024];
   const int t = threadIdx.x;
   const uint64_t id = (uint64_t)blockIdx.x * blockDim.x + t;
-  const Space<CF>& sp = *A.sp;
+  const auto& sp = *(SpacePtr<CF>)(uintptr_t)A.sp;
   const RmsdRef<CF>& R = *A.ref;
   CF pmin[N], pmax[N];
   for (int i = 0; i < N; ++i) { pmin[i] = (CF)1e30; pmax[i] = (CF)-1e30; }
