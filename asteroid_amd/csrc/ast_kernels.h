@@ -436,7 +436,7 @@ struct Machine {
     CF x0[N];
     CF cur[N + 1], nxt[N + 1];
     fetch<N + 1>(cur, 0, N);
-#pragma unroll(UN)
+#pragma unroll UN
     for (int i = 0; i < N; ++i) {
       if (i + 1 < N) fetch<N + 1>(nxt, i + 1, N);
       else fetch<N>(nxt, 0, 1);
@@ -450,7 +450,7 @@ struct Machine {
       __builtin_amdgcn_sched_barrier(0);
     }
     CF size2 = 0.0;
-#pragma unroll(UN)
+#pragma unroll UN
     for (int v = 0; v < N + 1; ++v) {
       if (v < N) fetch<N>(nxt, (v + 1) * N, 1);
       __builtin_amdgcn_sched_barrier(0);
