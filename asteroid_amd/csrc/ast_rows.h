@@ -145,9 +145,12 @@ __device__ CF chi2_model_rows(const double* params, PointPtr pts, LanePtr pts_g,
   static_assert(!(TR && (T2 || NU)), "PointRec.aux is the phase angle under TREND and the time otherwise");
   const int lane = (int)__lane_id() & (LP - 1);
   const bool odd = lane & 1;
-  double sy2[NF], sy[NF];
+  // With several filters a lane keeps the sums of filter lane (and lane + LP
+  // where there are more filters than lanes); with one, every lane keeps them.
+  constexpr int SLOTS = NF == 1 ? 1 : (NF + LP - 1) / LP;
+  double sy2[SLOTS], sy[SLOTS];
 #pragma unroll
-  for (int m = 0; m < NF; ++m) { sy2[m] = 0.0; sy[m] = 0.0; }
+  for (int m = 0; m < SLOTS; ++m) { sy2[m] = 0.0; sy[m] = 0.0; }
   const double bt = params[P::b_tumb], ct = params[P::c_tumb];
   const double den = __builtin_fma(ct, ct, bt * bt);
   const double Is = __builtin_fma(bt, bt, 1.0) / den;
@@ -230,6 +233,8 @@ __device__ CF chi2_model_rows(const double* params, PointPtr pts, LanePtr pts_g,
     const float pV = pr->V, pw = pr->w;
     double aux = 0.0;
     if constexpr (TR) aux = pr->aux;
+    int lane_filter = 0;
+    if constexpr (NF > 1) lane_filter = pr->filter;
     double cphi = 0.0, cth = 0.0, cps = 0.0;  // the Euler angles at the lane's point
     SpinFrame<double> Fl = Fd;                // and, with segments, its spin frame
     for (int j = 0; j < m; ++j) {
@@ -328,10 +333,10 @@ __device__ CF chi2_model_rows(const double* params, PointPtr pts, LanePtr pts_g,
         sy2[0] = __builtin_fma(qj, wj, sy2[0]);
         sy[0] = __builtin_fma(yj, wj, sy[0]);
       } else {
-        const int f = pts[i0 + (j < m ? j : m - 1)].filter;
+        const int f = __builtin_amdgcn_readlane(lane_filter, row0 + j);
 #pragma unroll
-        for (int k = 0; k < NF; ++k)
-          if (f == k) {
+        for (int k = 0; k < SLOTS; ++k)
+          if (lane + k * LP == f) {
             sy2[k] = __builtin_fma(qj, wj, sy2[k]);
             sy[k] = __builtin_fma(yj, wj, sy[k]);
           }
@@ -341,7 +346,13 @@ __device__ CF chi2_model_rows(const double* params, PointPtr pts, LanePtr pts_g,
   if constexpr (FORM == FORM_PLOT) return CF(0.0);
   if constexpr (NU)
     if (nu.failed) return CF(1e30);
-  return model_score<CF, VC, NF, FORM>(sy2, sy, n_filters, dof, sum_w, dV, NU ? &nu : nullptr, mr);
+  double all2[NF], all1[NF];
+  unroll_lanes<NF>([&](auto mc) {
+    constexpr int m = decltype(mc)::value;
+    all2[m] = NF == 1 ? sy2[0] : lane_of<LP, m % LP>(sy2[m / LP]);
+    all1[m] = NF == 1 ? sy[0] : lane_of<LP, m % LP>(sy[m / LP]);
+  });
+  return model_score<CF, VC, NF, FORM>(all2, all1, n_filters, dof, sum_w, dV, NU ? &nu : nullptr, mr);
 }
 
 }  // namespace ast
