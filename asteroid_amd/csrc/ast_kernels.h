@@ -205,10 +205,12 @@ struct Machine {
     reopt = __builtin_amdgcn_readfirstlane(reopt);
   }
 
-  // Makes the row addresses unknown to the compiler at this point.  Else it
-  // computes those of every row of every array once, ahead of the loop they
-  // are used in, and keeps the 200 of them in scratch memory.
+  // Makes the row addresses and the model space unknown to the compiler at
+  // this point.  Else it computes the addresses of every row of every array,
+  // and loads every limit, once, ahead of the loop they are used in, and keeps
+  // the 200 of them in scratch memory.
   __device__ void renew() {
+    pin_sgpr(sp);
     pin_sgpr(bX);
     pin_sgpr(bF);
     pin_sgpr(bX0);
@@ -359,55 +361,68 @@ struct Machine {
   }
 
   // The vertices in order of chi^2 (cuda.c:1570-1600), and the worst one: the
-  // reference takes the lowest value left, the last vertex of equal ones.
+  // reference takes the lowest value left, the last vertex of equal ones, so
+  // a vertex's place is the number of those before it.
   __device__ int sort_vertices() const {
     CF f[N + 1];
 #pragma unroll
     for (int v = 0; v <= N; ++v) f[v] = F(v);
     bool plain = true;  // every value can be taken (none is NaN or above 1e30)
 #pragma unroll
-    for (int v = 0; v <= N; ++v) plain = plain && f[v] <= (CF)1e30;
+    for (int v = 0; v <= N; ++v) plain = plain & (f[v] <= (CF)1e30);
+    int w = 0;
     if (plain) {
-      // A vertex's place is the number of those before it: one comparison
-      // per pair.
-      int place[N + 1];
+      if constexpr (N <= 16) {  // one comparison per pair
+        int place[N + 1];
 #pragma unroll
-      for (int v = 0; v <= N; ++v) place[v] = v;
+        for (int v = 0; v <= N; ++v) place[v] = v;
 #pragma unroll
-      for (int v = 1; v <= N; ++v)
+        for (int v = 1; v <= N; ++v)
 #pragma unroll
-        for (int u = 0; u < v; ++u) {
-          const int after = f[v] <= f[u] ? 1 : 0;  // v comes before u
-          place[u] += after;
-          place[v] -= after;
+          for (int u = 0; u < v; ++u) {
+            const int before = f[v] <= f[u] ? 1 : 0;  // v comes before u
+            place[u] += before;
+            place[v] -= before;
+          }
+#pragma unroll
+        for (int v = 0; v <= N; ++v) {
+          IND(place[v]) = (uint8_t)v;
+          w = place[v] == N ? v : w;
         }
-      int w = 0;
+      } else {
+#pragma unroll 1
+        for (int v = 0; v <= N; ++v) {
+          const CF fv = F(v);
+          int place = 0;
 #pragma unroll
-      for (int v = 0; v <= N; ++v) {
-        IND(place[v]) = (uint8_t)v;
-        if (place[v] == N) w = v;
+          for (int u = 0; u <= N; ++u) place += (f[u] < fv ? 1 : 0) + ((u > v) & (f[u] == fv) ? 1 : 0);
+          IND(place) = (uint8_t)v;
+          w = place == N ? v : w;
+        }
       }
-      return w;
-    }
-    uint64_t taken = 0;
+    } else {
+      uint64_t taken = 0;
+      int jmin = 0;
 #pragma unroll 1
-    for (int v = 0; v <= N; ++v) {
-      CF fmin = 1e30;
-      int jmin = -1;
+      for (int v = 0; v <= N && jmin >= 0; ++v) {
+        CF fmin = 1e30;
+        jmin = -1;
 #pragma unroll 1
-      for (int u = 0; u <= N; ++u) {
-        const CF fu = F(u);
-        if (!((taken >> u) & 1) && fu <= fmin) { fmin = fu; jmin = u; }
+        for (int u = 0; u <= N; ++u) {
+          const CF fu = F(u);
+          if (!((taken >> u) & 1) && fu <= fmin) { fmin = fu; jmin = u; }
+        }
+        if (jmin >= 0) {
+          IND(v) = (uint8_t)jmin;
+          taken |= 1ull << jmin;
+        } else {  // NaN values left (cuda.c:1592-1598)
+          IND(0) = 0;
+          F(0) = 1e30;
+        }
       }
-      if (jmin < 0) {  // NaN values left (cuda.c:1592-1598)
-        IND(0) = 0;
-        F(0) = 1e30;
-        break;
-      }
-      IND(v) = (uint8_t)jmin;
-      taken |= 1ull << jmin;
+      w = IND(N);
     }
-    return IND(N);
+    return w;
   }
 
   // K elements of the simplex, from row `first` on every `stride` rows.
@@ -491,10 +506,12 @@ struct Machine {
   // 370 us with the chip full, of 580 and 2900 us.)
   __device__ void advance(LaneRegs<CF>& R, CF val, bool has_result) {
     const CF GAMMA = 2.0, RHO = 0.5, SIGMA = 0.5;  // asteroid.h:240-242
-    if (!has_result && R.phase != PH_START) return;
+    bool more = has_result || R.phase == PH_START;
     CF xv[N];
-    for (;;) {
+    while (more) {
       renew();
+      more = false;
+      bool over = false;
       if (R.phase == PH_START) {
         start(R, xv);
         R.l = 0;
@@ -574,25 +591,25 @@ struct Machine {
         }
       }
       if (R.phase == PH_BEGIN) {
-        if (R.failed || !begin_step(R, xv)) {
-          finish(R);
-          return;
+        over = R.failed || !begin_step(R, xv);
+        if (over) finish(R);
+        else R.phase = PH_REFLECT;
+      }
+      if (!over) {
+        if (propose(xv)) {
+          if (R.phase == PH_SHRINK_NEXT) R.phase = PH_SHRINK;
+        } else {  // outside the hard limits
+          more = true;
+          if (R.phase == PH_INIT) {
+            R.failed = 1;
+            R.phase = PH_BEGIN;
+          } else if (R.phase == PH_SHRINK_NEXT) {
+            R.bad = 1;
+            R.j++;
+          } else {
+            val = 1e30;
+          }
         }
-        R.phase = PH_REFLECT;
-      }
-      if (propose(xv)) {
-        if (R.phase == PH_SHRINK_NEXT) R.phase = PH_SHRINK;
-        return;
-      }
-      // outside the hard limits
-      if (R.phase == PH_INIT) {
-        R.failed = 1;
-        R.phase = PH_BEGIN;
-      } else if (R.phase == PH_SHRINK_NEXT) {
-        R.bad = 1;
-        R.j++;
-      } else {
-        val = 1e30;
       }
     }
   }

@@ -89,3 +89,58 @@ def test_refilled_fits_on_few_lanes():
     want = pb.run(7, 64, seed=4, form=oracle.CANON, n_threads=8, **run)
     for g, k in zip(got, ("f", "params", "dV", "lane_f", "lane_nev", "lane_steps")):
         _same(g, want[k])
+
+
+BUILDS = {
+    "ls": lambda p: variants.make_variant(False, precision=p),
+    "bc": variants.bc_free,
+    "bc_torque": lambda p: variants.make_variant(True, True, precision=p),
+    "bw": lambda p: variants.make_variant(False, False, True, precision=p),
+    "bw_torque": variants.bw_ball_torque,
+    "trend": variants.ls_torque_trend,
+    "torque2": variants.ls_torque2,
+    "bc_rotate": variants.bc_rotate,
+    "bc_rotate_torque": lambda p: variants.bc_rotate(p, torque=True),
+    "rect": variants.rect,
+    "rect_torque": lambda p: variants.rect(p, torque=True),
+    "nudge": variants.ls_torque_nudge,
+    "nudge_bc": lambda p: variants.ls_torque_nudge(p, bc=True),
+    **{f"seg{n}{'_onele' if le else ''}{'_torque' if tq else ''}{'_bc' if bc else ''}":
+       (lambda p, n=n, le=le, tq=tq, bc=bc: variants.ls_segments(p, n_seg=n, one_le=le, torque=tq, bc=bc))
+       for n in (3, 4) for le in (True, False) for tq in (False, True) for bc in (False, True)},
+}
+
+
+@pytest.mark.parametrize("groups", [20, 65])  # 5120 fits: 4 lanes per model; 16640: one
+@pytest.mark.parametrize("name", list(BUILDS))
+def test_every_build_on_four_lanes_and_one(name, groups):
+    v = BUILDS[name](abi.PREC_FP64)
+    base = variants.make_variant(bool(v.torque), bool(v.bc), precision=abi.PREC_FP64) if v.n_seg > 1 else v
+    curve, truth = synth.make_curve(7, base, 56, 1.5, n_filters=2)
+    space = variants.default_model_space(v)
+    keep = {}
+    with api.Context(v) as ctx:
+        ctx.set_model_space(space)
+        if v.n_seg > 1:
+            keep["t_start"] = curve.mjd[0] - 0.01 + 1.5 * np.arange(v.n_seg) / v.n_seg
+            ctx.set_segments(keep["t_start"])
+        ctx.upload_curve(curve)
+        if v.nudge:
+            keep["minima"] = (curve.mjd[[9, 30]].astype(np.float32), curve.V[[9, 30]])
+            ctx.set_minima(*keep["minima"])
+        pb = oracle.Problem(space, curve, **keep)
+        run = dict(nstages=1, n_steps=4, eval_budget=space.n_params + 6)
+        ctx.rng_seed(8)
+        ctx.run(groups, 256, **run)
+        got = ctx.fetch() + ctx.fetch_lanes()
+        p = _models(pb, 200)
+        chi2 = ctx.chi2_batch(np.resize(p, (groups * 256, p.shape[1])))
+    want = pb.run(groups, 256, seed=8, form=oracle.CANON, n_threads=8, **run)
+    for g, k in zip(got, ("f", "params", "dV", "lane_f", "lane_nev", "lane_steps")):
+        _same(g, want[k])
+    want = pb.chi2(p)
+    n = len(want[0])
+    for a in (0, (groups * 256 // n - 1) * n):
+        _same(chi2[0][a:a + n], want[0])
+        if not v.nudge:  # delta_V of a failed NUDGE model is the caller's
+            _same(chi2[1][a:a + n], want[1])
