@@ -595,15 +595,19 @@ AST_AI ScaledDirs scaled_dirs(const double* a, const double* b, const double* c,
 }
 
 // Lommel-Seeliger magnitude from the scaled directions (cuda.c:672-689), FP64
-// canonical form.
+// canonical form.  Its square roots need no special cases (sqrt_pos): with a
+// zero or infinite sS2 or sE2 the quotient ca is NaN by its divisor, with a
+// zero sine sa the logarithm's argument is one over zero, and with a zero scn
+// its inverse is, each NaN in div_rn; so the magnitude is NaN with a root of 0
+// or infinity as it is with a root of NaN.
 AST_AI double ls_tail_f64(const ScaledDirs& u, double bcp) {
   const double sS2 = dot3(u.uSb, u.uSc, u.uSa, u.uSb, u.uSc, u.uSa);
   const double sE2 = dot3(u.uEb, u.uEc, u.uEa, u.uEb, u.uEc, u.uEa);
-  const double sS = astm::sqrt_rn(sS2);
-  const double sE = astm::sqrt_rn(sE2);
+  const double sS = astm::sqrt_pos(sS2);
+  const double sE = astm::sqrt_pos(sE2);
   const double ca = astm::div_rn(dot3(u.uSb, u.uSc, u.uSa, u.uEb, u.uEc, u.uEa), sS * sE);
-  const double sa = astm::sqrt_rn(__builtin_fma(-ca, ca, 1.0));
-  const double scn = astm::sqrt_rn(__builtin_fma((2.0 * sS) * sE, ca, sS2 + sE2));
+  const double sa = astm::sqrt_pos(__builtin_fma(-ca, ca, 1.0));
+  const double scn = astm::sqrt_pos(__builtin_fma((2.0 * sS) * sE, ca, sS2 + sE2));
   const double isc = astm::div_rn(1.0, scn);
   const double cl = __builtin_fma(sE, ca, sS) * isc;
   const double sl = (sE * sa) * isc;
