@@ -446,40 +446,34 @@ struct Machine {
     constexpr int UN = N <= 16 ? N : 1;  // whole rows in registers for the smaller simplexes
     R.l++;
     const int w = sort_vertices();
-    // Column by column for the centroid, then row by row for the size, each
-    // fetched while the one before it is summed.
-    CF x0[N];
-    CF cur[N + 1], nxt[N + 1];
+    // One pass over the simplex, column by column, each fetched while the one
+    // before it is worked on: the centroid's coordinate, then every vertex's
+    // share of the size (each vertex's sum takes the coordinates in their
+    // order, as a pass row by row would).
+    CF x0[N], dist2[N + 1], cur[N + 1], nxt[N + 1];
+#pragma unroll
+    for (int v = 0; v < N + 1; ++v) dist2[v] = 0.0;
     fetch<N + 1>(cur, 0, N);
 #pragma unroll UN
     for (int i = 0; i < N; ++i) {
       if (i + 1 < N) fetch<N + 1>(nxt, i + 1, N);
-      else fetch<N>(nxt, 0, 1);
       __builtin_amdgcn_sched_barrier(0);
       CF sum = 0.0;
 #pragma unroll
       for (int v = 0; v < N + 1; ++v) sum = sum + cur[v];
       x0[i] = sum / (N + 1);
 #pragma unroll
+      for (int v = 0; v < N + 1; ++v) {
+        CF dx = cur[v] - x0[i];
+        dist2[v] = dist2[v] + dx * dx;
+      }
+#pragma unroll
       for (int v = 0; v < N + 1; ++v) cur[v] = nxt[v];
       __builtin_amdgcn_sched_barrier(0);
     }
     CF size2 = 0.0;
-#pragma unroll UN
-    for (int v = 0; v < N + 1; ++v) {
-      if (v < N) fetch<N>(nxt, (v + 1) * N, 1);
-      __builtin_amdgcn_sched_barrier(0);
-      CF sum = 0.0;
 #pragma unroll
-      for (int i = 0; i < N; ++i) {
-        CF dx = cur[i] - x0[i];
-        sum = sum + dx * dx;
-      }
-      size2 = size2 + sum;
-#pragma unroll
-      for (int i = 0; i < N; ++i) cur[i] = nxt[i];
-      __builtin_amdgcn_sched_barrier(0);
-    }
+    for (int v = 0; v < N + 1; ++v) size2 = size2 + dist2[v];
     size2 = size2 / N;
     if (size2 < C.size2_min || R.l > C.n_steps || (C.eval_budget > 0 && R.nev >= C.eval_budget)) return false;
     CF xw[N];
