@@ -124,6 +124,95 @@ void dev_free(T*& p) {
   p = nullptr;
 }
 
+// -------------------------------------------------------- memory kept
+// A context's device and pinned host memory between calls.  An allocation and
+// a release cost a call about 15 us each (a release waits for the device as
+// well), three to fourteen of them a chi^2 batch or a job.
+//  * blocks: device blocks given back by finished calls and jobs, taken again
+//    by later ones of up to their size; at most KEEP_BYTES, the rest is
+//    released.  A call gives its blocks back when nothing on the device uses
+//    them any more.
+//  * pin: pinned host memory that kernels read and write in place, for inputs
+//    and results so small that a copy's latency is most of its time.
+// Calls on a context come from one thread at a time (the scheduler's while it
+// serves), so there is no lock.
+struct Memory {
+  static constexpr size_t KEEP_BYTES = (size_t)256 << 20, PIN_BYTES = (size_t)4 << 20;
+  std::vector<std::pair<size_t, void*>> blocks;
+  size_t kept = 0;
+  char* pin = nullptr;
+
+  int take(size_t bytes, void** p, size_t* cap) {
+    bytes = (bytes + 4095) & ~(size_t)4095;
+    int best = -1;
+    for (int k = 0; k < (int)blocks.size(); ++k)  // the smallest that holds it, of at most twice its size
+      if (blocks[k].first >= bytes && blocks[k].first <= 2 * bytes &&
+          (best < 0 || blocks[k].first < blocks[best].first))
+        best = k;
+    if (best >= 0) {
+      *cap = blocks[best].first;
+      *p = blocks[best].second;
+      kept -= *cap;
+      blocks.erase(blocks.begin() + best);
+      return 0;
+    }
+    *p = nullptr;
+    *cap = bytes;
+    if (hipMalloc(p, bytes) == hipSuccess) return 0;
+    (void)hipGetLastError();
+    release();  // what is kept may be what is missing
+    HIPCHK(hipMalloc(p, bytes));
+    return 0;
+  }
+  void give(void* p, size_t cap) {
+    if (!p) return;
+    if (kept + cap > KEEP_BYTES || blocks.size() >= 64) {
+      (void)hipFree(p);
+      return;
+    }
+    blocks.push_back({cap, p});
+    kept += cap;
+  }
+  void release() {
+    for (auto& b : blocks) (void)hipFree(b.second);
+    blocks.clear();
+    kept = 0;
+  }
+  // Pinned memory for `bytes`, or null (too many, or none to be had): the
+  // caller copies instead.
+  char* pinned(size_t bytes) {
+    if (bytes > PIN_BYTES) return nullptr;
+    if (!pin && hipHostMalloc((void**)&pin, PIN_BYTES, hipHostMallocDefault) != hipSuccess) {
+      (void)hipGetLastError();
+      pin = nullptr;
+    }
+    return pin;
+  }
+  void close() {
+    release();
+    if (pin) (void)hipHostFree(pin);
+    pin = nullptr;
+  }
+};
+
+// One device block of a call, given back at its end; carve() hands out its
+// parts, in the order and sizes of the reserve() calls before it.
+struct Scratch {
+  Memory& mem;
+  void* base = nullptr;
+  size_t cap = 0, need = 0, at = 0;
+  explicit Scratch(Memory& m) : mem(m) {}
+  ~Scratch() { mem.give(base, cap); }
+  static size_t padded(size_t bytes) { return (bytes + 255) & ~(size_t)255; }
+  template <class T> void reserve(size_t n) { need += padded(n * sizeof(T)); }
+  int take() { return mem.take(need ? need : 256, &base, &cap); }
+  template <class T> T* carve(size_t n) {
+    T* p = (T*)((char*)base + at);
+    at += padded(n * sizeof(T));
+    return p;
+  }
+};
+
 // ------------------------------------------------------------ validation
 // The variant codes built (one kernel family each), indexed by variant_index.
 constexpr int VARIANT_CODES[] = {0, VF_TQ, VF_BC, VF_TQ | VF_BC, VF_BW, VF_TQ | VF_BW,
@@ -397,12 +486,11 @@ int make_curve(const ast_variant& v, const ast_obs* obs, int n_data, int n_filte
 // from the 3-point ephemeris (read_data.c:345, the INTERP quadratic, then
 // normalised).  RK4 intervals between grid points as between observations
 // (cuda.c:321-323).  V, w and the filter are unused on a grid.
-int make_grid(const ast_variant& v, const CurveH& C, const ast_ephem3& eph, int n_plot, std::vector<PointRec>* out,
-              std::vector<double>* t_out, const double* seg_t = nullptr, int* g0 = nullptr) {
+// g takes n_plot + 1 records, t n_plot times.
+int make_grid(const ast_variant& v, const CurveH& C, const ast_ephem3& eph, int n_plot, PointRec* g, double* t,
+              const double* seg_t = nullptr, int* g0 = nullptr) {
   if (n_plot < 2 || C.n_data < 1) return AST_E_ARG;
-  std::vector<PointRec> g((size_t)n_plot + 1);
   g[n_plot] = C.pts[C.n_data];  // the minima record
-  std::vector<double> t((size_t)n_plot);
   const double h = (C.t_last - C.t_first) / (n_plot - 1);
   for (int i = 0; i < n_plot; ++i) {
     PointRec& p = g[i];
@@ -430,7 +518,7 @@ int make_grid(const ast_variant& v, const CurveH& C, const ast_ephem3& eph, int 
   if (v.n_seg > 1) {  // SEGMENT: each segment's first grid point restarts the rotation
     int start[AST_MAX_SEGMENTS];
     if (!seg_t || !g0) return AST_E_STATE;
-    if (segment_starts(v.n_seg, n_plot, t.data(), seg_t, start) < v.n_seg) return AST_E_DATA;
+    if (segment_starts(v.n_seg, n_plot, t, seg_t, start) < v.n_seg) return AST_E_DATA;
     for (int s = 0; s < v.n_seg; ++s)
       if (start[s] > 0) {
         PointRec& p = g[start[s]];
@@ -439,8 +527,6 @@ int make_grid(const ast_variant& v, const CurveH& C, const ast_ephem3& eph, int 
       }
     *g0 = start[0];  // grid points before it are not computed (their magnitudes are NaN)
   }
-  *out = std::move(g);
-  if (t_out) *t_out = std::move(t);
   return AST_OK;
 }
 
@@ -624,7 +710,9 @@ struct DevJob {
   int n_workers = 0;
   bool refill = false;
   bool reduced = false;        // refill: the groups' results have been formed
-  // device memory (owned unless borrowed)
+  // device memory: parts of one block (rng and the bests are the context's if borrowed)
+  void* block = nullptr;
+  size_t block_cap = 0;
   PointRec* pts = nullptr;
   double* sum_w = nullptr;
   void* sp = nullptr;          // Space<CF>
@@ -652,13 +740,10 @@ struct DevJob {
   double run_ms = 0;
 };
 
-void job_free(DevJob& j) {
-  dev_free(j.pts); dev_free(j.sum_w); dev_free(j.sp); dev_free(j.params0);
-  dev_free(j.fit_f); dev_free(j.fit_nev); dev_free(j.fit_steps); dev_free(j.fit_params); dev_free(j.fit_dV);
-  dev_free(j.queue);
+void job_free(DevJob& j, Memory& mem) {
+  mem.give(j.block, j.block_cap);
+  j.block = nullptr;
   j.done = nullptr;  // the pool's
-  dev_free(j.descs);
-  if (!j.borrowed) { dev_free(j.rng); dev_free(j.best_f); dev_free(j.best_params); dev_free(j.best_dV); }
 }
 
 int ticks_for(double cost, double work) {
@@ -686,80 +771,11 @@ size_t job_bytes(int n_groups, int group_size, int n_workers, int n_params, int 
          (size_t)n_groups * 256 + sizeof(PointRec) * n_records;
 }
 
-// Device memory of one job (its own streams and bests unless borrowed).  The
-// clears run on `s`, the stream the job's kernels run on, so they are ordered
-// before its first launch.
-int job_upload(DevJob& j, const Pool& pool, const CurveH& C, const double* params0, hipStream_t s) {
-  if (j.slots.empty() || j.slots[0] < 0 || j.slots[0] >= pool.n_slots) return AST_E_STATE;
-  if (j.n_workers <= 0) j.n_workers = j.rp.n_groups;
-  if ((int)j.slots.size() != j.n_workers || j.n_workers > j.rp.n_groups) return AST_E_STATE;
-  j.refill = j.n_workers < j.rp.n_groups;
-  if (j.refill && j.rp.nstages != 1) return AST_E_ARG;  // a stage reseed needs the whole group
-  const SpaceH& S = j.space;
-  j.cf = S.v.precision == AST_PREC_FP64 ? 8 : 4;
-  j.n_data = C.n_data;
-  j.n_all = C.n_all;
-  j.n_filters = C.n_filters;
-  const int N = S.n_params, G = j.rp.n_groups;
-  const size_t fits = (size_t)G * j.rp.group_size;
-  RETIF(dev_alloc(&j.pts, C.pts.size()));
-  RETIF(dev_alloc(&j.sum_w, (size_t)AST_MAX_FILTERS));
-  RETIF(dev_alloc((char**)&j.sp, sizeof(Space<double>)));
-  RETIF(dev_alloc(&j.params0, (size_t)AST_MAX_PARAMS));
-  HIPCHK(hipMemcpy(j.pts, C.pts.data(), sizeof(PointRec) * C.pts.size(), hipMemcpyHostToDevice));
-  HIPCHK(hipMemcpy(j.sum_w, C.sum_w, sizeof(double) * AST_MAX_FILTERS, hipMemcpyHostToDevice));
-  if (j.cf == 8) {
-    Space<double> sp = space_table<double>(S);
-    HIPCHK(hipMemcpy(j.sp, &sp, sizeof sp, hipMemcpyHostToDevice));
-  } else {
-    Space<float> sp = space_table<float>(S);
-    HIPCHK(hipMemcpy(j.sp, &sp, sizeof sp, hipMemcpyHostToDevice));
-  }
-  double p0[AST_MAX_PARAMS] = {0};
-  if (params0)
-    for (int i = 0; i < N; ++i) p0[i] = params0[i];
-  HIPCHK(hipMemcpy(j.params0, p0, sizeof p0, hipMemcpyHostToDevice));
-  j.done = pool.job_done + j.slots[0];
-  HIPCHK(hipMemsetAsync(j.done, 0, sizeof(int32_t), s));
-  if (!j.borrowed) {
-    RETIF(dev_alloc(&j.rng, fits));
-    RETIF(dev_alloc((char**)&j.best_f, (size_t)j.cf * G));
-    RETIF(dev_alloc(&j.best_params, (size_t)G * AST_MAX_PARAMS));
-    RETIF(dev_alloc(&j.best_dV, (size_t)G * AST_MAX_FILTERS));
-    std::vector<char> hf((size_t)j.cf * G);
-    for (int g = 0; g < G; ++g) {
-      if (j.cf == 8) { double v = 1e30; std::memcpy(&hf[(size_t)g * 8], &v, 8); }
-      else { float v = 1e30f; std::memcpy(&hf[(size_t)g * 4], &v, 4); }
-    }
-    HIPCHK(hipMemcpy(j.best_f, hf.data(), hf.size(), hipMemcpyHostToDevice));
-    HIPCHK(hipMemsetAsync(j.rng, 0, fits * sizeof(uint32_t), s));
-    HIPCHK(hipMemsetAsync(j.best_params, 0, sizeof(double) * G * AST_MAX_PARAMS, s));
-    HIPCHK(hipMemsetAsync(j.best_dV, 0, sizeof(double) * G * AST_MAX_FILTERS, s));
-  }
-  RETIF(dev_alloc((char**)&j.fit_f, (size_t)j.cf * fits));
-  RETIF(dev_alloc(&j.fit_nev, fits));
-  RETIF(dev_alloc(&j.fit_steps, fits));
-  HIPCHK(hipMemsetAsync(j.fit_nev, 0, fits * sizeof(int32_t), s));
-  HIPCHK(hipMemsetAsync(j.fit_steps, 0, fits * sizeof(int32_t), s));
-  if (j.refill) {
-    RETIF(dev_alloc(&j.fit_params, fits * (size_t)N));
-    RETIF(dev_alloc(&j.fit_dV, fits * (size_t)C.n_filters));
-    RETIF(dev_alloc(&j.queue, (size_t)2));
-    const int32_t q[2] = {(int32_t)((size_t)j.n_workers * j.rp.group_size), 0};
-    HIPCHK(hipMemcpy(j.queue, q, sizeof q, hipMemcpyHostToDevice));
-  }
-  j.reduced = false;
-  j.bytes = job_bytes(j.rp.n_groups, j.rp.group_size, j.n_workers, N, C.n_filters, C.pts.size());
-  return 0;
-}
-
 template <class CF>
-int job_descs_typed(DevJob& j, int ticks) {
-  const int G = j.n_workers;
-  std::vector<GroupDesc<CF>> d(G);
+void job_descs(DevJob& j, GroupDesc<CF>* d) {
   double sm = j.rp.size_min > 0 ? j.rp.size_min : (j.cf == 8 ? 1e-10 : 1e-5);  // asteroid.h:233-237
   CF smc = (CF)sm;
-  for (int g = 0; g < G; ++g) {
+  for (int g = 0; g < j.n_workers; ++g) {
     GroupDesc<CF>& D = d[g];
     std::memset(&D, 0, sizeof D);
     D.pts = j.pts;
@@ -782,7 +798,7 @@ int job_descs_typed(DevJob& j, int ticks) {
     D.reopt = j.space.x2.reopt;
     D.slot = j.slots[g];
     D.group_in_job = g;
-    D.ticks = ticks;
+    D.ticks = j.ticks;
     D.fit_f = (CF*)j.fit_f;
     D.fit_nev = j.fit_nev;
     D.fit_steps = j.fit_steps;
@@ -792,15 +808,84 @@ int job_descs_typed(DevJob& j, int ticks) {
     D.fit_params = j.fit_params;
     D.fit_dV = j.fit_dV;
   }
-  if (!j.descs) RETIF(dev_alloc((char**)&j.descs, sizeof(GroupDesc<CF>) * G));
-  HIPCHK(hipMemcpy(j.descs, d.data(), sizeof(GroupDesc<CF>) * G, hipMemcpyHostToDevice));
-  j.desc_host.resize(sizeof(GroupDesc<CF>) * G);
-  std::memcpy(j.desc_host.data(), d.data(), j.desc_host.size());
+}
+
+// Device memory of one job, as one block: first what the host fills in (one
+// copy), then what starts at zero (one clear on `s`, the stream the job's init
+// kernel runs on), then what the kernels write first.  j.ticks is set before.
+template <class CF>
+int job_upload_typed(DevJob& j, const Pool& pool, const CurveH& C, const double* params0, hipStream_t s,
+                     Memory& mem) {
+  if (j.slots.empty() || j.slots[0] < 0 || j.slots[0] >= pool.n_slots) return AST_E_STATE;
+  if (j.n_workers <= 0) j.n_workers = j.rp.n_groups;
+  if ((int)j.slots.size() != j.n_workers || j.n_workers > j.rp.n_groups) return AST_E_STATE;
+  j.refill = j.n_workers < j.rp.n_groups;
+  if (j.refill && j.rp.nstages != 1) return AST_E_ARG;  // a stage reseed needs the whole group
+  const SpaceH& S = j.space;
+  j.n_data = C.n_data;
+  j.n_all = C.n_all;
+  j.n_filters = C.n_filters;
+  const int N = S.n_params, G = j.rp.n_groups;
+  const size_t fits = (size_t)G * j.rp.group_size;
+  size_t at = 0;
+  auto part = [&](size_t bytes) {
+    const size_t p = at;
+    at += Scratch::padded(bytes);
+    return p;
+  };
+  const size_t o_pts = part(sizeof(PointRec) * C.pts.size()), o_sum_w = part(sizeof(double) * AST_MAX_FILTERS),
+               o_sp = part(sizeof(Space<CF>)), o_params0 = part(sizeof(double) * AST_MAX_PARAMS),
+               o_queue = part(2 * sizeof(int32_t)), o_descs = part(sizeof(GroupDesc<CF>) * j.n_workers),
+               o_best_f = part(j.borrowed ? 0 : sizeof(CF) * G), filled = at;
+  const size_t o_rng = part(j.borrowed ? 0 : sizeof(uint32_t) * fits),
+               o_best_params = part(j.borrowed ? 0 : sizeof(double) * G * AST_MAX_PARAMS),
+               o_best_dV = part(j.borrowed ? 0 : sizeof(double) * G * AST_MAX_FILTERS),
+               o_nev = part(sizeof(int32_t) * fits), o_steps = part(sizeof(int32_t) * fits), cleared = at;
+  const size_t o_fit_f = part(sizeof(CF) * fits), o_fit_params = part(j.refill ? sizeof(double) * fits * N : 0),
+               o_fit_dV = part(j.refill ? sizeof(double) * fits * C.n_filters : 0);
+  RETIF(mem.take(at, &j.block, &j.block_cap));
+  char* const dev = (char*)j.block;
+  j.pts = (PointRec*)(dev + o_pts);
+  j.sum_w = (double*)(dev + o_sum_w);
+  j.sp = dev + o_sp;
+  j.params0 = (double*)(dev + o_params0);
+  j.queue = j.refill ? (int32_t*)(dev + o_queue) : nullptr;
+  j.descs = dev + o_descs;
+  j.fit_nev = (int32_t*)(dev + o_nev);
+  j.fit_steps = (int32_t*)(dev + o_steps);
+  j.fit_f = dev + o_fit_f;
+  j.fit_params = j.refill ? (double*)(dev + o_fit_params) : nullptr;
+  j.fit_dV = j.refill ? (double*)(dev + o_fit_dV) : nullptr;
+  if (!j.borrowed) {
+    j.best_f = dev + o_best_f;
+    j.rng = (uint32_t*)(dev + o_rng);
+    j.best_params = (double*)(dev + o_best_params);
+    j.best_dV = (double*)(dev + o_best_dV);
+  }
+  j.done = pool.job_done + j.slots[0];
+  std::vector<char> h(filled, 0);
+  std::memcpy(&h[o_pts], C.pts.data(), sizeof(PointRec) * C.pts.size());
+  std::memcpy(&h[o_sum_w], C.sum_w, sizeof(double) * AST_MAX_FILTERS);
+  const Space<CF> sp = space_table<CF>(S);
+  std::memcpy(&h[o_sp], &sp, sizeof sp);
+  if (params0) std::memcpy(&h[o_params0], params0, sizeof(double) * N);
+  const int32_t q[2] = {(int32_t)((size_t)j.n_workers * j.rp.group_size), 0};
+  std::memcpy(&h[o_queue], q, sizeof q);
+  job_descs<CF>(j, (GroupDesc<CF>*)&h[o_descs]);
+  if (!j.borrowed) std::fill_n((CF*)&h[o_best_f], G, (CF)1e30);
+  HIPCHK(hipMemcpy(dev, h.data(), filled, hipMemcpyHostToDevice));
+  HIPCHK(hipMemsetAsync(j.done, 0, sizeof(int32_t), s));
+  HIPCHK(hipMemsetAsync(dev + filled, 0, cleared - filled, s));
+  j.desc_host.assign((unsigned char*)&h[o_descs], (unsigned char*)&h[o_descs] + sizeof(GroupDesc<CF>) * j.n_workers);
+  j.reduced = false;
+  j.bytes = job_bytes(j.rp.n_groups, j.rp.group_size, j.n_workers, N, C.n_filters, C.pts.size());
   return 0;
 }
 
-int job_descs(DevJob& j, int ticks) {
-  return j.cf == 8 ? job_descs_typed<double>(j, ticks) : job_descs_typed<float>(j, ticks);
+int job_upload(DevJob& j, const Pool& pool, const CurveH& C, const double* params0, hipStream_t s, Memory& mem) {
+  j.cf = j.space.v.precision == AST_PREC_FP64 ? 8 : 4;
+  return j.cf == 8 ? job_upload_typed<double>(j, pool, C, params0, s, mem)
+                   : job_upload_typed<float>(j, pool, C, params0, s, mem);
 }
 
 // The shapes the kernels assume: one workgroup of pool.G threads per group,
@@ -942,86 +1027,90 @@ constexpr double PGRAM_DT2 = 80.0 / 24.0;// dt2, days
 constexpr double PGRAM_S0 = 3;           // s0
 constexpr int PGRAM_MAX_MINIMA = 10000;  // NMIN_MAX
 
+// Frequency of bin i (misc.c:128).
+__host__ __device__ inline double pgram_fr(int i) {
+  const double fr0 = 1 / PGRAM_DT0, fr2 = 1 / PGRAM_DT2;
+  return fr2 + (double)i / (double)(PGRAM_BINS - 1) * (fr0 - fr2);
+}
+
 // Histogram counts: for each frequency bin i (period p = 1/fr[i]), the
 // number of pairs of minima a < b whose interval is within a fraction sgm of
 // a whole number of periods (misc.c:128-146).  Each thread owns one bin;
 // blockIdx.y takes every n_chunks-th first minimum a, and the per-chunk
-// counts go to partial[chunk][bin] (summed on the host, exactly).  The
+// counts go to partial[chunk][bin], summed by pgram_sum_kernel.  The
 // interval and the ratio are computed as the reference does (a subtraction
 // and an IEEE division), so the counts equal the reference's whatever the
 // order of the pairs.
-__global__ __launch_bounds__(256) void minima_hist_kernel(const double* __restrict__ tm, int n,
-                                                         const double* __restrict__ period, int n_bins,
-                                                         double sgm, int n_chunks, int32_t* __restrict__ partial) {
+__global__ __launch_bounds__(256) void minima_hist_kernel(const double* __restrict__ tm, int n, int n_chunks,
+                                                         int32_t* __restrict__ partial) {
   const int bin = blockIdx.x * blockDim.x + threadIdx.x;
   const int chunk = blockIdx.y;
-  if (bin >= n_bins) return;
-  const double p = period[bin];
+  if (bin >= PGRAM_BINS) return;
+  const double p = 1 / pgram_fr(bin);
   int32_t cnt = 0;
   for (int a = chunk; a < n - 1; a += n_chunks) {
     const double ta = tm[a];
     for (int b = a + 1; b < n; ++b) {
       const double q = (tm[b] - ta) / p;
       const double dv = fabs(q - (double)(int)(q + 0.5));
-      cnt += dv < sgm ? 1 : 0;
+      cnt += dv < PGRAM_SGM ? 1 : 0;
     }
   }
-  partial[(size_t)chunk * n_bins + bin] = cnt;
+  partial[(size_t)chunk * PGRAM_BINS + bin] = cnt;
+}
+__global__ __launch_bounds__(256) void pgram_sum_kernel(const int32_t* __restrict__ partial, int n_chunks,
+                                                       int32_t* __restrict__ counts) {
+  const int bin = blockIdx.x * blockDim.x + threadIdx.x;
+  if (bin >= PGRAM_BINS) return;
+  int32_t s = 0;
+  for (int ch = 0; ch < n_chunks; ++ch) s += partial[(size_t)ch * PGRAM_BINS + bin];
+  counts[bin] = s;
 }
 
-// Frequency of bin i (misc.c:128).
-inline double pgram_fr(int i) {
-  const double fr0 = 1 / PGRAM_DT0, fr2 = 1 / PGRAM_DT2;
-  return fr2 + (double)i / (double)(PGRAM_BINS - 1) * (fr0 - fr2);
-}
-
-int pgram_counts(hipStream_t s, const std::vector<double>& tm, std::vector<int32_t>* counts, double* ms_out) {
+// The counts of `tm`'s minima.  The host used to make the periods and sum the
+// chunks of a copy of them all: 158 us for a curve of 30 minima, 235 us for one
+// of 100, of which the kernel took 10; 73 and 75 us now.
+int pgram_counts(hipStream_t s, Memory& mem, const hipEvent_t* ev, const std::vector<double>& tm,
+                 std::vector<int32_t>* counts, double* ms_out) {
   counts->assign(PGRAM_BINS, 0);
   *ms_out = 0;
   const int n = (int)tm.size();
   if (n < 2) return AST_OK;
-  std::vector<double> period(PGRAM_BINS);
-  for (int i = 0; i < PGRAM_BINS; ++i) period[i] = 1 / pgram_fr(i);
   const int bx = (PGRAM_BINS + 255) / 256;
   const int n_chunks = std::max(1, std::min(n - 1, (2048 + bx - 1) / bx));
-  double *td = nullptr, *pd = nullptr;
-  int32_t* part = nullptr;
-  int rc = dev_alloc(&td, (size_t)n);
-  if (!rc) rc = dev_alloc(&pd, (size_t)PGRAM_BINS);
-  if (!rc) rc = dev_alloc(&part, (size_t)n_chunks * PGRAM_BINS);
-  if (rc) { dev_free(td); dev_free(pd); dev_free(part); return rc; }
-  std::vector<int32_t> host((size_t)n_chunks * PGRAM_BINS);
-  hipEvent_t e0 = nullptr, e1 = nullptr;
-  hipError_t he = hipEventCreate(&e0);
-  if (he == hipSuccess) he = hipEventCreate(&e1);
-  if (he == hipSuccess) he = hipMemcpy(td, tm.data(), sizeof(double) * n, hipMemcpyHostToDevice);
-  if (he == hipSuccess) he = hipMemcpy(pd, period.data(), sizeof(double) * PGRAM_BINS, hipMemcpyHostToDevice);
-  if (he == hipSuccess) he = hipEventRecord(e0, s);
+  Scratch sc(mem);
+  sc.reserve<double>(n);
+  sc.reserve<int32_t>((size_t)n_chunks * PGRAM_BINS);
+  sc.reserve<int32_t>(PGRAM_BINS);
+  RETIF(sc.take());
+  double* td = sc.carve<double>(n);
+  int32_t* part = sc.carve<int32_t>((size_t)n_chunks * PGRAM_BINS);
+  int32_t* sum = sc.carve<int32_t>(PGRAM_BINS);
+  char* pin = mem.pinned(sizeof(int32_t) * PGRAM_BINS);
+  hipError_t he = hipMemcpyAsync(td, tm.data(), sizeof(double) * n, hipMemcpyHostToDevice, s);
+  if (he == hipSuccess) he = hipEventRecord(ev[0], s);
   if (he == hipSuccess) {
-    hipLaunchKernelGGL(minima_hist_kernel, dim3(bx, n_chunks), dim3(256), 0, s, td, n, pd, PGRAM_BINS, PGRAM_SGM,
-                       n_chunks, part);
+    hipLaunchKernelGGL(minima_hist_kernel, dim3(bx, n_chunks), dim3(256), 0, s, td, n, n_chunks, part);
     he = hipGetLastError();
   }
-  if (he == hipSuccess) he = hipEventRecord(e1, s);
+  if (he == hipSuccess) {
+    hipLaunchKernelGGL(pgram_sum_kernel, dim3(bx), dim3(256), 0, s, part, n_chunks, pin ? (int32_t*)pin : sum);
+    he = hipGetLastError();
+  }
+  if (he == hipSuccess) he = hipEventRecord(ev[1], s);
+  if (!pin && he == hipSuccess)
+    he = hipMemcpyAsync(counts->data(), sum, sizeof(int32_t) * PGRAM_BINS, hipMemcpyDeviceToHost, s);
   if (he == hipSuccess) he = hipStreamSynchronize(s);
   float ms = 0;
-  if (he == hipSuccess) he = hipEventElapsedTime(&ms, e0, e1);
-  if (he == hipSuccess) he = hipMemcpy(host.data(), part, sizeof(int32_t) * host.size(), hipMemcpyDeviceToHost);
+  if (he == hipSuccess) he = hipEventElapsedTime(&ms, ev[0], ev[1]);
   if (he != hipSuccess) {
     (void)hipDeviceSynchronize();
     snprintf(g_hip_err, sizeof g_hip_err, "%s (periodogram)", hipGetErrorString(he));
-    rc = AST_E_HIP;
-  } else {
-    for (int ch = 0; ch < n_chunks; ++ch)
-      for (int i = 0; i < PGRAM_BINS; ++i) (*counts)[i] += host[(size_t)ch * PGRAM_BINS + i];
-    *ms_out = ms;
+    return AST_E_HIP;
   }
-  if (e0) (void)hipEventDestroy(e0);
-  if (e1) (void)hipEventDestroy(e1);
-  dev_free(td);
-  dev_free(pd);
-  dev_free(part);
-  return rc;
+  if (pin) std::memcpy(counts->data(), pin, sizeof(int32_t) * PGRAM_BINS);
+  *ms_out = ms;
+  return AST_OK;
 }
 
 // Normalisation and clusters (misc.c:148-266), on the host in the
@@ -1067,6 +1156,7 @@ void pgram_clusters(const std::vector<int32_t>& counts, int ncl, double* cl_fr, 
 
 struct ast_ctx {
   int device = 0;
+  Memory mem;                // device and pinned memory kept between calls
   hipStream_t streams[NSTREAMS] = {nullptr};
   hipEvent_t ev0[NSTREAMS] = {nullptr}, ev1[NSTREAMS] = {nullptr};
   ast_variant v{};
@@ -1524,8 +1614,8 @@ int batch_run(ast_ctx* c, const std::vector<const ast_job*>& jobs, int G, double
       const double t = std::ceil(evals[i] * work / w_max);
       ticks = t < 1 ? 1 : (t > 4096 ? 4096 : (int)t);
     }
-    rc = job_upload(j, c->pool, curves[i], p0[i].empty() ? nullptr : p0[i].data(), s);
-    if (!rc) rc = job_descs(j, ticks);
+    j.ticks = ticks;
+    rc = job_upload(j, c->pool, curves[i], p0[i].empty() ? nullptr : p0[i].data(), s, c->mem);
     if (!rc) {
       hipError_t e = job_launch(j, c->pool, 0, s);
       if (e != hipSuccess) {
@@ -1534,7 +1624,6 @@ int batch_run(ast_ctx* c, const std::vector<const ast_job*>& jobs, int G, double
       }
     }
     j.t_submit = j.t_admit = t0;
-    j.ticks = ticks;
     run.push_back(&j);
   }
   // Every tick completes one evaluation of each running simplex; a stage
@@ -1581,7 +1670,7 @@ int batch_run(ast_ctx* c, const std::vector<const ast_job*>& jobs, int G, double
       r.id = (uint64_t)i;
       r.tag = j.tag;
     }
-    job_free(j);
+    job_free(j, c->mem);
   }
   if (results) {
     c->last_evals = ev_tot;
@@ -1595,9 +1684,8 @@ int batch_run(ast_ctx* c, const std::vector<const ast_job*>& jobs, int G, double
 // under the scheduler lock when it was admitted.
 int serve_admit(ast_ctx* c, Serve& S, DevJob& j, const CurveH& curve, const std::vector<double>& p0) {
   const hipStream_t s = c->streams[0];
-  RETIF(job_upload(j, c->pool, curve, p0.empty() ? nullptr : p0.data(), s));
   j.ticks = ticks_for(j.cost, S.cfg.work_points_per_launch);
-  RETIF(job_descs(j, j.ticks));
+  RETIF(job_upload(j, c->pool, curve, p0.empty() ? nullptr : p0.data(), s, c->mem));
   HIPCHK(job_launch(j, c->pool, 0, s));
   return 0;
 }
@@ -1740,7 +1828,7 @@ void serve_loop(ast_ctx* c) {
       S.resident_bytes -= (int64_t)j.bytes;
       S.evals += ev;
       S.points += ev * j.n_data;
-      job_free(j);
+      job_free(j, c->mem);
       S.done.push_back(r);
       S.cv_done.notify_all();
     }
@@ -1756,19 +1844,20 @@ int rmsd_run(ast_ctx* c, const ast_rmsd_cfg& cfg, RmsdOut* out) {
   const size_t lanes = (size_t)ng * G;
   RETIF(ensure_streams(c, lanes, (size_t)ng));
   const Space<CF> sp_h = space_table<CF>(c->space);
-  Space<CF>* sp = nullptr;
-  RmsdRef<CF>* ref = nullptr;
-  double* p0 = nullptr;
-  float *pmin = nullptr, *pmax = nullptr;
-  int32_t* cnt = nullptr;
-  int rc = dev_alloc(&sp, 1);
-  if (!rc) rc = dev_alloc(&ref, 1);
-  if (!rc) rc = dev_alloc(&p0, (size_t)N);
-  if (!rc) rc = dev_alloc(&pmin, (size_t)ng * N);
-  if (!rc) rc = dev_alloc(&pmax, (size_t)ng * N);
-  if (!rc) rc = dev_alloc(&cnt, (size_t)ng * 2);
-  auto release = [&]() { dev_free(sp); dev_free(ref); dev_free(p0); dev_free(pmin); dev_free(pmax); dev_free(cnt); };
-  if (rc) { release(); return rc; }
+  Scratch sc(c->mem);
+  sc.reserve<Space<CF>>(1);
+  sc.reserve<RmsdRef<CF>>(1);
+  sc.reserve<double>((size_t)N);
+  sc.reserve<float>((size_t)ng * N);
+  sc.reserve<float>((size_t)ng * N);
+  sc.reserve<int32_t>((size_t)ng * 2);
+  RETIF(sc.take());
+  Space<CF>* sp = sc.carve<Space<CF>>(1);
+  RmsdRef<CF>* ref = sc.carve<RmsdRef<CF>>(1);
+  double* p0 = sc.carve<double>((size_t)N);
+  float* pmin = sc.carve<float>((size_t)ng * N);
+  float* pmax = sc.carve<float>((size_t)ng * N);
+  int32_t* cnt = sc.carve<int32_t>((size_t)ng * 2);
   RmsdArgs<CF> A{};
   A.pts = c->pts;
   A.sum_w = c->sum_w;
@@ -1814,7 +1903,6 @@ int rmsd_run(ast_ctx* c, const ast_rmsd_cfg& cfg, RmsdOut* out) {
   if (he != hipSuccess) {
     (void)hipDeviceSynchronize();
     snprintf(g_hip_err, sizeof g_hip_err, "%s (rmsd)", hipGetErrorString(he));
-    release();
     return AST_E_HIP;
   }
   out->n_tot = out->n_bad = 0;
@@ -1825,7 +1913,6 @@ int rmsd_run(ast_ctx* c, const ast_rmsd_cfg& cfg, RmsdOut* out) {
   out->f0 = rh.f0;
   out->f1 = rh.f1;
   out->ms = ms;
-  release();
   return AST_OK;
 }
 
@@ -1884,6 +1971,7 @@ int ast_ctx_create(ast_ctx** out, const ast_variant* v, int device) {
   if (e == hipSuccess) e = hipEventCreateWithFlags(&c->ev_fork, hipEventDisableTiming);
   if (e == hipSuccess) e = hipEventCreateWithFlags(&c->ev_pre, hipEventDisableTiming);
   if (e == hipSuccess) e = scratch_setup(device);
+  if (e == hipSuccess) (void)c->mem.pinned(1);  // for ast_chi2_batch_noalloc; without it the calls copy
   if (e != hipSuccess) {
     set_err(hipGetErrorString(e));
     ast_ctx_destroy(c);
@@ -1897,7 +1985,7 @@ int ast_ctx_destroy(ast_ctx* c) {
   if (!c) return AST_E_ARG;
   if (c->serve) ast_serve_stop(c);
   (void)hipSetDevice(c->device);
-  if (c->ref_job) job_free(*c->ref_job);
+  if (c->ref_job) job_free(*c->ref_job, c->mem);
   pool_free(c->pool);
   for (int k = 0; k < MAX_CLASSES; ++k) dev_free(c->batch[k].d_descs);
   dev_free(c->pts);
@@ -1906,6 +1994,7 @@ int ast_ctx_destroy(ast_ctx* c) {
   dev_free(c->best_f);
   dev_free(c->best_params);
   dev_free(c->best_dV);
+  c->mem.close();
   if (c->cg_exec) (void)hipGraphExecDestroy(c->cg_exec);
   for (int k = 0; k < NSTREAMS; ++k) {
     if (c->streams[k]) (void)hipStreamDestroy(c->streams[k]);
@@ -2042,7 +2131,7 @@ int ast_run_begin(ast_ctx* c, const ast_run_cfg* rc) {
   if (c->pool.nf < lanes || c->pool.G != G || c->pool.P < c->space.n_params)
     RETIF(pool_alloc(c->pool, lanes, G, c->space.n_params));
   // The reference path is one job that borrows the context's streams and bests.
-  if (c->ref_job) job_free(*c->ref_job);
+  if (c->ref_job) job_free(*c->ref_job, c->mem);
   c->ref_job.reset(new DevJob());
   DevJob& j = *c->ref_job;
   j.uid = c->next_uid++;
@@ -2063,10 +2152,6 @@ int ast_run_begin(ast_ctx* c, const ast_run_cfg* rc) {
   j.cls = class_of(c->v, c->curve.n_filters);
   const hipStream_t s = c->streams[0];
   for (int g = 0; g < workers; ++g) j.slots.push_back(g);
-  RETIF(job_upload(j, c->pool, c->curve, c->params0, s));
-  // The context's streams and bests were cleared by synchronous-API calls on
-  // the null stream, which the job's non-blocking stream does not wait for.
-  HIPCHK(hipDeviceSynchronize());
   int ticks;
   if (rc->ticks_per_launch > 0) {
     ticks = rc->ticks_per_launch > 4096 ? 4096 : rc->ticks_per_launch;
@@ -2074,9 +2159,14 @@ int ast_run_begin(ast_ctx* c, const ast_run_cfg* rc) {
     double tot = (double)lanes * c->curve.n_data;
     double t = 3.0e9 / (tot > 1 ? tot : 1);
     ticks = (int)(t < 16 ? 16 : (t > 4096 ? 4096 : t));
+    // with several lanes per model a stage ends between launches
+    if (rc->nstages > 1 && lanes_per_model((int64_t)lanes) > 1 && ticks > 64) ticks = 64;
   }
   j.ticks = ticks;
-  RETIF(job_descs(j, ticks));
+  RETIF(job_upload(j, c->pool, c->curve, c->params0, s, c->mem));
+  // The context's streams and bests were cleared by synchronous-API calls on
+  // the null stream, which the job's non-blocking stream does not wait for.
+  HIPCHK(hipDeviceSynchronize());
   HIPCHK(job_launch(j, c->pool, 0, s));
   c->last_ms = 0;
   c->last_launches = 0;
@@ -2214,20 +2304,7 @@ int ast_fetch_lanes(ast_ctx* c, double* f_last, int64_t* n_evals, int64_t* n_ste
   return AST_OK;
 }
 
-int ast_chi2_batch(ast_ctx* c, const double* params, int n, double* chi2, double* dV) {
-  if (!c || !params || n <= 0 || !chi2 || !dV) return AST_E_ARG;
-  if (c->serve) return AST_E_BUSY;  // its streams and events belong to the scheduler
-  if (!c->space_set || !c->curve_set || (c->v.nudge && !c->minima_set)) return AST_E_STATE;
-  if (c->curve.n_all - c->space.n_params - c->curve.n_filters <= 0) return AST_E_DATA;
-  RETIF(set_device(c));
-  double *pd = nullptr, *cd = nullptr, *dd = nullptr;
-  int rc = dev_alloc(&pd, (size_t)n * c->space.n_params);
-  if (!rc) rc = dev_alloc(&cd, (size_t)n);
-  if (!rc) rc = dev_alloc(&dd, (size_t)n * c->curve.n_filters);
-  if (rc) { dev_free(pd); dev_free(cd); dev_free(dd); return rc; }
-  int result = AST_OK;
-  hipStream_t s = c->streams[0];
-  hipError_t he = hipMemcpy(pd, params, sizeof(double) * n * c->space.n_params, hipMemcpyHostToDevice);
+static LaunchArgs chi2_args(const ast_ctx* c, const double* params, int n, double* chi2, double* dV, hipStream_t s) {
   LaunchArgs a{};
   a.op = 2;
   a.stream = s;
@@ -2236,31 +2313,84 @@ int ast_chi2_batch(ast_ctx* c, const double* params, int n, double* chi2, double
   a.n_data = c->curve.n_data;
   a.n_filters = c->curve.n_filters;
   a.dof = c->curve.n_all - c->space.n_params - c->curve.n_filters;
-  a.params = pd;
+  a.params = params;
   a.n = n;
-  a.chi2 = cd;
-  a.dV = dd;
-  if (he == hipSuccess) he = hipEventRecord(c->ev0[0], s);
+  a.chi2 = chi2;
+  a.dV = dV;
+  return a;
+}
+
+// Up to here inputs and results of a call go through pinned memory that the
+// kernel reads and writes in place: one model of 57 points takes 84 us a call
+// (the kernel 77), with three allocations and four copies it took 129.
+constexpr size_t IN_PLACE_BYTES = (size_t)256 << 10;
+// chi^2 of n models in place (pinned memory `pin`).
+static hipError_t chi2_in_place(ast_ctx* c, char* pin, const double* params, int n, double* chi2, double* dV,
+                                float* ms) {
+  const size_t np = (size_t)n * c->space.n_params, nd = (size_t)n * c->curve.n_filters;
+  const hipStream_t s = c->streams[0];
+  double* const pp = (double*)pin;
+  double *const cp = pp + np, *const dp = cp + n;
+  std::memcpy(pp, params, sizeof(double) * np);
+  LaunchArgs a = chi2_args(c, pp, n, cp, dp, s);
+  hipError_t he = hipEventRecord(c->ev0[0], s);
   if (he == hipSuccess) he = dispatch(c->v, a);
   if (he == hipSuccess) he = hipEventRecord(c->ev1[0], s);
   if (he == hipSuccess) he = hipStreamSynchronize(s);
+  if (he == hipSuccess) he = hipEventElapsedTime(ms, c->ev0[0], c->ev1[0]);
+  if (he == hipSuccess) {
+    std::memcpy(chi2, cp, sizeof(double) * n);
+    std::memcpy(dV, dp, sizeof(double) * nd);
+  }
+  return he;
+}
+
+static size_t chi2_bytes(const ast_ctx* c, int n) {
+  return sizeof(double) * (size_t)n * (c->space.n_params + 1 + c->curve.n_filters);
+}
+
+int ast_chi2_batch(ast_ctx* c, const double* params, int n, double* chi2, double* dV) {
+  if (!c || !params || n <= 0 || !chi2 || !dV) return AST_E_ARG;
+  if (c->serve) return AST_E_BUSY;  // its streams and events belong to the scheduler
+  if (!c->space_set || !c->curve_set || (c->v.nudge && !c->minima_set)) return AST_E_STATE;
+  if (c->curve.n_all - c->space.n_params - c->curve.n_filters <= 0) return AST_E_DATA;
+  RETIF(set_device(c));
+  const size_t N = c->space.n_params, NF = c->curve.n_filters;
   float ms = 0;
-  if (he == hipSuccess) he = hipEventElapsedTime(&ms, c->ev0[0], c->ev1[0]);
-  if (he == hipSuccess) he = hipMemcpy(chi2, cd, sizeof(double) * n, hipMemcpyDeviceToHost);
-  if (he == hipSuccess) he = hipMemcpy(dV, dd, sizeof(double) * n * c->curve.n_filters, hipMemcpyDeviceToHost);
+  hipError_t he = hipSuccess;
+  char* pin = chi2_bytes(c, n) <= IN_PLACE_BYTES ? c->mem.pinned(IN_PLACE_BYTES) : nullptr;
+  if (pin) {
+    he = chi2_in_place(c, pin, params, n, chi2, dV, &ms);
+    if (he != hipSuccess) (void)hipDeviceSynchronize();
+  } else {
+    Scratch sc(c->mem);
+    sc.reserve<double>((size_t)n * N);
+    sc.reserve<double>((size_t)n);
+    sc.reserve<double>((size_t)n * NF);
+    RETIF(sc.take());
+    double *pd = sc.carve<double>((size_t)n * N), *cd = sc.carve<double>((size_t)n),
+           *dd = sc.carve<double>((size_t)n * NF);
+    const hipStream_t s = c->streams[0];
+    he = hipMemcpy(pd, params, sizeof(double) * n * N, hipMemcpyHostToDevice);
+    LaunchArgs a = chi2_args(c, pd, n, cd, dd, s);
+    if (he == hipSuccess) he = hipEventRecord(c->ev0[0], s);
+    if (he == hipSuccess) he = dispatch(c->v, a);
+    if (he == hipSuccess) he = hipEventRecord(c->ev1[0], s);
+    if (he == hipSuccess) he = hipStreamSynchronize(s);
+    if (he == hipSuccess) he = hipEventElapsedTime(&ms, c->ev0[0], c->ev1[0]);
+    if (he == hipSuccess) he = hipMemcpy(chi2, cd, sizeof(double) * n, hipMemcpyDeviceToHost);
+    if (he == hipSuccess) he = hipMemcpy(dV, dd, sizeof(double) * n * NF, hipMemcpyDeviceToHost);
+    if (he != hipSuccess) (void)hipDeviceSynchronize();  // before the block is given back
+  }
   if (he != hipSuccess) {
     snprintf(g_hip_err, sizeof g_hip_err, "%s (chi2 batch)", hipGetErrorString(he));
-    result = AST_E_HIP;
-  } else {
-    c->last_ms = ms;
-    c->last_launches = 1;
-    c->last_evals = n;
-    c->last_points = (int64_t)n * c->curve.n_data;
+    return AST_E_HIP;
   }
-  dev_free(pd);
-  dev_free(cd);
-  dev_free(dd);
-  return result;
+  c->last_ms = ms;
+  c->last_launches = 1;
+  c->last_evals = n;
+  c->last_points = (int64_t)n * c->curve.n_data;
+  return AST_OK;
 }
 
 // A plain streaming copy of n 16-byte words (one load and one store per
@@ -2322,33 +2452,28 @@ int ast_chi2_batch_noalloc(ast_ctx* c, const double* params, int n, double* chi2
   double* const base = c->device >= 0 && c->device < SCRATCH_MAX_DEVICES ? g_scratch_ptr[c->device] : nullptr;
   if (!base) return AST_E_STATE;
   RETIF(set_device(c));
-  double* pd = base;                     // models, n * n_params
-  double* cd = base + NOALLOC_PARAMS;    // chi^2, n
-  double* dd = cd + NOALLOC_CHI2;        // delta_V, n * n_filters
-  const hipStream_t s = c->streams[0];
-  const int N = c->space.n_params, NF = c->curve.n_filters;
-  LaunchArgs a{};
-  a.op = 2;
-  a.stream = s;
-  a.pts = c->pts;
-  a.sum_w = c->sum_w;
-  a.n_data = c->curve.n_data;
-  a.n_filters = NF;
-  a.dof = c->curve.n_all - N - NF;
-  a.params = pd;
-  a.n = n;
-  a.chi2 = cd;
-  a.dV = dd;
-  hipError_t he = hipMemcpyAsync(pd, params, sizeof(double) * (size_t)n * N, hipMemcpyHostToDevice, s);
-  if (he == hipSuccess) he = hipEventRecord(c->ev0[0], s);
-  if (he == hipSuccess) he = dispatch(c->v, a);
-  if (he == hipSuccess) he = hipEventRecord(c->ev1[0], s);
-  if (he == hipSuccess) he = hipMemcpyAsync(chi2, cd, sizeof(double) * (size_t)n, hipMemcpyDeviceToHost, s);
-  if (he == hipSuccess) he = hipMemcpyAsync(dV, dd, sizeof(double) * (size_t)n * NF, hipMemcpyDeviceToHost, s);
-  if (he == hipSuccess) he = hipStreamSynchronize(s);
   float ms = 0;
-  if (he == hipSuccess) he = hipEventElapsedTime(&ms, c->ev0[0], c->ev1[0]);
+  hipError_t he;
+  if (c->mem.pin && chi2_bytes(c, n) <= IN_PLACE_BYTES) {  // (allocated by ast_ctx_create)
+    he = chi2_in_place(c, c->mem.pin, params, n, chi2, dV, &ms);
+  } else {
+    double* pd = base;                     // models, n * n_params
+    double* cd = base + NOALLOC_PARAMS;    // chi^2, n
+    double* dd = cd + NOALLOC_CHI2;        // delta_V, n * n_filters
+    const hipStream_t s = c->streams[0];
+    const size_t N = c->space.n_params, NF = c->curve.n_filters;
+    LaunchArgs a = chi2_args(c, pd, n, cd, dd, s);
+    he = hipMemcpyAsync(pd, params, sizeof(double) * (size_t)n * N, hipMemcpyHostToDevice, s);
+    if (he == hipSuccess) he = hipEventRecord(c->ev0[0], s);
+    if (he == hipSuccess) he = dispatch(c->v, a);
+    if (he == hipSuccess) he = hipEventRecord(c->ev1[0], s);
+    if (he == hipSuccess) he = hipMemcpyAsync(chi2, cd, sizeof(double) * (size_t)n, hipMemcpyDeviceToHost, s);
+    if (he == hipSuccess) he = hipMemcpyAsync(dV, dd, sizeof(double) * (size_t)n * NF, hipMemcpyDeviceToHost, s);
+    if (he == hipSuccess) he = hipStreamSynchronize(s);
+    if (he == hipSuccess) he = hipEventElapsedTime(&ms, c->ev0[0], c->ev1[0]);
+  }
   if (he != hipSuccess) {
+    (void)hipDeviceSynchronize();
     snprintf(g_hip_err, sizeof g_hip_err, "%s (chi2 batch, no allocation)", hipGetErrorString(he));
     return AST_E_HIP;
   }
@@ -2391,65 +2516,79 @@ int ast_model_curve(ast_ctx* c, const double* params, int n, const ast_ephem3* e
   if (c->serve) return AST_E_BUSY;
   if (!c->space_set || !c->curve_set || (c->v.nudge && !c->minima_set)) return AST_E_STATE;
   if (c->curve.n_all - c->space.n_params - c->curve.n_filters <= 0) return AST_E_DATA;
-  std::vector<PointRec> grid;
-  std::vector<double> tg;
-  int g0 = 0;
-  RETIF(make_grid(c->v, c->curve, *eph, n_plot, &grid, &tg, c->seg_t, &g0));
   RETIF(set_device(c));
-  const int np = c->space.n_params, nf = c->curve.n_filters;
-  PointRec* gd = nullptr;
-  double *pd = nullptr, *cd = nullptr, *dd = nullptr, *vd = nullptr;
-  int rc = dev_alloc(&gd, grid.size());
-  if (!rc) rc = dev_alloc(&pd, (size_t)n * np);
-  if (!rc) rc = dev_alloc(&cd, (size_t)n);
-  if (!rc) rc = dev_alloc(&dd, (size_t)n * nf);
-  if (!rc) rc = dev_alloc(&vd, (size_t)n * n_plot);
-  auto release = [&]() { dev_free(gd); dev_free(pd); dev_free(cd); dev_free(dd); dev_free(vd); };
-  if (rc) { release(); return rc; }
-  hipStream_t s = c->streams[0];
-  hipError_t he = hipMemcpy(gd, grid.data(), sizeof(PointRec) * grid.size(), hipMemcpyHostToDevice);
-  if (he == hipSuccess) he = hipMemcpy(pd, params, sizeof(double) * n * np, hipMemcpyHostToDevice);
-  LaunchArgs a{};
-  a.op = 3;
-  a.stream = s;
-  a.pts = c->pts;
-  a.sum_w = c->sum_w;
-  a.n_data = c->curve.n_data;
-  a.n_filters = nf;
-  a.dof = c->curve.n_all - np - nf;
-  a.params = pd;
-  a.n = n;
-  a.chi2 = cd;
-  a.dV = dd;
+  const size_t np = c->space.n_params, nf = c->curve.n_filters;
+  const size_t n_vmod = (size_t)n * n_plot, recs = (size_t)n_plot + 1;
+  // The grid is built in pinned memory where it fits (its copy is then one
+  // transfer), and small results are written in place behind it.
+  const size_t grid_bytes = Scratch::padded(sizeof(PointRec) * recs);
+  const size_t out_bytes = sizeof(double) * ((size_t)n * (np + 1 + nf) + n_vmod);
+  char* pin = c->mem.pinned(grid_bytes);
+  char* const out = pin && out_bytes <= IN_PLACE_BYTES && grid_bytes + out_bytes <= Memory::PIN_BYTES
+                        ? pin + grid_bytes : nullptr;
+  std::vector<PointRec> grid_v(pin ? 0 : recs);
+  std::vector<double> tg(t ? 0 : n_plot);
+  PointRec* const grid = pin ? (PointRec*)pin : grid_v.data();
+  Scratch sc(c->mem);
+  sc.reserve<PointRec>(recs);
+  if (!out) {
+    sc.reserve<double>((size_t)n * np);
+    sc.reserve<double>((size_t)n);
+    sc.reserve<double>((size_t)n * nf);
+    sc.reserve<double>(n_vmod);
+  }
+  RETIF(sc.take());
+  PointRec* const gd = sc.carve<PointRec>(recs);
+  double* const pd = out ? (double*)out : sc.carve<double>((size_t)n * np);
+  double* const cd = out ? pd + (size_t)n * np : sc.carve<double>((size_t)n);
+  double* const dd = out ? cd + n : sc.carve<double>((size_t)n * nf);
+  double* const vd = out ? dd + (size_t)n * nf : sc.carve<double>(n_vmod);
+  const hipStream_t s = c->streams[0];
+  hipError_t he = hipSuccess;
+  if (out) std::memcpy(pd, params, sizeof(double) * n * np);
+  else he = hipMemcpyAsync(pd, params, sizeof(double) * n * np, hipMemcpyHostToDevice, s);
+  LaunchArgs a = chi2_args(c, pd, n, cd, dd, s);
+  if (he == hipSuccess) he = hipEventRecord(c->ev0[0], s);
+  const bool rows = lanes_per_model(n) == 16;
+  if (rows && he == hipSuccess) he = dispatch(c->v, a);  // the observations' part, while the grid is built
+  int g0 = 0;
+  const int rc = make_grid(c->v, c->curve, *eph, n_plot, grid, t ? t : tg.data(), c->seg_t, &g0);
+  if (rc) {
+    (void)hipStreamSynchronize(s);
+    return rc;
+  }
+  a.op = rows ? 6 : 3;
   a.grid = gd;
   a.n_plot = n_plot;
   a.vmod = vd;
-  if (he == hipSuccess) he = hipEventRecord(c->ev0[0], s);
+  if (he == hipSuccess) he = hipMemcpyAsync(gd, grid, sizeof(PointRec) * recs, hipMemcpyHostToDevice, s);
   if (he == hipSuccess) he = dispatch(c->v, a);
   if (he == hipSuccess) he = hipEventRecord(c->ev1[0], s);
+  if (!out) {
+    if (he == hipSuccess) he = hipMemcpyAsync(chi2, cd, sizeof(double) * n, hipMemcpyDeviceToHost, s);
+    if (he == hipSuccess) he = hipMemcpyAsync(dV, dd, sizeof(double) * n * nf, hipMemcpyDeviceToHost, s);
+    if (he == hipSuccess) he = hipMemcpyAsync(vmod, vd, sizeof(double) * n_vmod, hipMemcpyDeviceToHost, s);
+  }
   if (he == hipSuccess) he = hipStreamSynchronize(s);
   float ms = 0;
   if (he == hipSuccess) he = hipEventElapsedTime(&ms, c->ev0[0], c->ev1[0]);
-  if (he == hipSuccess) he = hipMemcpy(chi2, cd, sizeof(double) * n, hipMemcpyDeviceToHost);
-  if (he == hipSuccess) he = hipMemcpy(dV, dd, sizeof(double) * n * nf, hipMemcpyDeviceToHost);
-  if (he == hipSuccess) he = hipMemcpy(vmod, vd, sizeof(double) * n * (size_t)n_plot, hipMemcpyDeviceToHost);
-  if (he == hipSuccess)
-    for (int k = 0; k < n; ++k)
-      for (int i = 0; i < g0; ++i) vmod[(size_t)k * n_plot + i] = std::nan("");
-  int result = AST_OK;
   if (he != hipSuccess) {
     (void)hipDeviceSynchronize();
     snprintf(g_hip_err, sizeof g_hip_err, "%s (model curve)", hipGetErrorString(he));
-    result = AST_E_HIP;
-  } else {
-    if (t) std::memcpy(t, tg.data(), sizeof(double) * n_plot);
-    c->last_ms = ms;
-    c->last_launches = 1;
-    c->last_evals = n;
-    c->last_points = (int64_t)n * (c->curve.n_data + n_plot);
+    return AST_E_HIP;
   }
-  release();
-  return result;
+  if (out) {
+    std::memcpy(chi2, cd, sizeof(double) * n);
+    std::memcpy(dV, dd, sizeof(double) * n * nf);
+    std::memcpy(vmod, vd, sizeof(double) * n_vmod);
+  }
+  for (int k = 0; k < n && g0 > 0; ++k)
+    for (int i = 0; i < g0; ++i) vmod[(size_t)k * n_plot + i] = std::nan("");
+  c->last_ms = ms;
+  c->last_launches = 1;
+  c->last_evals = n;
+  c->last_points = (int64_t)n * (c->curve.n_data + n_plot);
+  return AST_OK;
 }
 
 int ast_periodogram(ast_ctx* c, const double* t, const double* vm, int n, int n_clusters, double* cl_fr,
@@ -2467,7 +2606,8 @@ int ast_periodogram(ast_ctx* c, const double* t, const double* vm, int n, int n_
   }
   std::vector<int32_t> counts;
   RETIF(set_device(c));
-  RETIF(pgram_counts(c->streams[0], tm, &counts, &c->last_ms));
+  const hipEvent_t ev[2] = {c->ev0[0], c->ev1[0]};
+  RETIF(pgram_counts(c->streams[0], c->mem, ev, tm, &counts, &c->last_ms));
   c->last_launches = tm.size() >= 2 ? 1 : 0;
   pgram_clusters(counts, n_clusters, cl_fr, cl_H);
   return AST_OK;

@@ -1324,7 +1324,8 @@ __global__ __launch_bounds__(W == 4 ? 1024 : 256) __attribute__((amdgpu_waves_pe
 
 // --------------------------------------------------------- launch interface
 struct LaunchArgs {
-  int op;  // 0 init groups, 1 fit ticks, 2 chi2 batch, 3 model curve
+  int op;  // 0 init groups, 1 fit ticks, 2 chi2 batch, 3 model curve, 4 and 5 RMSD,
+           // 6 the grid of a model curve (16 lanes per model, after its chi2 batch)
   int precision;
   hipStream_t stream;
   // fit: descriptors of the groups of this launch (device), their count, G
@@ -1406,8 +1407,7 @@ hipError_t launch_nf(const LaunchArgs& a) {
     int blocks = (a.n + 255) / 256;
     hipLaunchKernelGGL((chi2_batch_kernel<CF, VC, NF, MX>), dim3(blocks), dim3(256), 0, a.stream, a.pts,
                        a.sum_w, a.n_data, a.n_filters, a.dof, a.params, a.n, a.chi2, a.dV);
-  } else if (a.op == 3 && lanes_per_model(a.n) == 16) {
-    launch_chi2_rows<CF, VC, NF, MX, 16>(a);
+  } else if (a.op == 6) {
     hipLaunchKernelGGL((curve_rows_kernel<CF, VC, NF, MX, 16>), dim3((a.n + 3) / 4), dim3(64), 0, a.stream, a.sum_w,
                        a.n_filters, a.dof, a.grid, a.n_plot, a.params, a.n, a.dV, a.vmod);
   } else if (a.op == 3) {

@@ -24,6 +24,10 @@ from . import abi
 LIGHT_SPEED = 173.144632674  # au/day (asteroid.h:287)
 
 
+_OBS = np.dtype([("mjd", "f8"), ("V", "f4"), ("w", "f4"), ("filter", "i4"), ("pad_", "i4"), ("E", "f8", 3),
+                 ("S", "f8", 3)])  # abi.Obs
+
+
 class Curve:
     """One light curve after ingest: the contents of ast_upload_curve."""
 
@@ -43,15 +47,11 @@ class Curve:
 
     def obs_array(self):
         arr = (abi.Obs * self.n_data)()
-        for i in range(self.n_data):
-            o = arr[i]
-            o.mjd = self.mjd[i]
-            o.V = self.V[i]
-            o.w = self.w[i]
-            o.filter = int(self.filter[i])
-            for c in range(3):
-                o.E[c] = self.E[i, c]
-                o.S[c] = self.S[i, c]
+        if not self.n_data:
+            return arr
+        rec = np.frombuffer(arr, dtype=_OBS)  # a view: filled column by column
+        rec["mjd"], rec["V"], rec["w"], rec["filter"] = self.mjd, self.V, self.w, self.filter
+        rec["E"], rec["S"] = self.E, self.S
         return arr
 
     def ephem3(self):
