@@ -1252,6 +1252,34 @@ int class_batch_update(ast_ctx* c, int k, const std::vector<DevJob*>& members) {
   return 0;
 }
 
+// A cycle of few fits with more classes than streams: classes that differ in
+// their filter capacity only share the launch of the larger one (which keeps
+// a fit's values as they are: the sums of filters a job does not have are not
+// used), while there are too many.  A class more than streams makes a cycle
+// up to twice as long: 8 served requests in 5 classes took 58 ms, in 4 they take
+// 44.
+void merge_classes(std::vector<DevJob*>* members, double* load) {
+  for (;;) {
+    int n = 0, to = -1, from = -1;
+    for (int k = 0; k < MAX_CLASSES; ++k) {
+      if (members[k].empty()) continue;
+      n++;
+      // class index (variant * 3 + capacity) * 3 + precision form
+      for (int q = k + 3; q / 9 == k / 9; q += 3)
+        if (!members[q].empty() && (to < 0 || std::max(load[k], load[q]) < std::max(load[from], load[to]))) {
+          from = k;
+          to = q;
+        }
+    }
+    if (n <= NSTREAMS || to < 0) return;
+    // the job with the most filters first: it gives the launch its capacity
+    members[to].insert(members[to].end(), members[from].begin(), members[from].end());
+    members[from].clear();
+    load[to] = std::max(load[to], load[from]);
+    load[from] = 0;
+  }
+}
+
 // One fit-kernel launch of class k over the class batch, on its stream.
 hipError_t launch_class(ast_ctx* c, int k, const DevJob& j0, int lanes, int stream) {
   LaunchArgs a{};
@@ -1334,6 +1362,7 @@ int run_cycle_once(ast_ctx* c, std::vector<DevJob*>& jobs, double* kernel_ms, in
     fits += (double)j->n_workers * c->pool.G * (t / longest);
   }
   const int lanes = lanes_per_model((int64_t)std::ceil(fits));  // the classes of a cycle run side by side
+  if (lanes > 1) merge_classes(members, load);
   int stream[MAX_CLASSES];
   assign_streams(load, stream);
   for (int k = 0; k < MAX_CLASSES; ++k)
