@@ -854,6 +854,36 @@ __device__ inline void store_lane(const SlotBufs<CF>& B, size_t fit, size_t fo, 
   B.sf[fo] = R.sf;
 }
 
+// One evaluation with LP lanes per model (chi2_model_rows), for the kernels
+// below: parameters at PRM[i * stride], delta_V to DV[m * dv_stride].  Out of
+// line, so that a kernel class has one copy of it for its kernels.
+template <class CF, int VC, int NF, bool MX, int LP>
+__device__ __attribute__((noinline)) CF eval_rows(const double* PRM, size_t stride, CF* DV, size_t dv_stride,
+                                                   const PointRec* pts_g, int n_data, int n_filters, int dof,
+                                                   const double* sum_w) {
+  constexpr int N = Pos<VC>::N;
+  const uint64_t pu = (uint64_t)(uintptr_t)pts_g;
+  const uint64_t plo = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)pu);
+  const uint64_t phi = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(pu >> 32));
+  const uintptr_t pa = (uintptr_t)((phi << 32) | plo);
+  n_data = __builtin_amdgcn_readfirstlane(n_data);
+  n_filters = __builtin_amdgcn_readfirstlane(n_filters);
+  dof = __builtin_amdgcn_readfirstlane(dof);
+  double prm[N];
+#pragma unroll
+  for (int i = 0; i < N; ++i) prm[i] = PRM[(size_t)i * stride];
+  CF dv[NF];
+#pragma unroll
+  for (int m = 0; m < NF; ++m)  // a failed NUDGE model leaves delta_V as it was
+    dv[m] = VarF<VC>::NU && m < n_filters ? DV[(size_t)m * dv_stride] : CF(0);
+  CF fv = chi2_model_rows<CF, VC, NF, MX, FORM_CHI2, LP>(prm, (PointPtr)pa, (LanePtr)pa, n_data, n_filters,
+                                                         dof, sum_w, dv);
+#pragma unroll
+  for (int m = 0; m < NF; ++m)
+    if (m < n_filters) DV[(size_t)m * dv_stride] = dv[m];
+  return fv;
+}
+
 // ---------------------------------------------------------------- fit kernel
 // One workgroup = one group (the reference's block); it runs D.ticks rounds
 // of "evaluate the pending points, advance every lane", then saves its state.
@@ -933,7 +963,11 @@ void fit_kernel(const GroupDesc<CF>* descs, SlotBufs<CF> B) {
     // back through LDS.  Fits that stop at an evaluation budget still end
     // within 12 rounds of each other (a shrink is finished): 224 groups, two
     // stages of 50 evaluations, 78 -> 72 ms; 2^18 fits of 100, mixed, 215 -> 209.
-    const bool pack = pending <= G - 64;
+    // With the chip's SIMDs not shared (groups of 65536 fits at most), few enough
+    // points take 4 or 16 lanes each.
+    const bool spread = (size_t)gridDim.x * G <= 65536;
+    const int lp = spread && pending * 16 <= G ? 16 : spread && pending * 4 <= G ? 4 : 1;
+    const bool pack = pending <= G - 64 || lp > 1;
     int e = t;
     bool eval = have;
     if (pack) {
@@ -946,12 +980,20 @@ void fit_kernel(const GroupDesc<CF>* descs, SlotBufs<CF> B) {
       base = __builtin_amdgcn_readfirstlane(base);
       if (have) s_fit[base + __popcll(mask & ((1ull << lane) - 1ull))] = (uint16_t)t;
       __syncthreads();
-      eval = t < pending;
-      if (eval) e = s_fit[t];
+      eval = t / lp < pending;
+      if (eval) e = s_fit[t / lp];
     }
-    if (eval)
-      fv = eval_lane<CF, VC, NF, MX, MX ? 4 : W>(B.PRM, B.DV, nf, (size_t)slot * G + e, rs,
-                                                 (size_t)slot * G * KC + e, D.pts, D.n_data, D.n_filters, D.dof,
+    const size_t efit = (size_t)slot * G + e, efo = (size_t)slot * G * KC + e;
+    if (lp == 16) {
+      if (eval)
+        fv = eval_rows<CF, VC, NF, MX, 16>(B.PRM + efit, nf, B.DV + efo, rs, D.pts, D.n_data, D.n_filters, D.dof,
+                                           D.sum_w);
+    } else if (lp == 4) {
+      if (eval)
+        fv = eval_rows<CF, VC, NF, MX, 4>(B.PRM + efit, nf, B.DV + efo, rs, D.pts, D.n_data, D.n_filters, D.dof,
+                                          D.sum_w);
+    } else if (eval)
+      fv = eval_lane<CF, VC, NF, MX, MX ? 4 : W>(B.PRM, B.DV, nf, efit, rs, efo, D.pts, D.n_data, D.n_filters, D.dof,
                                                  D.sum_w);
     if (pack) {
       if (eval) s_val[e] = fv;
@@ -977,36 +1019,6 @@ void fit_kernel(const GroupDesc<CF>* descs, SlotBufs<CF> B) {
 }
 
 // ---------------------------------------------------- several lanes per model
-// One evaluation with LP lanes per model (chi2_model_rows), for the kernels
-// below: parameters at PRM[i * stride], delta_V to DV[m * dv_stride].  Out of
-// line, so that a kernel class has one copy of it for its kernels.
-template <class CF, int VC, int NF, bool MX, int LP>
-__device__ __attribute__((noinline)) CF eval_rows(const double* PRM, size_t stride, CF* DV, size_t dv_stride,
-                                                   const PointRec* pts_g, int n_data, int n_filters, int dof,
-                                                   const double* sum_w) {
-  constexpr int N = Pos<VC>::N;
-  const uint64_t pu = (uint64_t)(uintptr_t)pts_g;
-  const uint64_t plo = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)pu);
-  const uint64_t phi = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(pu >> 32));
-  const uintptr_t pa = (uintptr_t)((phi << 32) | plo);
-  n_data = __builtin_amdgcn_readfirstlane(n_data);
-  n_filters = __builtin_amdgcn_readfirstlane(n_filters);
-  dof = __builtin_amdgcn_readfirstlane(dof);
-  double prm[N];
-#pragma unroll
-  for (int i = 0; i < N; ++i) prm[i] = PRM[(size_t)i * stride];
-  CF dv[NF];
-#pragma unroll
-  for (int m = 0; m < NF; ++m)  // a failed NUDGE model leaves delta_V as it was
-    dv[m] = VarF<VC>::NU && m < n_filters ? DV[(size_t)m * dv_stride] : CF(0);
-  CF fv = chi2_model_rows<CF, VC, NF, MX, FORM_CHI2, LP>(prm, (PointPtr)pa, (LanePtr)pa, n_data, n_filters,
-                                                         dof, sum_w, dv);
-#pragma unroll
-  for (int m = 0; m < NF; ++m)
-    if (m < n_filters) DV[(size_t)m * dv_stride] = dv[m];
-  return fv;
-}
-
 // Registers for one or two waves per SIMD: these kernels run where the chip
 // is not full.
 #define AST_ROWS_BOUNDS __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 2)))
