@@ -1281,7 +1281,7 @@ void merge_classes(std::vector<DevJob*>* members, double* load) {
 }
 
 // One fit-kernel launch of class k over the class batch, on its stream.
-hipError_t launch_class(ast_ctx* c, int k, const DevJob& j0, int lanes, int stream) {
+hipError_t launch_class(ast_ctx* c, int k, const DevJob& j0, int64_t fits, int stream) {
   LaunchArgs a{};
   a.op = 1;
   a.stream = c->streams[stream];
@@ -1294,19 +1294,22 @@ hipError_t launch_class(ast_ctx* c, int k, const DevJob& j0, int lanes, int stre
   a.group_size = c->pool.G;
   a.n_filters = j0.n_filters;
   a.waves = c->waves[k];
-  a.lanes = lanes;
+  a.fits = fits;
   return dispatch(j0.space.v, a);
 }
 
 // The cycle as a HIP graph: every class launch, forked from stream 0 onto
 // the classes' streams and joined back.  Valid while the class batches, the
 // pool and the register budgets are unchanged (the key).
-int cycle_graph(ast_ctx* c, std::vector<DevJob*>* members, const bool* used_s, int lanes, const int* stream) {
+int cycle_graph(ast_ctx* c, std::vector<DevJob*>* members, const bool* used_s, int64_t fits, const int* stream) {
   std::vector<uint64_t> key{(uint64_t)(uintptr_t)c->pool.X, (uint64_t)c->pool.nf, (uint64_t)c->pool.G};
   for (int k = 0; k < MAX_CLASSES; ++k) {
     if (members[k].empty()) continue;
     key.push_back((uint64_t)k);
     key.push_back((uint64_t)c->waves[k]);
+    const ast_variant& v = members[k][0]->space.v;
+    const RowShape shape = fit_shape(v.torque || v.torque2, v.torque2, fits);
+    key.push_back((uint64_t)(2 * shape.lanes + shape.team));
     key.push_back((uint64_t)(uintptr_t)c->batch[k].d_descs);
     key.push_back((uint64_t)c->batch[k].n_groups);
     for (uint64_t u : c->batch[k].members) key.push_back(u);
@@ -1321,7 +1324,7 @@ int cycle_graph(ast_ctx* c, std::vector<DevJob*>* members, const bool* used_s, i
   for (int k = 1; k < NSTREAMS && e == hipSuccess; ++k)
     if (used_s[k]) e = hipStreamWaitEvent(c->streams[k], c->ev_fork, 0);
   for (int k = 0; k < MAX_CLASSES && e == hipSuccess; ++k)
-    if (!members[k].empty()) e = launch_class(c, k, *members[k][0], lanes, stream[k]);
+    if (!members[k].empty()) e = launch_class(c, k, *members[k][0], fits, stream[k]);
   for (int k = 1; k < NSTREAMS && e == hipSuccess; ++k)
     if (used_s[k]) {
       e = hipEventRecord(c->ev_join[k], c->streams[k]);
@@ -1361,8 +1364,8 @@ int run_cycle_once(ast_ctx* c, std::vector<DevJob*>& jobs, double* kernel_ms, in
     load[j->cls] = std::max(load[j->cls], t);
     fits += (double)j->n_workers * c->pool.G * (t / longest);
   }
-  const int lanes = lanes_per_model((int64_t)std::ceil(fits));  // the classes of a cycle run side by side
-  if (lanes > 1) merge_classes(members, load);
+  const int64_t side = (int64_t)std::ceil(fits);  // the classes of a cycle run side by side
+  if (side <= ROWS_MAX) merge_classes(members, load);
   int stream[MAX_CLASSES];
   assign_streams(load, stream);
   for (int k = 0; k < MAX_CLASSES; ++k)
@@ -1377,7 +1380,7 @@ int run_cycle_once(ast_ctx* c, std::vector<DevJob*>& jobs, double* kernel_ms, in
   std::vector<int32_t> done(jobs.size());
   if (graphs && n_cls > 0) {
     // one graph launch on stream 0; every class stream joins back into it
-    RETIF(cycle_graph(c, members, used_s, lanes, stream));
+    RETIF(cycle_graph(c, members, used_s, side, stream));
     const hipStream_t s0 = c->streams[0];
     HIPCHK(hipEventRecord(c->ev0[0], s0));
     HIPCHK(hipGraphLaunch(c->cg_exec, s0));
@@ -1398,7 +1401,7 @@ int run_cycle_once(ast_ctx* c, std::vector<DevJob*>& jobs, double* kernel_ms, in
       if (used_s[k]) HIPCHK(hipEventRecord(c->ev0[k], c->streams[k]));
     for (int k = 0; k < MAX_CLASSES; ++k) {
       if (members[k].empty()) continue;
-      HIPCHK(launch_class(c, k, *members[k][0], lanes, stream[k]));
+      HIPCHK(launch_class(c, k, *members[k][0], side, stream[k]));
       (*launches)++;
     }
     for (int k = 0; k < NSTREAMS; ++k)
@@ -2189,7 +2192,7 @@ int ast_run_begin(ast_ctx* c, const ast_run_cfg* rc) {
     double t = 3.0e9 / (tot > 1 ? tot : 1);
     ticks = (int)(t < 16 ? 16 : (t > 4096 ? 4096 : t));
     // with several lanes per model a stage ends between launches
-    if (rc->nstages > 1 && lanes_per_model((int64_t)lanes) > 1 && ticks > 64) ticks = 64;
+    if (rc->nstages > 1 && (int64_t)lanes <= ROWS_MAX && ticks > 64) ticks = 64;
   }
   j.ticks = ticks;
   RETIF(job_upload(j, c->pool, c->curve, c->params0, s, c->mem));
@@ -2596,7 +2599,7 @@ int ast_model_curve(ast_ctx* c, const double* params, int n, const ast_ephem3* e
   else he = hipMemcpyAsync(pd, params, sizeof(double) * n * np, hipMemcpyHostToDevice, s);
   LaunchArgs a = chi2_args(c, pd, n, cd, dd, s);
   if (he == hipSuccess) he = hipEventRecord(c->ev0[0], s);
-  const bool rows = lanes_per_model(n) == 16;
+  const bool rows = n <= CURVE_ROWS_MAX;
   if (rows && he == hipSuccess) he = dispatch(c->v, a);  // the observations' part, while the grid is built
   int g0 = 0;
   const int rc = make_grid(c->v, c->curve, *eph, n_plot, grid, t ? t : tg.data(), c->seg_t, &g0);

@@ -857,10 +857,10 @@ __device__ inline void store_lane(const SlotBufs<CF>& B, size_t fit, size_t fo, 
 // One evaluation with LP lanes per model (chi2_model_rows), for the kernels
 // below: parameters at PRM[i * stride], delta_V to DV[m * dv_stride].  Out of
 // line, so that a kernel class has one copy of it for its kernels.
-template <class CF, int VC, int NF, bool MX, int LP>
+template <class CF, int VC, int NF, bool MX, int LP, int ROLE = ROLE_ALL>
 __device__ __attribute__((noinline)) CF eval_rows(const double* PRM, size_t stride, CF* DV, size_t dv_stride,
                                                    const PointRec* pts_g, int n_data, int n_filters, int dof,
-                                                   const double* sum_w) {
+                                                   const double* sum_w, TeamPtr<VC, LP> team = nullptr) {
   constexpr int N = Pos<VC>::N;
   const uint64_t pu = (uint64_t)(uintptr_t)pts_g;
   const uint64_t plo = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)pu);
@@ -876,8 +876,8 @@ __device__ __attribute__((noinline)) CF eval_rows(const double* PRM, size_t stri
 #pragma unroll
   for (int m = 0; m < NF; ++m)  // a failed NUDGE model leaves delta_V as it was
     dv[m] = VarF<VC>::NU && m < n_filters ? DV[(size_t)m * dv_stride] : CF(0);
-  CF fv = chi2_model_rows<CF, VC, NF, MX, FORM_CHI2, LP>(prm, (PointPtr)pa, (LanePtr)pa, n_data, n_filters,
-                                                         dof, sum_w, dv);
+  CF fv = chi2_model_rows<CF, VC, NF, MX, FORM_CHI2, LP, ROLE>(prm, (PointPtr)pa, (LanePtr)pa, n_data, n_filters,
+                                                               dof, sum_w, dv, nullptr, 0.0, team);
 #pragma unroll
   for (int m = 0; m < NF; ++m)
     if (m < n_filters) DV[(size_t)m * dv_stride] = dv[m];
@@ -1060,6 +1060,55 @@ __global__ AST_ROWS_BOUNDS void curve_rows_kernel(const double* sum_w, int n_fil
                                                  sum_w, dv, vmod + (size_t)k * n_plot, dV[(size_t)k * n_filters]);
 }
 
+// The two kernels above with a team of wavefronts for 64 / LP models (rows past
+// the last model repeat it).
+#define AST_TEAM_BOUNDS __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(1, 3)))
+template <int VC>
+constexpr int TEAM_THREADS = VarF<VC>::TQ ? 192 : 128;
+
+template <class CF, int VC, int NF, bool MX, int LP>
+__global__ AST_TEAM_BOUNDS void chi2_team_kernel(const PointRec* pts_g, const double* sum_w, int n_data, int n_filters,
+                                                 int dof, const double* params, int n, double* chi2, double* dV) {
+  astm::sincos_table_load();
+  constexpr int N = Pos<VC>::N, M = 64 / LP;
+  __shared__ TeamLds<VarF<VC>::TQ, LP> s_team;
+  __shared__ CF s_dv[M][NF];
+  const TeamPtr<VC, LP> team = (TeamPtr<VC, LP>)&s_team;
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x / 64);
+  const int row = (int)threadIdx.x % 64 / LP;
+  const int k = (int)blockIdx.x * M + row < n ? (int)blockIdx.x * M + row : n - 1;
+  const double* prm = params + (size_t)k * N;
+  if (wave > 0) return team_helper<VC, LP>(wave, prm, 1, pts_g, n_data, team);
+  for (int m = 0; m < NF; ++m) s_dv[row][m] = VarF<VC>::NU ? CF(__builtin_nan("")) : CF(0);
+  const CF c = eval_rows<CF, VC, NF, MX, LP, ROLE_LIGHT>(prm, 1, s_dv[row], 1, pts_g, n_data, n_filters, dof, sum_w,
+                                                         team);
+  chi2[k] = c;
+  for (int m = 0; m < n_filters; ++m) dV[(size_t)k * n_filters + m] = s_dv[row][m];
+}
+
+template <class CF, int VC, int NF, bool MX, int LP>
+__global__ AST_TEAM_BOUNDS void curve_team_kernel(const double* sum_w, int n_filters, int dof, const PointRec* grid_g,
+                                                  int n_plot, const double* params, int n, const double* dV,
+                                                  double* vmod) {
+  astm::sincos_table_load();
+  constexpr int N = Pos<VC>::N, M = 64 / LP;
+  __shared__ TeamLds<VarF<VC>::TQ, LP> s_team;
+  const TeamPtr<VC, LP> team = (TeamPtr<VC, LP>)&s_team;
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x / 64);
+  const int row = (int)threadIdx.x % 64 / LP;
+  const int k = (int)blockIdx.x * M + row < n ? (int)blockIdx.x * M + row : n - 1;
+  const double* pk = params + (size_t)k * N;
+  if (wave > 0) return team_helper<VC, LP>(wave, pk, 1, grid_g, n_plot, team);
+  double prm[N];
+#pragma unroll
+  for (int i = 0; i < N; ++i) prm[i] = pk[i];
+  CF dv[NF];
+  chi2_model_rows<CF, VC, NF, MX, FORM_PLOT, LP, ROLE_LIGHT>(prm, (PointPtr)(uintptr_t)grid_g,
+                                                             (LanePtr)(uintptr_t)grid_g, n_plot, n_filters, dof, sum_w,
+                                                             dv, vmod + (size_t)k * n_plot,
+                                                             dV[(size_t)k * n_filters], team);
+}
+
 // take_fit for LP lanes per model: one fit per asking model.
 template <int LP>
 __device__ inline int take_fit_rows(int32_t* queue) {
@@ -1084,19 +1133,37 @@ __device__ inline int take_fit_rows(int32_t* queue) {
 // the model's state (equal values to the same addresses).  A wavefront ends
 // its launch when none of its simplexes has a pending point; the end of the
 // group's stage, which needs them all, is group_step_kernel's, launched
-// after it.
-template <class CF, int VC, int NF, bool MX, int LP>
-__global__ AST_ROWS_BOUNDS void fit_rows_kernel(const GroupDesc<CF>* descs, SlotBufs<CF> B, int G) {
+// after it.  With TEAM the wavefront is the first of a team, whose others
+// take their parts of its evaluations.
+template <class CF, int VC, int NF, bool MX, int LP, bool TEAM>
+__device__ inline void fit_rows(const GroupDesc<CF>* descs, const SlotBufs<CF>& B, int G) {
   astm::sincos_table_load();
   constexpr int KC = 8 / sizeof(CF), MODELS = 64 / LP;
   const int per_group = G / MODELS;
   const GroupDesc<CF>& D = descs[blockIdx.x / per_group];
-  const int t = (int)(blockIdx.x % per_group) * MODELS + (int)threadIdx.x / LP;
+  const int t = (int)(blockIdx.x % per_group) * MODELS + (int)threadIdx.x % 64 / LP;
   const int slot = D.slot;
   const size_t nf = B.nf, rs = KC * nf;
   const size_t fit = (size_t)slot * G + t;
   const size_t fo = (size_t)slot * G * KC + t;
   if (B.g_done[slot]) return;
+  TeamPtr<VC, LP> team = nullptr;
+  uint64_t* pending = nullptr;  // the lanes to evaluate; 0 ends the launch
+  if constexpr (TEAM) {
+    __shared__ TeamLds<VarF<VC>::TQ, LP> s_team;
+    __shared__ uint64_t s_pending;
+    team = (TeamPtr<VC, LP>)&s_team;
+    pending = &s_pending;
+    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x / 64);
+    if (wave > 0) {
+      for (;;) {
+        __syncthreads();
+        const uint64_t lanes = s_pending;
+        if (lanes == 0) return;
+        if (lanes >> __lane_id() & 1) team_helper<VC, LP>(wave, B.PRM + fit, nf, D.pts, D.n_data, team);
+      }
+    }
+  }
   Machine<CF, VC> M = Machine<CF, VC>::of(D, B, fit, fo, (uint64_t)B.fitid[fit], B.g_reopt[slot]);
   const int ticks = D.ticks;
   LaneRegs<CF> R = load_lane(B, fit, fo, D.rng[M.jfit]);
@@ -1119,10 +1186,15 @@ __global__ AST_ROWS_BOUNDS void fit_rows_kernel(const GroupDesc<CF>* descs, Slot
       }
     }
     have = phase_pending(R.phase);
-    if (tick == ticks || __ballot(have) == 0) break;
+    const uint64_t lanes = tick == ticks ? 0 : __ballot(have);
+    if constexpr (TEAM) {
+      *pending = lanes;
+      __syncthreads();
+    }
+    if (lanes == 0) break;
     if (have) {
-      fv = eval_rows<CF, VC, NF, MX, LP>(B.PRM + fit, nf, B.DV + fo, rs, D.pts, D.n_data, D.n_filters, D.dof,
-                                         D.sum_w);
+      fv = eval_rows<CF, VC, NF, MX, LP, TEAM ? ROLE_LIGHT : ROLE_ALL>(B.PRM + fit, nf, B.DV + fo, rs, D.pts, D.n_data,
+                                                                       D.n_filters, D.dof, D.sum_w, team);
       R.nev++;
       R.nev_tot++;
       R.work++;
@@ -1131,6 +1203,15 @@ __global__ AST_ROWS_BOUNDS void fit_rows_kernel(const GroupDesc<CF>* descs, Slot
   const uint64_t jfit = M.jfit;
   store_lane(B, fit, fo, R, jfit);
   D.rng[jfit] = R.rng;
+}
+
+template <class CF, int VC, int NF, bool MX, int LP>
+__global__ AST_ROWS_BOUNDS void fit_rows_kernel(const GroupDesc<CF>* descs, SlotBufs<CF> B, int G) {
+  fit_rows<CF, VC, NF, MX, LP, false>(descs, B, G);
+}
+template <class CF, int VC, int NF, bool MX, int LP>
+__global__ AST_TEAM_BOUNDS void fit_team_kernel(const GroupDesc<CF>* descs, SlotBufs<CF> B, int G) {
+  fit_rows<CF, VC, NF, MX, LP, true>(descs, B, G);
 }
 
 // After fit_rows_kernel: one workgroup per group ends the group's stage once
@@ -1386,7 +1467,7 @@ struct LaunchArgs {
   const void* bufs;    // SlotBufs<CF>*
   int n_groups, group_size, n_filters;
   int waves;           // fit kernel register budget: 4, 3 or 2 waves per SIMD
-  int lanes;           // fit: lanes per model (lanes_per_model)
+  int64_t fits;        // fit: fits evaluated side by side (fit_shape)
   // batch
   const PointRec* pts;
   const double* sum_w;
@@ -1403,42 +1484,88 @@ struct LaunchArgs {
   const void* rmsd;
 };
 
-// Lanes per model for n models evaluated side by side: as many as leave each
-// of the 1024 SIMDs one wavefront, since a wavefront alone takes its own time
-// whatever its lanes hold.  Kernel time at 16 / 4 / 1 lanes, LS + torque,
-// 400 points over 3 days, FP64 -- chi^2: 64 models 292 / 363 / 530 us, 4096
-// 356 / 376 / 533, 6144 588 / 389 / 533, 16384 1132 / 418 / 533, 24576
-// - / 679 / 539; fits of 30 evaluations: 4096 17.2 / 17.9 / 38.4 ms, 16384
-// 54.6 / 24.9 / 39.7, 24576 - / 37.3 / 39.8.  The mixed form and the form
-// without torque cross at the same sizes.
-constexpr int ROWS16_MAX = 4096, ROWS4_MAX = 16384;
-inline int lanes_per_model(int64_t n) { return n <= ROWS16_MAX ? 16 : n <= ROWS4_MAX ? 4 : 1; }
+// Lanes per model, and whether a team of wavefronts walks the models of a
+// wavefront, for n models (fits, in a cycle) evaluated side by side: as many
+// lanes as leave each of the 1024 SIMDs one wavefront, since a wavefront alone
+// takes its own time whatever its lanes hold, and teams where their two
+// wavefronts (three with torque, of which the first is idle half the time)
+// find a SIMD each; the model cut in two parts (torque2) has no teams, its
+// step counts being the model's own.
+// Kernel time at 16 / 4 / 1 lanes without teams, LS + torque, 400 points over 3
+// days, FP64 -- chi^2: 64 models 279 / 363 / 530 us, 4096 346 / 376 / 533, 6144
+// 588 / 371 / 533, 16384 1132 / 423 / 533, 24576 - / 679 / 539; fits of 30
+// evaluations: 4096 15.3 / 17.9 / 38.4 ms, 16384 54.6 / 22.3 / 39.7, 24576
+// - / 37.3 / 39.8.
+// Teams of 16 / 4 lanes -- torque: chi^2 64 models 245 / 260 us, 1024 262 / 265,
+// 2048 - / 268, 4096 - / 279 (without 346), 6144 - / 345 (371), 12288 - / 397
+// (401); fits 1024 11.6 / 12.9 ms (13.0), 4096 - / 13.3 (15.3), 6144 - / 23.5
+// (18.6).  Without torque, where only the brightness is taken off: chi^2 1024
+// 292 / 306 us (301), 4096 - / 318 (345), 8192 - / 341 (405), 16384 - / 437
+// (442); fits 1024 12.2 / 13.9 ms (13.0), 8192 - / 16.1 (19.6), 12288 - / 26.2
+// (21.6), but re-optimised fits of 818 points on 3328 lanes 45.5 against 44.0,
+// since a wavefront then runs 16 simplexes' bookkeeping instead of 4.
+struct RowShape {
+  int lanes;
+  bool team;
+};
+constexpr RowShape chi2_shape(bool torque, bool torque2, int64_t n) {
+  if (torque2) return {n <= 4096 ? 16 : n <= 16384 ? 4 : 1, false};
+  const bool team = n <= (torque ? 4096 : 8192);
+  return {n <= 1024 ? 16 : n <= 16384 ? 4 : 1, team};
+}
+constexpr RowShape fit_shape(bool torque, bool torque2, int64_t n) {
+  if (torque && !torque2) return chi2_shape(torque, torque2, n);
+  return {n <= 4096 ? 16 : n <= 16384 ? 4 : 1, !torque2 && n > 4096 && n <= 8192};
+}
+constexpr int64_t ROWS_MAX = 16384;       // more models take a lane each
+constexpr int CURVE_ROWS_MAX = 4096;      // more model curves
 
-template <class CF, int VC, int NF, bool MX, int LP>
+template <class CF, int VC, int NF, bool MX, int LP, bool TEAM>
 void launch_chi2_rows(const LaunchArgs& a) {
-  constexpr int M = 64 / LP;
-  hipLaunchKernelGGL((chi2_rows_kernel<CF, VC, NF, MX, LP>), dim3((a.n + M - 1) / M), dim3(64), 0, a.stream, a.pts,
-                     a.sum_w, a.n_data, a.n_filters, a.dof, a.params, a.n, a.chi2, a.dV);
+  const dim3 grid((a.n + 64 / LP - 1) / (64 / LP));
+  if constexpr (TEAM)
+    hipLaunchKernelGGL((chi2_team_kernel<CF, VC, NF, MX, LP>), grid, dim3(TEAM_THREADS<VC>), 0, a.stream, a.pts,
+                       a.sum_w, a.n_data, a.n_filters, a.dof, a.params, a.n, a.chi2, a.dV);
+  else
+    hipLaunchKernelGGL((chi2_rows_kernel<CF, VC, NF, MX, LP>), grid, dim3(64), 0, a.stream, a.pts, a.sum_w, a.n_data,
+                       a.n_filters, a.dof, a.params, a.n, a.chi2, a.dV);
 }
 template <class CF, int VC, int NF, bool MX, int LP>
+void launch_curve_rows(const LaunchArgs& a) {
+  const dim3 grid((a.n + 64 / LP - 1) / (64 / LP));
+  if constexpr (VarF<VC>::T2)
+    hipLaunchKernelGGL((curve_rows_kernel<CF, VC, NF, MX, LP>), grid, dim3(64), 0, a.stream, a.sum_w, a.n_filters,
+                       a.dof, a.grid, a.n_plot, a.params, a.n, a.dV, a.vmod);
+  else
+    hipLaunchKernelGGL((curve_team_kernel<CF, VC, NF, MX, LP>), grid, dim3(TEAM_THREADS<VC>), 0, a.stream, a.sum_w,
+                       a.n_filters, a.dof, a.grid, a.n_plot, a.params, a.n, a.dV, a.vmod);
+}
+template <class CF, int VC, int NF, bool MX, int LP, bool TEAM>
 void launch_fit_rows(const LaunchArgs& a) {
-  constexpr int M = 64 / LP;
   const GroupDesc<CF>* d = (const GroupDesc<CF>*)a.descs;
   const SlotBufs<CF>& B = *(const SlotBufs<CF>*)a.bufs;
-  hipLaunchKernelGGL((fit_rows_kernel<CF, VC, NF, MX, LP>), dim3(a.n_groups * (a.group_size / M)), dim3(64), 0,
-                     a.stream, d, B, a.group_size);
+  const dim3 grid(a.n_groups * (a.group_size / (64 / LP)));
+  if constexpr (TEAM)
+    hipLaunchKernelGGL((fit_team_kernel<CF, VC, NF, MX, LP>), grid, dim3(TEAM_THREADS<VC>), 0, a.stream, d, B,
+                       a.group_size);
+  else
+    hipLaunchKernelGGL((fit_rows_kernel<CF, VC, NF, MX, LP>), grid, dim3(64), 0, a.stream, d, B, a.group_size);
   hipLaunchKernelGGL((group_step_kernel<CF, VC>), dim3(a.n_groups), dim3(a.group_size), 0, a.stream, d, B);
 }
 
 template <class CF, int VC, int NF, bool MX>
 hipError_t launch_nf(const LaunchArgs& a) {
+  constexpr bool TQ = VarF<VC>::TQ, T2 = VarF<VC>::T2;
+  const RowShape fit = fit_shape(TQ, T2, a.fits), chi2 = chi2_shape(TQ, T2, a.n);
   if (a.op == 0) {
     hipLaunchKernelGGL((fit_init_kernel<CF, VC>), dim3(a.n_groups), dim3(a.group_size), 0, a.stream,
                        (const GroupDesc<CF>*)a.descs, *(const SlotBufs<CF>*)a.bufs);
-  } else if (a.op == 1 && a.lanes == 16) {
-    launch_fit_rows<CF, VC, NF, MX, 16>(a);
-  } else if (a.op == 1 && a.lanes == 4) {
-    launch_fit_rows<CF, VC, NF, MX, 4>(a);
+  } else if (a.op == 1 && fit.lanes == 16) {
+    launch_fit_rows<CF, VC, NF, MX, 16, TQ && !T2>(a);
+  } else if (a.op == 1 && fit.lanes == 4 && fit.team) {
+    launch_fit_rows<CF, VC, NF, MX, 4, !T2>(a);
+  } else if (a.op == 1 && fit.lanes == 4) {
+    launch_fit_rows<CF, VC, NF, MX, 4, false>(a);
   } else if (a.op == 1) {
     const GroupDesc<CF>* d = (const GroupDesc<CF>*)a.descs;
     const SlotBufs<CF>& B = *(const SlotBufs<CF>*)a.bufs;
@@ -1452,17 +1579,20 @@ hipError_t launch_nf(const LaunchArgs& a) {
     else
       hipLaunchKernelGGL((fit_kernel<CF, VC, NF, MX, 4>), dim3(a.n_groups), dim3(a.group_size), 0, a.stream,
                          d, B);
-  } else if (a.op == 2 && lanes_per_model(a.n) == 16) {
-    launch_chi2_rows<CF, VC, NF, MX, 16>(a);
-  } else if (a.op == 2 && lanes_per_model(a.n) == 4) {
-    launch_chi2_rows<CF, VC, NF, MX, 4>(a);
+  } else if (a.op == 2 && chi2.lanes == 16) {
+    launch_chi2_rows<CF, VC, NF, MX, 16, !T2>(a);
+  } else if (a.op == 2 && chi2.lanes == 4 && chi2.team) {
+    launch_chi2_rows<CF, VC, NF, MX, 4, !T2>(a);
+  } else if (a.op == 2 && chi2.lanes == 4) {
+    launch_chi2_rows<CF, VC, NF, MX, 4, false>(a);
   } else if (a.op == 2) {
     int blocks = (a.n + 255) / 256;
     hipLaunchKernelGGL((chi2_batch_kernel<CF, VC, NF, MX>), dim3(blocks), dim3(256), 0, a.stream, a.pts,
                        a.sum_w, a.n_data, a.n_filters, a.dof, a.params, a.n, a.chi2, a.dV);
+  } else if (a.op == 6 && chi2.lanes == 16) {
+    launch_curve_rows<CF, VC, NF, MX, 16>(a);
   } else if (a.op == 6) {
-    hipLaunchKernelGGL((curve_rows_kernel<CF, VC, NF, MX, 16>), dim3((a.n + 3) / 4), dim3(64), 0, a.stream, a.sum_w,
-                       a.n_filters, a.dof, a.grid, a.n_plot, a.params, a.n, a.dV, a.vmod);
+    if constexpr (!T2) launch_curve_rows<CF, VC, NF, MX, 4>(a);  // torque2: CURVE_ROWS_MAX models take 16
   } else if (a.op == 3) {
     int blocks = (a.n + 255) / 256;
     hipLaunchKernelGGL((model_curve_kernel<CF, VC, NF, MX>), dim3(blocks), dim3(256), 0, a.stream, a.pts,

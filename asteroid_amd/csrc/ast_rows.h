@@ -3,17 +3,25 @@
 // With one lane per model a launch of few models leaves the chip idle: 4096
 // models are 64 wavefronts on 1024 SIMDs, and a wavefront alone on its SIMD
 // issues one FP64 instruction every 4.3 cycles whatever its lanes hold, so
-// its time is its instruction count (620 per point of the torque form: 1.35
-// RK4 steps of 252 and 280 of brightness, 1.3 us).  Here LP = 16 or 4
+// its time is its instruction count (600 per point of the torque form: 1.35
+// RK4 steps of 248 and 263 of brightness, 1.3 us).  Here LP = 16 or 4
 // neighbouring lanes (a DPP row or quad) share one model and the count per
-// point falls to about 300 or 390:
+// point falls to about 300 or 350 (0.70 and 0.90 us):
 //
 //   * the two sine/cosine pairs of an RK4 stage (theta and psi; without
 //     torque theta and 2 psi) are one call, even lanes taking the first angle
-//     and odd lanes the second, the results handed round by DPP moves;
+//     and odd lanes the second, the results handed round by DPP moves (a step
+//     is then 197 instructions);
 //   * the brightness, which needs only the Euler angles at its point, runs
 //     once per LP points, lane j doing point j of the batch;
 //   * the chi^2 sums then take the batch's residuals in the points' order.
+//
+// Where SIMDs are still free, a team of wavefronts walks the models of one:
+// the Euler angles are a serial chain that nothing else has to wait in.  Their
+// wavefront is left 153 instructions a step (132 without torque); with torque
+// a second one integrates the angular velocity, which does not depend on the
+// angles, ahead of it, and another one follows with the brightness and the
+// sums (0.61 us per point; a 57-point chi^2 call of one model 93 -> 76 us).
 //
 // Every value comes from the same operations on the same operands as in
 // chi2_model, in the same order where order matters (the integration and the
@@ -33,6 +41,20 @@ __device__ long long dpp_mov_b64(long long old, long long src, int ctrl, int row
 // The table as vector loads read it (a generic pointer would make them FLAT
 // loads, which the table reads in LDS have to wait for).
 typedef __attribute__((address_space(1))) const PointRec* LanePtr;
+
+// A team's exchange buffers: 64 / LP models, each a row of LP lanes in every
+// one of its wavefronts.
+typedef double double2x __attribute__((ext_vector_type(2)));
+typedef __attribute__((address_space(3))) double2x* SpinPtr;
+template <bool TQ, int LP>
+struct TeamLds {
+  static constexpr int STEPS = LP == 16 ? 4 : 8;  // RK4 steps between two barriers
+  double2x spin[TQ ? 2 : 1][STEPS][64 / LP][6];   // angular velocities of a step's later stages and its end
+  double angle[2][LP][64];                        // of a point: theta, psi and phi in lanes 0, 1, 2 of a row
+};
+template <int VC, int LP>
+using TeamPtr = __attribute__((address_space(3))) TeamLds<VarF<VC>::TQ, LP>*;
+enum { ROLE_ALL, ROLE_ANGLES, ROLE_SPIN, ROLE_LIGHT };
 
 // As pin_sgpr, for a value a vector load gives: what was loaded before this
 // point is waited for here and not, over and over, at its uses in a loop.
@@ -66,6 +88,20 @@ AST_AI void unroll_lanes(const F& f) {
   }
 }
 
+// Stage `stage` of an RK4 step of the angular velocity w: from its value fw at
+// the stage to that at the next one, or at the last stage to the step's end in
+// w; sw sums the slopes.
+AST_AI void spin_stage(int stage, double* w, double* fw, double* sw, const double* mu, double hs, double h6) {
+  const double k[3] = {__builtin_fma(mu[0] * fw[1], fw[2], mu[3]), __builtin_fma(mu[1] * fw[2], fw[0], mu[4]),
+                       __builtin_fma(mu[2] * fw[0], fw[1], mu[5])};
+#pragma unroll
+  for (int j = 0; j < 3; ++j) {
+    sw[j] = stage == 0 ? k[j] : stage < 3 ? __builtin_fma(2.0, k[j], sw[j]) : sw[j] + k[j];
+    if (stage < 3) fw[j] = __builtin_fma(hs, k[j], w[j]);
+    else w[j] = __builtin_fma(h6, sw[j], w[j]);
+  }
+}
+
 // One RK4 step of the shared integration (cuda.c:348-372).  w holds the
 // angular velocity (torque form only), phi the first Euler angle and p the
 // lane's angle (theta on even lanes, psi on odd ones); sc the sine/cosine
@@ -74,12 +110,18 @@ AST_AI void unroll_lanes(const F& f) {
 // chi2_model's step; their order puts the next stage's table read as early as
 // its angle is known (the barrier keeps it there) and the angular velocity's
 // part of the stage behind it, so that a wavefront alone on its SIMD does not
-// wait for the read.
-template <bool TQ, int LP>
+// wait for the read.  With FED the angular velocities at the later stages and
+// the step's end are read from rec, where another wavefront left them.
+template <bool TQ, int LP, bool FED = false>
 AST_AI void rk4_shared(double* w, double& phi, double& p, double* sc, const double* mu, double mu02, bool odd,
-                       double h, double hh, double h6) {
+                       double h, double hh, double h6, SpinPtr rec = nullptr) {
   const double twice = odd ? 2.0 : 1.0;  // without torque the odd lanes' argument is 2 psi
   double sw[3] = {0, 0, 0}, fw[3] = {w[0], w[1], w[2]}, sphi, sp;
+  double2x fed[6];
+  if constexpr (FED) {
+#pragma unroll
+    for (int k = 0; k < 6; ++k) fed[k] = rec[k];
+  }
 #pragma unroll
   for (int stage = 0; stage < 4; ++stage) {
     double kphi, kp;
@@ -107,15 +149,15 @@ AST_AI void rk4_shared(double* w, double& phi, double& p, double* sc, const doub
     double ts, tc, s, c;
     astm::sctab_get(astm::sctab_index(kb), &ts, &tc);
     __builtin_amdgcn_sched_barrier(0);
-    if (TQ) {
-      const double k[3] = {__builtin_fma(mu[0] * fw[1], fw[2], mu[3]), __builtin_fma(mu[1] * fw[2], fw[0], mu[4]),
-                           __builtin_fma(mu[2] * fw[0], fw[1], mu[5])};
+    if constexpr (FED) {
 #pragma unroll
       for (int j = 0; j < 3; ++j) {
-        sw[j] = stage == 0 ? k[j] : stage < 3 ? __builtin_fma(2.0, k[j], sw[j]) : sw[j] + k[j];
-        if (stage < 3) fw[j] = __builtin_fma(hs, k[j], w[j]);
-        else w[j] = __builtin_fma(h6, sw[j], w[j]);
+        const int k = 3 * stage + j;
+        if (stage < 3) fw[j] = fed[k / 2][k % 2];
+        else w[j] = fed[k / 2][k % 2];
       }
+    } else if (TQ) {
+      spin_stage(stage, w, fw, sw, mu, hs, h6);
     }
     if (stage == 0) {
       sphi = kphi;
@@ -134,14 +176,43 @@ AST_AI void rk4_shared(double* w, double& phi, double& p, double* sc, const doub
   }
 }
 
+// The angular velocity's part of an RK4 step alone, its values at the later
+// stages and the end left in rec for rk4_shared.
+AST_AI void rk4_spin(double* w, const double* mu, double h, double hh, double h6, SpinPtr rec) {
+  double sw[3], fw[3] = {w[0], w[1], w[2]}, out[12];
+#pragma unroll
+  for (int stage = 0; stage < 4; ++stage) {
+    spin_stage(stage, w, fw, sw, mu, stage < 2 ? hh : h, h6);
+#pragma unroll
+    for (int j = 0; j < 3; ++j) out[3 * stage + j] = stage < 3 ? fw[j] : w[j];
+  }
+#pragma unroll
+  for (int k = 0; k < 6; ++k) rec[k] = double2x{out[2 * k], out[2 * k + 1]};
+}
+
 // chi2_model with LP lanes per model (same arguments, same results in every
 // lane of a model).  All lanes of a model must be active together.  With
 // FORM_PLOT vplot is the model's own curve (stride 1).
-template <class CF, int VC, int NF, bool MX, int FORM, int LP>
+//
+// ROLE other than ROLE_ALL is one wavefront's part of a team of two (without
+// torque) or three that walks the curve together, exchanging through `team`:
+//   ROLE_SPIN    the angular velocities, a chunk of TEAM_STEPS steps ahead,
+//   ROLE_ANGLES  the Euler angles, from those,
+//   ROLE_LIGHT   brightness and sums of the batch of points before.
+// All three run the same loops over the curve's steps and meet at a barrier
+// where ROLE_ANGLES starts a chunk (a batch's last chunk may be short, and a
+// batch without steps has one too) and once more at the end.  Both buffers
+// are used in turn: while chunk k is read chunk k + 1 is written; a batch's
+// angles are read between the next batch's first barrier and its second, and
+// written again from the first barrier after that on.
+template <class CF, int VC, int NF, bool MX, int FORM, int LP, int ROLE = ROLE_ALL>
 __device__ CF chi2_model_rows(const double* params, PointPtr pts, LanePtr pts_g, int n_data, int n_filters, int dof,
-                              const double* sum_w, CF* dV, double* vplot = nullptr, double dv0 = 0.0) {
+                              const double* sum_w, CF* dV, double* vplot = nullptr, double dv0 = 0.0,
+                              TeamPtr<VC, LP> team = nullptr) {
   using P = Pos<VC>;
   AST_VFLAGS(VC);
+  static_assert(ROLE == ROLE_ALL || !T2, "a team's models share their step counts");
+  constexpr int TEAM_STEPS = TeamLds<TQ, LP>::STEPS;
   static_assert(!(TR && (T2 || NU)), "PointRec.aux is the phase angle under TREND and the time otherwise");
   const int lane = (int)__lane_id() & (LP - 1);
   const bool odd = lane & 1;
@@ -218,7 +289,17 @@ __device__ CF chi2_model_rows(const double* params, PointPtr pts, LanePtr pts_g,
   double nx_h = pts_g[lane < n_data ? lane : n_data - 1].h;
   pin_vgpr(nx_steps);
   pin_vgpr(nx_h);
+  int left = 0;  // a team's: steps until the next barrier
+  int spin_buf = 0, angle_buf = 0;
+  const int row = (int)__lane_id() / LP;
+  if constexpr (ROLE == ROLE_ANGLES) spin_buf = 1;
+  if constexpr (ROLE == ROLE_LIGHT) __syncthreads();
   for (int i0 = 0; i0 < n_data; i0 += LP) {
+    if constexpr (ROLE == ROLE_ANGLES) {
+      __syncthreads();
+      spin_buf ^= 1;
+    }
+    left = TEAM_STEPS;
     const int m = n_data - i0 < LP ? n_data - i0 : LP;
     const int lane_steps = nx_steps;
     const uint64_t lane_h = astm::bits_of(nx_h);
@@ -246,6 +327,28 @@ __device__ CF chi2_model_rows(const double* params, PointPtr pts, LanePtr pts_g,
       double hh = 0.5 * h, h6 = 1 / 6.0 * h;  // as the table's
       if constexpr (SG) {
         if (nsteps < 0) begin(-1 - nsteps);
+      }
+      if constexpr (ROLE == ROLE_LIGHT) {
+        for (left -= nsteps > 0 ? nsteps : 0; left < 0; left += TEAM_STEPS) __syncthreads();
+        if constexpr (SG) {
+          if (lane == j) Fl = Fd;
+        }
+        continue;
+      }
+      if constexpr (ROLE == ROLE_ANGLES || ROLE == ROLE_SPIN) {
+        for (int l = 0; l < nsteps; ++l) {
+          if (left == 0) {
+            __syncthreads();
+            spin_buf ^= 1;
+            left = TEAM_STEPS;
+          }
+          const SpinPtr rec = team->spin[TQ ? spin_buf : 0][TEAM_STEPS - left][row];
+          if constexpr (ROLE == ROLE_ANGLES) rk4_shared<TQ, LP, TQ>(w, phi, p, sc, mu, mu02, odd, h, hh, h6, rec);
+          else rk4_spin(w, mu, h, hh, h6, rec);
+          --left;
+        }
+        if constexpr (ROLE == ROLE_ANGLES) team->angle[angle_buf][j][__lane_id()] = lane == 2 ? phi : p;
+        continue;
       }
       int nsub = 1;
       double t2_end = 0.0;
@@ -286,6 +389,22 @@ __device__ CF chi2_model_rows(const double* params, PointPtr pts, LanePtr pts_g,
     }
     pin_vgpr(nx_steps);
     pin_vgpr(nx_h);
+    if constexpr (ROLE == ROLE_ANGLES) {
+      angle_buf ^= 1;
+      continue;
+    }
+    if constexpr (ROLE == ROLE_SPIN || ROLE == ROLE_LIGHT) __syncthreads();
+    if constexpr (ROLE == ROLE_SPIN) {
+      spin_buf ^= 1;
+      continue;
+    }
+    if constexpr (ROLE == ROLE_LIGHT) {
+      const auto angle = &team->angle[angle_buf][lane][row * LP];
+      cth = lane < m ? angle[0] : 0.0;
+      cps = lane < m ? angle[1] : 0.0;
+      cphi = lane < m ? angle[2] : 0.0;
+      angle_buf ^= 1;
+    }
     // Brightness of the lane's point.
     double asc[4], a[3], b[3], c[3];
     astm::sincos_t(cth, &asc[0], &asc[1]);
@@ -343,6 +462,10 @@ __device__ CF chi2_model_rows(const double* params, PointPtr pts, LanePtr pts_g,
       }
     });
   }
+  if constexpr (ROLE == ROLE_ANGLES || ROLE == ROLE_SPIN) {
+    __syncthreads();
+    return CF(0.0);
+  }
   if constexpr (FORM == FORM_PLOT) return CF(0.0);
   if constexpr (NU)
     if (nu.failed) return CF(1e30);
@@ -353,6 +476,34 @@ __device__ CF chi2_model_rows(const double* params, PointPtr pts, LanePtr pts_g,
     all1[m] = NF == 1 ? sy[0] : lane_of<LP, m % LP>(sy[m / LP]);
   });
   return model_score<CF, VC, NF, FORM>(all2, all1, n_filters, dof, sum_w, dV, NU ? &nu : nullptr, mr);
+}
+
+// The parts of a team that do not depend on the form, the filters or the type
+// of the score: one copy for all kernels of a build.
+template <int VC, int LP, int ROLE>
+__device__ __attribute__((noinline)) void team_walk(const double* params, size_t stride, const PointRec* pts_g,
+                                                    int n_data, TeamPtr<VC, LP> team) {
+  constexpr int N = Pos<VC>::N;
+  const uint64_t pu = (uint64_t)(uintptr_t)pts_g;
+  const uint64_t plo = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)pu);
+  const uint64_t phi = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(pu >> 32));
+  const uintptr_t pa = (uintptr_t)((phi << 32) | plo);
+  n_data = __builtin_amdgcn_readfirstlane(n_data);
+  double prm[N];
+#pragma unroll
+  for (int i = 0; i < N; ++i) prm[i] = params[(size_t)i * stride];
+  chi2_model_rows<double, VC, 1, false, FORM_CHI2, LP, ROLE>(prm, (PointPtr)pa, (LanePtr)pa, n_data, 1, 0, nullptr,
+                                                             nullptr, nullptr, 0.0, team);
+}
+
+// What the wavefronts of a team other than its first do: wave 1 the Euler
+// angles, wave 2 (with torque) the angular velocities.
+template <int VC, int LP>
+__device__ inline void team_helper(int wave, const double* params, size_t stride, const PointRec* pts_g, int n_data,
+                                   TeamPtr<VC, LP> team) {
+  if (wave == 1) team_walk<VC, LP, ROLE_ANGLES>(params, stride, pts_g, n_data, team);
+  if constexpr (VarF<VC>::TQ)
+    if (wave == 2) team_walk<VC, LP, ROLE_SPIN>(params, stride, pts_g, n_data, team);
 }
 
 }  // namespace ast

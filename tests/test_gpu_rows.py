@@ -1,8 +1,9 @@
 """The evaluator with several lanes per model (ast_rows.h) against the oracle,
 bit for bit: chi^2 batches and fits at the sizes where the number of lanes per
-model changes (16 up to 4096 models, 4 up to 16384, then one), curves whose
-length leaves every kind of remainder in a batch of 16 or 4 points, curves on
-short grids, and a run whose groups end their stages in separate launches."""
+model or the use of teams changes (1024, 4096, 8192 and 16384 models), curves
+whose length leaves every kind of remainder in a batch of 16 or 4 points or in a
+team's chunk of steps, curves on short grids, and a run whose groups end their
+stages in separate launches."""
 import numpy as np
 import pytest
 
@@ -144,3 +145,82 @@ def test_every_build_on_four_lanes_and_one(name, groups):
         _same(chi2[0][a:a + n], want[0])
         if not v.nudge:  # delta_V of a failed NUDGE model is the caller's
             _same(chi2[1][a:a + n], want[1])
+
+
+@pytest.mark.parametrize("fits,group_size", [(256, 64), (2048, 256), (5120, 256)])  # 16 lanes, teams of 4, 4 or teams
+@pytest.mark.parametrize("name", list(BUILDS))
+def test_every_build_on_few_models(name, fits, group_size):
+    v = BUILDS[name](abi.PREC_FP64)
+    base = variants.make_variant(bool(v.torque), bool(v.bc), precision=abi.PREC_FP64) if v.n_seg > 1 else v
+    curve, truth = synth.make_curve(7, base, 61, 1.5, n_filters=2)
+    space = variants.default_model_space(v)
+    keep = {}
+    with api.Context(v) as ctx:
+        ctx.set_model_space(space)
+        if v.n_seg > 1:
+            keep["t_start"] = curve.mjd[0] - 0.01 + 1.5 * np.arange(v.n_seg) / v.n_seg
+            ctx.set_segments(keep["t_start"])
+        ctx.upload_curve(curve)
+        if v.nudge:
+            keep["minima"] = (curve.mjd[[9, 30]].astype(np.float32), curve.V[[9, 30]])
+            ctx.set_minima(*keep["minima"])
+        pb = oracle.Problem(space, curve, **keep)
+        run = dict(nstages=1, n_steps=4, eval_budget=space.n_params + 6)
+        ctx.rng_seed(8)
+        ctx.run(fits // group_size, group_size, **run)
+        got = ctx.fetch() + ctx.fetch_lanes()
+        p = _models(pb, 70)
+        n = len(p)
+        chi2 = ctx.chi2_batch(np.resize(p, (fits + n, p.shape[1])))
+        plots = [(n, 37, ctx.model_curve(p, n_plot=37))]
+        if v.n_seg > 1:  # a grid without a point in every segment is refused
+            with pytest.raises(api.AsteroidError):
+                ctx.model_curve(p[:3], n_plot=2)
+        else:
+            plots.append((3, 2, ctx.model_curve(p[:3], n_plot=2)))
+        many = ctx.model_curve(np.resize(p, (1024 + n, p.shape[1])), n_plot=19)
+    want = pb.run(fits // group_size, group_size, seed=8, form=oracle.CANON, n_threads=8, **run)
+    for g, k in zip(got, ("f", "params", "dV", "lane_f", "lane_nev", "lane_steps")):
+        _same(g, want[k])
+    want = pb.chi2(p)
+    last = (fits // n) * n
+    for a, m in ((0, n), (last - n, n), (last, fits + n - last)):
+        m = min(m, n)
+        _same(chi2[0][a:a + m], want[0][:m])
+        if not v.nudge:  # delta_V of a failed NUDGE model is the caller's
+            _same(chi2[1][a:a + m], want[1][:m])
+    a = (1024 // n) * n
+    plots += [(n, 19, [many[0]] + [g[k:k + n] for g in many[1:]]) for k in (0, a)]
+    for m, n_plot, got in plots:
+        t, vmod, f, dv = pb.model_curve(p[:m], n_plot=n_plot)
+        _same(got[0], t)
+        _same(got[2], f)
+        ok = f < 1e29  # a failed NUDGE model has no delta_V
+        _same(got[1][ok], vmod[ok])
+        _same(got[3][ok], dv[ok])
+
+
+@pytest.mark.parametrize("make", [variants.ls_torque, variants.bc_free], ids=["tq", "bc"])
+@pytest.mark.parametrize("n", [1023, 1024, 1025, 4095, 4096, 4097, 8192, 8193])
+def test_chi2_where_teams_begin_and_end(make, n):
+    v, curve, _, space, pb = _problem(make, "f32simplex", 18, 3, span=2.5)
+    p = _models(pb, 300)
+    with _ctx(v, space, curve) as ctx:
+        got = ctx.chi2_batch(np.resize(p, (n, p.shape[1])))
+    want = pb.chi2(p)
+    for g, w in zip(got, want):
+        _same(g, np.resize(w, (n,) + w.shape[1:]))
+
+
+@pytest.mark.parametrize("make", [variants.ls_torque, variants.bc_free], ids=["tq", "bc"])
+@pytest.mark.parametrize("groups,group_size,resident", [(30, 64, 3), (9, 256, 4), (30, 256, 8), (40, 256, 24)])
+def test_refilled_fits_on_teams(make, groups, group_size, resident):
+    v, curve, _, space, pb = _problem(make, "f32simplex", 18, 3, span=2.5)
+    run = dict(nstages=1, n_steps=12, eval_budget=24)
+    with _ctx(v, space, curve) as ctx:
+        ctx.rng_seed(4)
+        ctx.run(groups, group_size, resident_groups=resident, **run)
+        got = ctx.fetch() + ctx.fetch_lanes()
+    want = pb.run(groups, group_size, seed=4, form=oracle.CANON, n_threads=8, **run)
+    for g, k in zip(got, ("f", "params", "dV", "lane_f", "lane_nev", "lane_steps")):
+        _same(g, want[k])
