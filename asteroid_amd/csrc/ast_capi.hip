@@ -2353,8 +2353,9 @@ static LaunchArgs chi2_args(const ast_ctx* c, const double* params, int n, doubl
 }
 
 // Up to here inputs and results of a call go through pinned memory that the
-// kernel reads and writes in place: one model of 57 points takes 84 us a call
-// (the kernel 77), with three allocations and four copies it took 129.
+// kernel reads and writes in place: one model of 57 points takes 76 us a call
+// (the kernel 60); before, with the kernel at 77, 84 us, and with three
+// allocations and four copies 129.
 constexpr size_t IN_PLACE_BYTES = (size_t)256 << 10;
 // From here a chi^2 batch is copied and launched in two halves, each of at
 // least a wavefront for half of the SIMDs: 131072 models of 400 points 1610

@@ -1459,7 +1459,7 @@ __global__ __launch_bounds__(W == 4 ? 1024 : 256) __attribute__((amdgpu_waves_pe
 // --------------------------------------------------------- launch interface
 struct LaunchArgs {
   int op;  // 0 init groups, 1 fit ticks, 2 chi2 batch, 3 model curve, 4 and 5 RMSD,
-           // 6 the grid of a model curve (16 lanes per model, after its chi2 batch)
+           // 6 the grid of a model curve (several lanes per model, after its chi2 batch)
   int precision;
   hipStream_t stream;
   // fit: descriptors of the groups of this launch (device), their count, G
