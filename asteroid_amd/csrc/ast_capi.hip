@@ -2357,10 +2357,11 @@ static LaunchArgs chi2_args(const ast_ctx* c, const double* params, int n, doubl
 // (the kernel 60); before, with the kernel at 77, 84 us, and with three
 // allocations and four copies 129.
 constexpr size_t IN_PLACE_BYTES = (size_t)256 << 10;
-// From here a chi^2 batch is copied and launched in two halves, each of at
-// least a wavefront for half of the SIMDs: 131072 models of 400 points 1610
-// -> 1305 us a call.  (Four quarters by asynchronous copies took 2130: a
-// pageable copy of 3 MB costs 400 us.)
+// With more than a wavefront for each SIMD a chi^2 batch is copied and
+// launched in two halves: 131072 models of 400 points 1610 -> 1305 us a call,
+// 81920 1428 -> 1210.  Up to there a half takes as long as the whole (65536
+// models 936 us, in halves 1152).  (Four quarters by asynchronous copies took
+// 2130 for the 131072: a pageable copy of 3 MB costs 400 us.)
 constexpr int SPLIT_MODELS = 65536;
 
 // chi^2 of n models in place (pinned memory `pin`).
@@ -2412,7 +2413,7 @@ int ast_chi2_batch(ast_ctx* c, const double* params, int n, double* chi2, double
            *dd = sc.carve<double>((size_t)n * NF);
     // A large batch in two launches on two streams: the second half is copied
     // in while the first computes.
-    parts = n >= SPLIT_MODELS ? 2 : 1;
+    parts = n > SPLIT_MODELS ? 2 : 1;
     const size_t per = (((size_t)n + parts - 1) / parts + 255) & ~(size_t)255;
     for (int k = 0; k < parts && he == hipSuccess; ++k) {
       const size_t a0 = k * per, m = std::min(per, (size_t)n - a0);

@@ -224,3 +224,13 @@ def test_refilled_fits_on_teams(make, groups, group_size, resident):
     want = pb.run(groups, group_size, seed=4, form=oracle.CANON, n_threads=8, **run)
     for g, k in zip(got, ("f", "params", "dV", "lane_f", "lane_nev", "lane_steps")):
         _same(g, want[k])
+
+
+@pytest.mark.parametrize("n", [65536, 65537, 131071])  # in one launch, in two halves
+def test_chi2_batches_in_halves(n):
+    v, curve, _, space, pb = _problem(variants.ls_torque, "fp64", 18, 2)
+    p = _models(pb, 301)
+    with _ctx(v, space, curve) as ctx:
+        got = ctx.chi2_batch(np.resize(p, (n, p.shape[1])))
+    for g, w in zip(got, pb.chi2(p)):
+        _same(g, np.resize(w, (n,) + w.shape[1:]))
