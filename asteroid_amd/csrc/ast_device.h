@@ -349,31 +349,6 @@ __device__ inline void body_axes(const SpinFrame<T>& F, T sf, T cf, T st, T ctt,
   c[2] = fmx(-a[1], b[0], a[0] * b[1]);
 }
 
-// ODE right-hand side.  With FIRST the sin/cos of theta (and psi) come from
-// sc[] (those of the state, shared with the body axes), else they are computed.
-template <bool TQ, bool FIRST>
-__device__ inline void ode(const double* y, double* f, const double* mu, double mu02, const double* sc) {
-  if (TQ) {  // cuda.c:46-58
-    double s5, c5, s4, c4;
-    if (FIRST) { s4 = sc[0]; c4 = sc[1]; s5 = sc[2]; c5 = sc[3]; }
-    else { astm::sincos_t(y[5], &s5, &c5); astm::sincos_t(y[4], &s4, &c4); }
-    f[0] = __builtin_fma(mu[0] * y[1], y[2], mu[3]);
-    f[1] = __builtin_fma(mu[1] * y[2], y[0], mu[4]);
-    f[2] = __builtin_fma(mu[2] * y[0], y[1], mu[5]);
-    f[3] = astm::div_rn(__builtin_fma(y[1], c5, y[0] * s5), s4);
-    f[4] = __builtin_fma(-y[1], s5, y[0] * c5);
-    f[5] = __builtin_fma(-f[3], c4, y[2]);
-  } else {   // cuda.c:69-75
-    double s2, c2, s1, c1;
-    astm::sincos_t(2.0 * y[2], &s2, &c2);
-    if (FIRST) { s1 = sc[0]; c1 = sc[1]; }
-    else astm::sincos_t(y[1], &s1, &c1);
-    f[0] = mu[0] * __builtin_fma(-mu[2], c2, mu[1]);
-    f[1] = (mu02 * s1) * s2;
-    f[2] = c1 * (mu[0] - f[0]);
-  }
-}
-
 typedef __attribute__((address_space(4))) const PointRec* PointPtr;
 
 // An empty asm that takes a wave-uniform value in scalar registers and
@@ -503,6 +478,71 @@ struct ModelConsts {
 };
 
 #define AST_AI __device__ __attribute__((always_inline)) inline
+
+// Stage `stage` of an RK4 step of the angular velocity w: from its value fw at
+// the stage to that at the next one, or at the last stage to the step's end in
+// w; sw sums the slopes.
+AST_AI void spin_stage(int stage, double* w, double* fw, double* sw, const double* mu, double hs, double h6) {
+  const double k[3] = {__builtin_fma(mu[0] * fw[1], fw[2], mu[3]), __builtin_fma(mu[1] * fw[2], fw[0], mu[4]),
+                       __builtin_fma(mu[2] * fw[0], fw[1], mu[5])};
+#pragma unroll
+  for (int j = 0; j < 3; ++j) {
+    sw[j] = stage == 0 ? k[j] : stage < 3 ? __builtin_fma(2.0, k[j], sw[j]) : sw[j] + k[j];
+    if (stage < 3) fw[j] = __builtin_fma(hs, k[j], w[j]);
+    else w[j] = __builtin_fma(h6, sw[j], w[j]);
+  }
+}
+
+// One RK4 step (cuda.c:348-372 with the right-hand sides of cuda.c:46-58, 69-75)
+// of y = angular velocity and Euler angles, without torque the angles alone.
+// sc holds the sines and cosines of theta and psi (without torque of theta and
+// 2 psi) at the step's start and is replaced by those at its end.
+// A wavefront alone on its SIMD, as a search of 57344 fits has them, waits for
+// whatever the compiler puts right behind a read of the table: seven
+// instructions, of a round trip of about 30, four times a step.  So a stage
+// reads for theta as soon as its angle is known, before psi's slope and its
+// division, then for psi, and only then does the rest: the angular velocity,
+// the slopes' sums, the reductions (the barriers keep it so).
+template <bool TQ>
+AST_AI void rk4_step(double* y, double* sc, const double* mu, double mu02, double h, double hh, double h6) {
+  constexpr int A = TQ ? 3 : 0;  // phi, theta and psi are y[A], y[A + 1], y[A + 2]
+  double sw[3], fw[3] = {y[0], y[1], y[2]}, sum[3];
+#pragma unroll
+  for (int stage = 0; stage < 4; ++stage) {
+    const double hs = stage < 2 ? hh : h;
+    double k[3], a[2], kb[2], ts[2], tc[2];
+    // the angle of slope k[j] for the next stage or, at the last, the step's end
+    auto angle = [&](int j) {
+      if (stage < 3) return __builtin_fma(hs, k[j], y[A + j]);
+      y[A + j] = __builtin_fma(h6, sum[j] + k[j], y[A + j]);
+      return y[A + j];
+    };
+    if (TQ) k[1] = __builtin_fma(-fw[1], sc[2], fw[0] * sc[3]);
+    else k[1] = (mu02 * sc[0]) * sc[2];
+    a[0] = angle(1);
+    kb[0] = astm::sincos_t_k(a[0]);
+    astm::sctab_get(astm::sctab_index(kb[0]), &ts[0], &tc[0]);
+    __builtin_amdgcn_sched_barrier(0);
+    if (TQ) {
+      k[0] = astm::div_rn(__builtin_fma(fw[1], sc[3], fw[0] * sc[2]), sc[0]);
+      k[2] = __builtin_fma(-k[0], sc[1], fw[2]);
+    } else {
+      k[0] = mu[0] * __builtin_fma(-mu[2], sc[3], mu[1]);
+      k[2] = sc[1] * (mu[0] - k[0]);
+    }
+    a[1] = TQ ? angle(2) : 2.0 * angle(2);
+    kb[1] = astm::sincos_t_k(a[1]);
+    astm::sctab_get(astm::sctab_index(kb[1]), &ts[1], &tc[1]);
+    __builtin_amdgcn_sched_barrier(0);
+    if (TQ) spin_stage(stage, y, fw, sw, mu, hs, h6);
+    if (stage == 3) y[A] = __builtin_fma(h6, sum[0] + k[0], y[A]);
+#pragma unroll
+    for (int j = 0; j < 3; ++j)
+      if (stage < 3) sum[j] = stage == 0 ? k[j] : __builtin_fma(2.0, k[j], sum[j]);
+    astm::sincos_t_end(a[0], kb[0], ts[0], tc[0], &sc[0], &sc[1]);
+    astm::sincos_t_end(a[1], kb[1], ts[1], tc[1], &sc[2], &sc[3]);
+  }
+}
 
 // Body axes at one observation (FP64, both forms) from the spin frame, phi
 // and the sines and cosines of theta (sc[0..1]) and, with torque, of psi
@@ -844,15 +884,15 @@ __device__ CF chi2_model(const double* params, PointPtr pts, int n_data, int n_f
   const double Ii = __builtin_fma(ct, ct, 1.0) / den;
   const double Is_inv = 1.0 / Is;
   const double Ii_inv = 1.0 / Ii;
-  constexpr int NODE = TQ ? 6 : 3;
   SpinFrame<double> Fd;
   double mu[6];
   double mu02 = 0.0;
   double y[6];
-  // sin/cos of the current theta and psi, shared by the next RK4 step's
-  // first stage and the body axes at the observation.
+  // sin/cos of the current theta and psi (without torque 2 psi), shared by the
+  // next RK4 step's first stage and the body axes at the observation.
   double sc[4];
   begin_rotation<VC>(params, 0, Is_inv, Ii_inv, Is, Ii, Fd, y, mu, mu02, sc);
+  if (!TQ) astm::sincos_t(2.0 * y[2], &sc[2], &sc[3]);
   double phi, theta, psi;
   ModelConsts K{0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
   if constexpr (RO) {
@@ -912,7 +952,10 @@ __device__ CF chi2_model(const double* params, PointPtr pts, int n_data, int n_f
       // rotation starts again from the segment's own parameters (cuda.c:163-252
       // inside the segment loop); the shape, and so the brightness
       // constants, are shared.
-      if (nsteps < 0) begin_rotation<VC>(params, -1 - nsteps, Is_inv, Ii_inv, Is, Ii, Fd, y, mu, mu02, sc);
+      if (nsteps < 0) {
+        begin_rotation<VC>(params, -1 - nsteps, Is_inv, Ii_inv, Is, Ii, Fd, y, mu, mu02, sc);
+        if (!TQ) astm::sincos_t(2.0 * y[2], &sc[2], &sc[3]);
+      }
     }
     int nsub = 1;
     double t2_end = 0.0;
@@ -942,27 +985,7 @@ __device__ CF chi2_model(const double* params, PointPtr pts, int n_data, int n_f
         switched = true;
       }
     }
-    for (int l = 0; l < nsteps; ++l) {  // RK4, cuda.c:348-372
-      double f[6], K4[6], s[6];
-      ode<TQ, true>(y, K4, mu, mu02, sc);
-#pragma unroll
-      for (int j = 0; j < NODE; ++j) { s[j] = K4[j]; f[j] = __builtin_fma(hh, K4[j], y[j]); }
-      ode<TQ, false>(f, K4, mu, mu02, sc);
-#pragma unroll
-      for (int j = 0; j < NODE; ++j) { s[j] = __builtin_fma(2.0, K4[j], s[j]); f[j] = __builtin_fma(hh, K4[j], y[j]); }
-      ode<TQ, false>(f, K4, mu, mu02, sc);
-#pragma unroll
-      for (int j = 0; j < NODE; ++j) { s[j] = __builtin_fma(2.0, K4[j], s[j]); f[j] = __builtin_fma(h, K4[j], y[j]); }
-      ode<TQ, false>(f, K4, mu, mu02, sc);
-#pragma unroll
-      for (int j = 0; j < NODE; ++j) y[j] = __builtin_fma(h6, s[j] + K4[j], y[j]);
-      if (TQ) {
-        astm::sincos_t(y[4], &sc[0], &sc[1]);
-        astm::sincos_t(y[5], &sc[2], &sc[3]);
-      } else {
-        astm::sincos_t(y[1], &sc[0], &sc[1]);
-      }
-    }
+    for (int l = 0; l < nsteps; ++l) rk4_step<TQ>(y, sc, mu, mu02, h, hh, h6);
     }  // sub-intervals
     if (TQ) { phi = y[3]; theta = y[4]; psi = y[5]; }
     else { phi = y[0]; theta = y[1]; psi = y[2]; }

@@ -88,26 +88,12 @@ AST_AI void unroll_lanes(const F& f) {
   }
 }
 
-// Stage `stage` of an RK4 step of the angular velocity w: from its value fw at
-// the stage to that at the next one, or at the last stage to the step's end in
-// w; sw sums the slopes.
-AST_AI void spin_stage(int stage, double* w, double* fw, double* sw, const double* mu, double hs, double h6) {
-  const double k[3] = {__builtin_fma(mu[0] * fw[1], fw[2], mu[3]), __builtin_fma(mu[1] * fw[2], fw[0], mu[4]),
-                       __builtin_fma(mu[2] * fw[0], fw[1], mu[5])};
-#pragma unroll
-  for (int j = 0; j < 3; ++j) {
-    sw[j] = stage == 0 ? k[j] : stage < 3 ? __builtin_fma(2.0, k[j], sw[j]) : sw[j] + k[j];
-    if (stage < 3) fw[j] = __builtin_fma(hs, k[j], w[j]);
-    else w[j] = __builtin_fma(h6, sw[j], w[j]);
-  }
-}
-
 // One RK4 step of the shared integration (cuda.c:348-372).  w holds the
 // angular velocity (torque form only), phi the first Euler angle and p the
 // lane's angle (theta on even lanes, psi on odd ones); sc the sine/cosine
 // pairs at the step's start (theta and psi, without torque theta and 2 psi),
-// replaced by those at its end.  The same operations as ode() and
-// chi2_model's step; their order puts the next stage's table read as early as
+// replaced by those at its end.  The same operations as
+// rk4_step's; their order puts the next stage's table read as early as
 // its angle is known (the barrier keeps it there) and the angular velocity's
 // part of the stage behind it, so that a wavefront alone on its SIMD does not
 // wait for the read.  With FED the angular velocities at the later stages and
