@@ -561,7 +561,7 @@ def main_plot(args):
     out.update({"kernel_ms": ms, "model_points_per_s_kernel": pts / (ms / 1e3),
                 "roofline": {"bound": "valu", "achieved": round(achieved, 3), "peak": FP64_PEAK_TFLOPS,
                              "unit": "TFLOP/s", "frac": round(achieved / FP64_PEAK_TFLOPS, 4),
-                             "kernel": "model_curve_kernel", "flop_per_model": round(f_model, 1),
+                             "kernel": "curve_team_kernel", "flop_per_model": round(f_model, 1),
                              "lanes": n_models},
                 "single_model": {"kernel_ms": one_ms, "call_ms": one_wall * 1e3,
                                  "periodogram_ms": pg_wall * 1e3, "periodogram_kernel_ms": pg_ms,
