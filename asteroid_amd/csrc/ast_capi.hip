@@ -944,6 +944,17 @@ int job_reduce(DevJob& j, hipStream_t s) {
 // All fits of the job have ended.
 bool job_complete(const DevJob& j) { return j.groups_done >= j.n_workers; }
 
+// Launch cycles a job needs at most.  Every tick completes one evaluation of
+// each running simplex; a stage needs at most (N+1) + n_steps*(N+2) of them,
+// and with refill a lane runs its share of the fits one after another.  With
+// several lanes per model a stage ends between launches, so each stage may
+// leave the rest of one unused.
+long cycles_needed(const DevJob& j) {
+  const double N = j.space.n_params, per_stage = (N + 1) + (double)j.rp.n_steps * (N + 2);
+  const double rounds = std::ceil((double)j.rp.n_groups / (double)j.n_workers) + 1.0;
+  return (long)((per_stage * j.rp.nstages * rounds + 16.0) / j.ticks) + j.rp.nstages + 4;
+}
+
 // Kernel class of a job: one fit-kernel instantiation (variant, filter
 // capacity, precision form).
 int class_of(const ast_variant& v, int n_filters) {
@@ -1658,14 +1669,9 @@ int batch_run(ast_ctx* c, const std::vector<const ast_job*>& jobs, int G, double
     j.t_submit = j.t_admit = t0;
     run.push_back(&j);
   }
-  // Every tick completes one evaluation of each running simplex; a stage
-  // needs at most (N+1) + n_steps*(N+2) of them.
   long max_cycles = 0;
-  for (DevJob* j : run) {
-    const double per_stage = (double)(j->space.n_params + 1) + (double)j->rp.n_steps * (j->space.n_params + 2);
-    const long mc = (long)((per_stage * j->rp.nstages + 16.0) / j->ticks) + 4;
-    if (mc > max_cycles) max_cycles = mc;
-  }
+  if (!rc)
+    for (DevJob* j : run) max_cycles = std::max(max_cycles, cycles_needed(*j));
   for (long L = 0; !rc; ++L) {
     bool all = true;
     for (DevJob* j : run) all = all && job_complete(*j);
@@ -2204,12 +2210,7 @@ int ast_run_begin(ast_ctx* c, const ast_run_cfg* rc) {
   c->last_launches = 0;
   c->last_evals = 0;
   c->last_points = 0;
-  // Every tick completes one evaluation of each running simplex; a stage
-  // needs at most (N+1) + n_steps*(N+2) of them, and with refill a lane runs
-  // its share of the fits one after another.
-  const double per_stage = (double)(c->space.n_params + 1) + (double)rc->n_steps * (c->space.n_params + 2);
-  const double rounds = std::ceil((double)fits / (double)lanes) + 1.0;
-  c->run_max_cycles = (long)((per_stage * rc->nstages * rounds + 16.0) / ticks) + 4;
+  c->run_max_cycles = cycles_needed(j);
   c->run_cycles = 0;
   c->run_graphs = rc->use_graphs != 0;
   c->run_active = true;
