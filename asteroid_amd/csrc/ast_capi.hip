@@ -1222,13 +1222,16 @@ int set_device(ast_ctx* c) {
 
 // One cycle: one fit-kernel launch per kernel class over every running
 // group of every job of that class, every stream drained at the end; adds
-// the cycle's kernel time (the longest stream).
-int run_cycle_once(ast_ctx* c, std::vector<DevJob*>& jobs, double* kernel_ms, int* launches, bool graphs);
+// the cycle's kernel time (the longest stream).  With one_lane every class
+// runs its fit_kernel, however few the fits are.
+int run_cycle_once(ast_ctx* c, std::vector<DevJob*>& jobs, double* kernel_ms, int* launches, bool graphs,
+                   bool one_lane);
 
 // A failed cycle may leave kernels in flight: drain the device before the
 // caller frees anything they use.
-int run_cycle(ast_ctx* c, std::vector<DevJob*>& jobs, double* kernel_ms, int* launches, bool graphs = false) {
-  int rc = run_cycle_once(c, jobs, kernel_ms, launches, graphs);
+int run_cycle(ast_ctx* c, std::vector<DevJob*>& jobs, double* kernel_ms, int* launches, bool graphs = false,
+              bool one_lane = false) {
+  int rc = run_cycle_once(c, jobs, kernel_ms, launches, graphs, one_lane);
   if (rc) (void)hipDeviceSynchronize();
   return rc;
 }
@@ -1355,7 +1358,8 @@ int cycle_graph(ast_ctx* c, std::vector<DevJob*>* members, const bool* used_s, i
   return 0;
 }
 
-int run_cycle_once(ast_ctx* c, std::vector<DevJob*>& jobs, double* kernel_ms, int* launches, bool graphs) {
+int run_cycle_once(ast_ctx* c, std::vector<DevJob*>& jobs, double* kernel_ms, int* launches, bool graphs,
+                   bool one_lane) {
   std::vector<DevJob*> members[MAX_CLASSES];
   bool used_s[NSTREAMS] = {false};
   // A job's time in this cycle, alone: its evaluation rounds times the cost of
@@ -1375,7 +1379,8 @@ int run_cycle_once(ast_ctx* c, std::vector<DevJob*>& jobs, double* kernel_ms, in
     load[j->cls] = std::max(load[j->cls], t);
     fits += (double)j->n_workers * c->pool.G * (t / longest);
   }
-  const int64_t side = (int64_t)std::ceil(fits);  // the classes of a cycle run side by side
+  // the classes of a cycle run side by side
+  const int64_t side = std::max<int64_t>((int64_t)std::ceil(fits), one_lane ? ROWS_MAX + 1 : 0);
   if (side <= ROWS_MAX) merge_classes(members, load);
   int stream[MAX_CLASSES];
   assign_streams(load, stream);
@@ -1604,8 +1609,10 @@ int make_job(ast_ctx* c, const ast_job* job, int G, std::unique_ptr<DevJob>* out
 // Upload `jobs` into slots 0.., run them in shared cycles and collect their
 // results (results may be null).  cycle_limit > 0 stops after that many
 // cycles (the autotuner's fixed work); 0 runs every job to completion.
+// one_lane: as run_cycle_once.
 int batch_run(ast_ctx* c, const std::vector<const ast_job*>& jobs, int G, double work, long cycle_limit,
-              ast_result* results, double* kernel_ms, int* launches, bool graphs, int schedule = 0) {
+              ast_result* results, double* kernel_ms, int* launches, bool graphs, int schedule = 0,
+              bool one_lane = false) {
   const int n_jobs = (int)jobs.size();
   std::vector<std::unique_ptr<DevJob>> J(n_jobs);
   std::vector<CurveH> curves(n_jobs);
@@ -1681,7 +1688,7 @@ int batch_run(ast_ctx* c, const std::vector<const ast_job*>& jobs, int G, double
       rc = AST_E_STATE;
       break;
     }
-    rc = run_cycle(c, run, kernel_ms, launches, graphs);
+    rc = run_cycle(c, run, kernel_ms, launches, graphs, one_lane);
   }
   if (rc) (void)hipDeviceSynchronize();
   int64_t ev_tot = 0, pts_tot = 0;
@@ -2783,8 +2790,9 @@ int ast_autotune(ast_ctx* c, const ast_job* jobs, int n_jobs, const ast_batch_cf
         int launches = 0;
         double t = 0;
         // the same jobs from the same start each time: identical work, so the
-        // kernel times compare the register budgets alone
-        RETIF(batch_run(c, kv.second, G, work, cycles, nullptr, &t, &launches, false));
+        // kernel times compare the register budgets alone.  By fit_kernel, which
+        // has the three, also where so few fits would take several lanes each.
+        RETIF(batch_run(c, kv.second, G, work, cycles, nullptr, &t, &launches, false, 0, true));
         if (pass == 0 || t < ms[w]) ms[w] = t;
       }
     }

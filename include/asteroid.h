@@ -493,7 +493,10 @@ int ast_run_jobs(ast_ctx* ctx, const ast_job* jobs, int n_jobs, const ast_batch_
  * filter capacity, precision) has three builds of the fitting kernel with
  * different register budgets: 4 waves per SIMD (128 VGPRs, groups of up to
  * 1024 simplexes), 3 (168 VGPRs) and 2 (256 VGPRs), the last two for groups
- * of up to 256.  They compute exactly the same results.  ast_autotune runs
+ * of up to 256.  They compute exactly the same results.  Launches of 16384
+ * fits or fewer run other kernels, with several lanes per fit and a budget of
+ * their own; ast_autotune times the three builds whatever the jobs' fits, for
+ * the larger launches.  It runs
  * `cycles` launch cycles of the given jobs (one class at a time, from the
  * same start for every budget, so the work is identical) at each budget,
  * twice, interleaved, keeping each budget's faster time; it keeps the
