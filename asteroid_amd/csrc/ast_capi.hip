@@ -34,6 +34,7 @@
 
 #include "../../include/asteroid.h"
 #include "ast_kernels.h"
+#include "ast_memory.h"
 
 namespace ast {
 template <int VC> hipError_t launch_variant(const LaunchArgs& a);
@@ -112,10 +113,10 @@ double ms_since(Clock::time_point t0) {
 }
 
 template <class T>
-int dev_alloc(T** p, size_t count) {
+int dev_alloc(Memory& mem, T** p, size_t count) {
   *p = nullptr;
   if (count == 0) count = 1;
-  HIPCHK(hipMalloc((void**)p, count * sizeof(T)));
+  HIPCHK(mem.alloc((void**)p, count * sizeof(T)));
   return 0;
 }
 template <class T>
@@ -123,95 +124,6 @@ void dev_free(T*& p) {
   if (p) (void)hipFree(p);
   p = nullptr;
 }
-
-// -------------------------------------------------------- memory kept
-// A context's device and pinned host memory between calls.  An allocation and
-// a release cost a call about 15 us each (a release waits for the device as
-// well), three to fourteen of them a chi^2 batch or a job.
-//  * blocks: device blocks given back by finished calls and jobs, taken again
-//    by later ones of up to their size; at most KEEP_BYTES, the rest is
-//    released.  A call gives its blocks back when nothing on the device uses
-//    them any more.
-//  * pin: pinned host memory that kernels read and write in place, for inputs
-//    and results so small that a copy's latency is most of its time.
-// Calls on a context come from one thread at a time (the scheduler's while it
-// serves), so there is no lock.
-struct Memory {
-  static constexpr size_t KEEP_BYTES = (size_t)256 << 20, PIN_BYTES = (size_t)4 << 20;
-  std::vector<std::pair<size_t, void*>> blocks;
-  size_t kept = 0;
-  char* pin = nullptr;
-
-  int take(size_t bytes, void** p, size_t* cap) {
-    bytes = (bytes + 4095) & ~(size_t)4095;
-    int best = -1;
-    for (int k = 0; k < (int)blocks.size(); ++k)  // the smallest that holds it, of at most twice its size
-      if (blocks[k].first >= bytes && blocks[k].first <= 2 * bytes &&
-          (best < 0 || blocks[k].first < blocks[best].first))
-        best = k;
-    if (best >= 0) {
-      *cap = blocks[best].first;
-      *p = blocks[best].second;
-      kept -= *cap;
-      blocks.erase(blocks.begin() + best);
-      return 0;
-    }
-    *p = nullptr;
-    *cap = bytes;
-    if (hipMalloc(p, bytes) == hipSuccess) return 0;
-    (void)hipGetLastError();
-    release();  // what is kept may be what is missing
-    HIPCHK(hipMalloc(p, bytes));
-    return 0;
-  }
-  void give(void* p, size_t cap) {
-    if (!p) return;
-    if (kept + cap > KEEP_BYTES || blocks.size() >= 64) {
-      (void)hipFree(p);
-      return;
-    }
-    blocks.push_back({cap, p});
-    kept += cap;
-  }
-  void release() {
-    for (auto& b : blocks) (void)hipFree(b.second);
-    blocks.clear();
-    kept = 0;
-  }
-  // Pinned memory for `bytes`, or null (too many, or none to be had): the
-  // caller copies instead.
-  char* pinned(size_t bytes) {
-    if (bytes > PIN_BYTES) return nullptr;
-    if (!pin && hipHostMalloc((void**)&pin, PIN_BYTES, hipHostMallocDefault) != hipSuccess) {
-      (void)hipGetLastError();
-      pin = nullptr;
-    }
-    return pin;
-  }
-  void close() {
-    release();
-    if (pin) (void)hipHostFree(pin);
-    pin = nullptr;
-  }
-};
-
-// One device block of a call, given back at its end; carve() hands out its
-// parts, in the order and sizes of the reserve() calls before it.
-struct Scratch {
-  Memory& mem;
-  void* base = nullptr;
-  size_t cap = 0, need = 0, at = 0;
-  explicit Scratch(Memory& m) : mem(m) {}
-  ~Scratch() { mem.give(base, cap); }
-  static size_t padded(size_t bytes) { return (bytes + 255) & ~(size_t)255; }
-  template <class T> void reserve(size_t n) { need += padded(n * sizeof(T)); }
-  int take() { return mem.take(need ? need : 256, &base, &cap); }
-  template <class T> T* carve(size_t n) {
-    T* p = (T*)((char*)base + at);
-    at += padded(n * sizeof(T));
-    return p;
-  }
-};
 
 // ------------------------------------------------------------ validation
 // The variant codes built (one kernel family each), indexed by variant_index.
@@ -635,12 +547,12 @@ void pool_free(Pool& p) {
   p.free_slots.clear();
 }
 
-int pool_alloc(Pool& p, size_t nf, int G, int n_params) {
+int pool_alloc(Pool& p, Memory& mem, size_t nf, int G, int n_params) {
   pool_free(p);
   if (n_params <= 0 || n_params > AST_MAX_PARAMS) return AST_E_ARG;
   const size_t P = (size_t)n_params;
   int rc = 0;
-#define ALLOC(ptr, type, count) if (!rc) rc = dev_alloc((type**)&(ptr), (count))
+#define ALLOC(ptr, type, count) if (!rc) rc = dev_alloc(mem, (type**)&(ptr), (count))
   ALLOC(p.X, double, (P + 1) * P * nf);
   ALLOC(p.F, double, (P + 1) * nf);
   ALLOC(p.X0, double, P * nf);
@@ -843,7 +755,7 @@ int job_upload_typed(DevJob& j, const Pool& pool, const CurveH& C, const double*
                o_nev = part(sizeof(int32_t) * fits), o_steps = part(sizeof(int32_t) * fits), cleared = at;
   const size_t o_fit_f = part(sizeof(CF) * fits), o_fit_params = part(j.refill ? sizeof(double) * fits * N : 0),
                o_fit_dV = part(j.refill ? sizeof(double) * fits * C.n_filters : 0);
-  RETIF(mem.take(at, &j.block, &j.block_cap));
+  HIPCHK(mem.take(at, &j.block, &j.block_cap));
   char* const dev = (char*)j.block;
   j.pts = (PointRec*)(dev + o_pts);
   j.sum_w = (double*)(dev + o_sum_w);
@@ -1093,7 +1005,7 @@ int pgram_counts(hipStream_t s, Memory& mem, const hipEvent_t* ev, const std::ve
   sc.reserve<double>(n);
   sc.reserve<int32_t>((size_t)n_chunks * PGRAM_BINS);
   sc.reserve<int32_t>(PGRAM_BINS);
-  RETIF(sc.take());
+  HIPCHK(sc.take());
   double* td = sc.carve<double>(n);
   int32_t* part = sc.carve<int32_t>((size_t)n_chunks * PGRAM_BINS);
   int32_t* sum = sc.carve<int32_t>(PGRAM_BINS);
@@ -1251,7 +1163,7 @@ int class_batch_update(ast_ctx* c, int k, const std::vector<DevJob*>& members) {
   if (bytes > cb.cap) {
     dev_free(cb.d_descs);
     cb.cap = 0;
-    RETIF(dev_alloc((char**)&cb.d_descs, bytes));
+    RETIF(dev_alloc(c->mem, (char**)&cb.d_descs, bytes));
     cb.cap = bytes;
   }
   std::vector<unsigned char> h(bytes);
@@ -1454,7 +1366,7 @@ int run_cycle_once(ast_ctx* c, std::vector<DevJob*>& jobs, double* kernel_ms, in
 int ensure_streams(ast_ctx* c, size_t fits, size_t groups) {
   if (c->rng_cap < fits) {
     uint32_t* nr = nullptr;
-    RETIF(dev_alloc(&nr, fits));
+    RETIF(dev_alloc(c->mem, &nr, fits));
     HIPCHK(hipMemset(nr, 0, fits * sizeof(uint32_t)));
     if (c->rng) HIPCHK(hipMemcpy(nr, c->rng, c->rng_cap * sizeof(uint32_t), hipMemcpyDeviceToDevice));
     dev_free(c->rng);
@@ -1465,9 +1377,9 @@ int ensure_streams(ast_ctx* c, size_t fits, size_t groups) {
   if (c->best_cap < groups || !c->best_f) {
     void* nf = nullptr;
     double *np = nullptr, *nd = nullptr;
-    int rc = dev_alloc((char**)&nf, (size_t)cf * groups);
-    if (!rc) rc = dev_alloc(&np, groups * AST_MAX_PARAMS);
-    if (!rc) rc = dev_alloc(&nd, groups * AST_MAX_FILTERS);
+    int rc = dev_alloc(c->mem, (char**)&nf, (size_t)cf * groups);
+    if (!rc) rc = dev_alloc(c->mem, &np, groups * AST_MAX_PARAMS);
+    if (!rc) rc = dev_alloc(c->mem, &nd, groups * AST_MAX_FILTERS);
     if (rc) { dev_free(nf); dev_free(np); dev_free(nd); return rc; }
     std::vector<char> hf((size_t)cf * groups);
     for (size_t g = 0; g < groups; ++g) {
@@ -1627,7 +1539,7 @@ int batch_run(ast_ctx* c, const std::vector<const ast_job*>& jobs, int G, double
   }
   RETIF(set_device(c));
   if ((size_t)c->pool.n_slots < groups || c->pool.G != G || c->pool.P < n_params)
-    RETIF(pool_alloc(c->pool, groups * G, G, n_params));
+    RETIF(pool_alloc(c->pool, c->mem, groups * G, G, n_params));
   c->last_groups = 0;  // the pool's rows no longer hold an ast_run's lanes
   // Work of one simplex of each job: an upper bound of its evaluations (the
   // budget, or the step limit) times the cost of one.
@@ -1820,6 +1732,8 @@ void serve_loop(ast_ctx* c) {
       std::lock_guard<std::mutex> lk(S.mu);
       for (auto& j : S.resident)
         if (!j->cancelled && j->status == AST_OK) run.push_back(j.get());
+      if (S.cfg.hbm_budget_bytes > 0)  // the blocks kept for later jobs count as well
+        c->mem.trim((size_t)std::max<int64_t>(0, S.cfg.hbm_budget_bytes - S.resident_bytes));
     }
     if (!run.empty()) {
       double ms = 0;
@@ -1896,7 +1810,7 @@ int rmsd_run(ast_ctx* c, const ast_rmsd_cfg& cfg, RmsdOut* out) {
   sc.reserve<float>((size_t)ng * N);
   sc.reserve<float>((size_t)ng * N);
   sc.reserve<int32_t>((size_t)ng * 2);
-  RETIF(sc.take());
+  HIPCHK(sc.take());
   Space<CF>* sp = sc.carve<Space<CF>>(1);
   RmsdRef<CF>* ref = sc.carve<RmsdRef<CF>>(1);
   double* p0 = sc.carve<double>((size_t)N);
@@ -2006,6 +1920,7 @@ int ast_ctx_create(ast_ctx** out, const ast_variant* v, int device) {
   if (!c) return AST_E_NOMEM;
   c->device = device;
   c->v = *v;
+  c->mem.open(device);
   hipError_t e = hipSetDevice(device);
   for (int k = 0; k < NSTREAMS && e == hipSuccess; ++k) {
     e = hipStreamCreateWithFlags(&c->streams[k], hipStreamNonBlocking);
@@ -2077,8 +1992,8 @@ int ast_upload_curve(ast_ctx* c, const ast_obs* obs, int n_data, int n_filters, 
   RETIF(set_device(c));
   dev_free(c->pts);
   dev_free(c->sum_w);
-  RETIF(dev_alloc(&c->pts, C.pts.size()));
-  RETIF(dev_alloc(&c->sum_w, (size_t)AST_MAX_FILTERS));
+  RETIF(dev_alloc(c->mem, &c->pts, C.pts.size()));
+  RETIF(dev_alloc(c->mem, &c->sum_w, (size_t)AST_MAX_FILTERS));
   HIPCHK(hipMemcpy(c->pts, C.pts.data(), sizeof(PointRec) * C.pts.size(), hipMemcpyHostToDevice));
   HIPCHK(hipMemcpy(c->sum_w, C.sum_w, sizeof(double) * AST_MAX_FILTERS, hipMemcpyHostToDevice));
   c->curve = std::move(C);
@@ -2174,7 +2089,7 @@ int ast_run_begin(ast_ctx* c, const ast_run_cfg* rc) {
   const size_t fits = (size_t)rc->n_groups * G, lanes = (size_t)workers * G;
   RETIF(ensure_streams(c, fits, rc->n_groups));
   if (c->pool.nf < lanes || c->pool.G != G || c->pool.P < c->space.n_params)
-    RETIF(pool_alloc(c->pool, lanes, G, c->space.n_params));
+    RETIF(pool_alloc(c->pool, c->mem, lanes, G, c->space.n_params));
   // The reference path is one job that borrows the context's streams and bests.
   if (c->ref_job) job_free(*c->ref_job, c->mem);
   c->ref_job.reset(new DevJob());
@@ -2416,7 +2331,7 @@ int ast_chi2_batch(ast_ctx* c, const double* params, int n, double* chi2, double
     sc.reserve<double>((size_t)n * N);
     sc.reserve<double>((size_t)n);
     sc.reserve<double>((size_t)n * NF);
-    RETIF(sc.take());
+    HIPCHK(sc.take());
     double *pd = sc.carve<double>((size_t)n * N), *cd = sc.carve<double>((size_t)n),
            *dd = sc.carve<double>((size_t)n * NF);
     // A large batch in two launches on two streams: the second half is copied
@@ -2471,8 +2386,8 @@ int ast_copy_bandwidth(ast_ctx* c, int64_t bytes, int reps, double* bytes_per_s)
   RETIF(set_device(c));
   const size_t n = (size_t)bytes / 16;
   uint4 *src = nullptr, *dst = nullptr;
-  int rc = dev_alloc(&src, n);
-  if (!rc) rc = dev_alloc(&dst, n);
+  int rc = dev_alloc(c->mem, &src, n);
+  if (!rc) rc = dev_alloc(c->mem, &dst, n);
   if (rc) { dev_free(src); dev_free(dst); return rc; }
   hipStream_t s = c->streams[0];
   const unsigned blocks = (unsigned)std::min<size_t>((n + 255) / 256, 8192);
@@ -2597,7 +2512,7 @@ int ast_model_curve(ast_ctx* c, const double* params, int n, const ast_ephem3* e
     sc.reserve<double>((size_t)n * nf);
     sc.reserve<double>(n_vmod);
   }
-  RETIF(sc.take());
+  HIPCHK(sc.take());
   PointRec* const gd = sc.carve<PointRec>(recs);
   double* const pd = out ? (double*)out : sc.carve<double>((size_t)n * np);
   double* const cd = out ? pd + (size_t)n * np : sc.carve<double>((size_t)n);
@@ -2697,7 +2612,7 @@ int ast_serve_start(ast_ctx* c, const ast_serve_cfg* cfg) {
     return AST_E_ARG;
   RETIF(set_device(c));
   size_t fits = (size_t)(cfg->max_resident_fits / G) * G;
-  RETIF(pool_alloc(c->pool, fits, G, P));
+  RETIF(pool_alloc(c->pool, c->mem, fits, G, P));
   c->serve.reset(new Serve());
   c->serve->cfg = *cfg;
   c->serve->cfg.group_size = G;
