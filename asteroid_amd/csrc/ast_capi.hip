@@ -2351,9 +2351,10 @@ int ast_chi2_batch(ast_ctx* c, const double* params, int n, double* chi2, double
       he = hipStreamSynchronize(c->streams[k]);
       if (he == hipSuccess) he = hipMemcpy(chi2 + a0, cd + a0, sizeof(double) * m, hipMemcpyDeviceToHost);
       if (he == hipSuccess) he = hipMemcpy(dV + a0 * NF, dd + a0 * NF, sizeof(double) * m * NF, hipMemcpyDeviceToHost);
-      float t = 0;  // from the first launch's start to this one's end
+      float t = 0, idle = 0;  // from the first launch's start to this one's end, without the time between them
       if (he == hipSuccess) he = hipEventElapsedTime(&t, c->ev0[0], c->ev1[k]);
-      ms = std::max(ms, t);
+      if (k > 0 && he == hipSuccess) he = hipEventElapsedTime(&idle, c->ev1[0], c->ev0[k]);
+      ms = std::max(ms, t - std::max(0.0f, idle));
     }
     if (he != hipSuccess) (void)hipDeviceSynchronize();  // before the block is given back
   }
@@ -2523,9 +2524,12 @@ int ast_model_curve(ast_ctx* c, const double* params, int n, const ast_ephem3* e
   if (out) std::memcpy(pd, params, sizeof(double) * n * np);
   else he = hipMemcpyAsync(pd, params, sizeof(double) * n * np, hipMemcpyHostToDevice, s);
   LaunchArgs a = chi2_args(c, pd, n, cd, dd, s);
-  if (he == hipSuccess) he = hipEventRecord(c->ev0[0], s);
   const bool rows = n <= CURVE_ROWS_MAX;
-  if (rows && he == hipSuccess) he = dispatch(c->v, a);  // the observations' part, while the grid is built
+  if (rows) {  // the observations' part, while the grid is built
+    if (he == hipSuccess) he = hipEventRecord(c->ev0[1], s);
+    if (he == hipSuccess) he = dispatch(c->v, a);
+    if (he == hipSuccess) he = hipEventRecord(c->ev1[1], s);
+  }
   int g0 = 0;
   const int rc = make_grid(c->v, c->curve, *eph, n_plot, grid, t ? t : tg.data(), c->seg_t, &g0);
   if (rc) {
@@ -2537,6 +2541,7 @@ int ast_model_curve(ast_ctx* c, const double* params, int n, const ast_ephem3* e
   a.n_plot = n_plot;
   a.vmod = vd;
   if (he == hipSuccess) he = hipMemcpyAsync(gd, grid, sizeof(PointRec) * recs, hipMemcpyHostToDevice, s);
+  if (he == hipSuccess) he = hipEventRecord(c->ev0[0], s);
   if (he == hipSuccess) he = dispatch(c->v, a);
   if (he == hipSuccess) he = hipEventRecord(c->ev1[0], s);
   if (!out) {
@@ -2545,8 +2550,9 @@ int ast_model_curve(ast_ctx* c, const double* params, int n, const ast_ephem3* e
     if (he == hipSuccess) he = hipMemcpyAsync(vmod, vd, sizeof(double) * n_vmod, hipMemcpyDeviceToHost, s);
   }
   if (he == hipSuccess) he = hipStreamSynchronize(s);
-  float ms = 0;
+  float ms = 0, ms_obs = 0;
   if (he == hipSuccess) he = hipEventElapsedTime(&ms, c->ev0[0], c->ev1[0]);
+  if (rows && he == hipSuccess) he = hipEventElapsedTime(&ms_obs, c->ev0[1], c->ev1[1]);
   if (he != hipSuccess) {
     (void)hipDeviceSynchronize();
     snprintf(g_hip_err, sizeof g_hip_err, "%s (model curve)", hipGetErrorString(he));
@@ -2559,8 +2565,8 @@ int ast_model_curve(ast_ctx* c, const double* params, int n, const ast_ephem3* e
   }
   for (int k = 0; k < n && g0 > 0; ++k)
     for (int i = 0; i < g0; ++i) vmod[(size_t)k * n_plot + i] = std::nan("");
-  c->last_ms = ms;
-  c->last_launches = 1;
+  c->last_ms = ms + ms_obs;
+  c->last_launches = rows ? 2 : 1;
   c->last_evals = n;
   c->last_points = (int64_t)n * (c->curve.n_data + n_plot);
   return AST_OK;
@@ -2583,7 +2589,7 @@ int ast_periodogram(ast_ctx* c, const double* t, const double* vm, int n, int n_
   RETIF(set_device(c));
   const hipEvent_t ev[2] = {c->ev0[0], c->ev1[0]};
   RETIF(pgram_counts(c->streams[0], c->mem, ev, tm, &counts, &c->last_ms));
-  c->last_launches = tm.size() >= 2 ? 1 : 0;
+  c->last_launches = tm.size() >= 2 ? 2 : 0;
   pgram_clusters(counts, n_clusters, cl_fr, cl_H);
   return AST_OK;
 }

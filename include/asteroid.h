@@ -377,8 +377,11 @@ typedef struct {
 int ast_rmsd(ast_ctx* ctx, const ast_rmsd_cfg* cfg, float* par_min, float* par_max, int64_t* n_tot,
              int64_t* n_bad, double* f0, double* f1);
 
-/* Timing of the last ast_run / ast_chi2_batch, from HIP events on the
- * context's stream: total kernel milliseconds and the number of launches. */
+/* Timing of the last ast_run, ast_chi2_batch, ast_model_curve, ast_rmsd,
+ * ast_periodogram or ast_run_jobs, from HIP events on the context's streams:
+ * total kernel milliseconds (without host work or copies between launches)
+ * and the number of launches.  In a run's cycle a launch is a kernel class's
+ * (with several lanes per fit, its fits' kernel and its stage ends'). */
 int ast_last_timing(ast_ctx* ctx, double* kernel_ms, int* launches);
 
 /* Algorithmic counts of the last ast_run: chi^2 evaluations and
