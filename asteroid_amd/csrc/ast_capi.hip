@@ -2503,7 +2503,7 @@ int ast_model_curve(ast_ctx* c, const double* params, int n, const ast_ephem3* e
   char* const out = pin && out_bytes <= IN_PLACE_BYTES && grid_bytes + out_bytes <= Memory::PIN_BYTES
                         ? pin + grid_bytes : nullptr;
   std::vector<PointRec> grid_v(pin ? 0 : recs);
-  std::vector<double> tg(t ? 0 : n_plot);
+  const std::unique_ptr<double[]> tg(new double[n_plot]);  // the caller's t is written on success only
   PointRec* const grid = pin ? (PointRec*)pin : grid_v.data();
   Scratch sc(c->mem);
   sc.reserve<PointRec>(recs);
@@ -2531,7 +2531,7 @@ int ast_model_curve(ast_ctx* c, const double* params, int n, const ast_ephem3* e
     if (he == hipSuccess) he = hipEventRecord(c->ev1[1], s);
   }
   int g0 = 0;
-  const int rc = make_grid(c->v, c->curve, *eph, n_plot, grid, t ? t : tg.data(), c->seg_t, &g0);
+  const int rc = make_grid(c->v, c->curve, *eph, n_plot, grid, tg.get(), c->seg_t, &g0);
   if (rc) {
     (void)hipStreamSynchronize(s);
     return rc;
@@ -2563,6 +2563,7 @@ int ast_model_curve(ast_ctx* c, const double* params, int n, const ast_ephem3* e
     std::memcpy(dV, dd, sizeof(double) * n * nf);
     std::memcpy(vmod, vd, sizeof(double) * n_vmod);
   }
+  if (t) std::memcpy(t, tg.get(), sizeof(double) * n_plot);
   for (int k = 0; k < n && g0 > 0; ++k)
     for (int i = 0; i < g0; ++i) vmod[(size_t)k * n_plot + i] = std::nan("");
   c->last_ms = ms + ms_obs;
