@@ -46,12 +46,18 @@ class Curve:
         return len(self.mjd)
 
     def obs_array(self):
-        arr = (abi.Obs * self.n_data)()
-        if not self.n_data:
+        n = self.n_data
+        arr = (abi.Obs * n)()
+        if not n:
             return arr
         rec = np.frombuffer(arr, dtype=_OBS)  # a view: filled column by column
-        rec["mjd"], rec["V"], rec["w"], rec["filter"] = self.mjd, self.V, self.w, self.filter
-        rec["E"], rec["S"] = self.E, self.S
+        for name in ("mjd", "V", "w", "filter", "E", "S"):
+            column = np.asarray(getattr(self, name))[:n]  # of a longer one its first n
+            if name in "ES":
+                column = column[:, :3]
+            if column.shape != rec[name].shape:  # a shorter one is not repeated
+                raise IndexError(f"{name}: {column.shape} for {n} observations")
+            rec[name] = column
         return arr
 
     def ephem3(self):
