@@ -1722,7 +1722,10 @@ void serve_loop(ast_ctx* c) {
     for (size_t k = 0; k < admitted.size(); ++k) {
       DevJob& j = *admitted[k];
       int rc = serve_admit(c, S, j, admitted_in[k].first, admitted_in[k].second);
-      if (rc) j.status = rc;
+      if (rc) {
+        j.status = rc;
+        (void)hipDeviceSynchronize();  // its clears may be in flight, and its block goes to the next job
+      }
       j.t_admit = Clock::now();
       std::lock_guard<std::mutex> lk(S.mu);
       S.resident.push_back(std::move(admitted[k]));
