@@ -498,13 +498,24 @@ struct Machine {
   // with pointers read through memory every load of the simplex was waited
   // for by itself: 110 us per round of 64-lane FP64 fits of 11 parameters,
   // 370 us with the chip full, of 580 and 2900 us.)
+  //
+  // The loop has one exit, and in the SEGMENT builds `more` goes through a
+  // register the compiler cannot see through, so that it does not make several
+  // again from what it knows of `more`.  With several it keeps, per exit, the
+  // mask of the lanes that took it in a lane of a spill register; and ROCm 7.2's
+  // hipcc declares that register without a value at the head of the block that
+  // adds to the mask, inside the loop, so that it may give it to other spills
+  // for the rest of a pass.  It did in the FP64 build of four segments with
+  // torque and BC (40 parameters), whose fits then never ended; in ten other
+  // SEGMENT builds the register happened to stay free.  (In every build the
+  // register costs 0.5% of 2^18 mixed fits and 0.9% of re-optimised BC fits.)
   __device__ void advance(LaneRegs<CF>& R, CF val, bool has_result) {
     const CF GAMMA = 2.0, RHO = 0.5, SIGMA = 0.5;  // asteroid.h:240-242
-    bool more = has_result || R.phase == PH_START;
+    int more = has_result || R.phase == PH_START;
     CF xv[N];
     while (more) {
       renew();
-      more = false;
+      more = 0;
       bool over = false;
       if (R.phase == PH_START) {
         start(R, xv);
@@ -593,7 +604,7 @@ struct Machine {
         if (propose(xv)) {
           if (R.phase == PH_SHRINK_NEXT) R.phase = PH_SHRINK;
         } else {  // outside the hard limits
-          more = true;
+          more = 1;
           if (R.phase == PH_INIT) {
             R.failed = 1;
             R.phase = PH_BEGIN;
@@ -605,6 +616,7 @@ struct Machine {
           }
         }
       }
+      if constexpr (VarF<VC>::SG) pin_vgpr(more);
     }
   }
 };
