@@ -879,8 +879,8 @@ int class_of(const ast_variant& v, int n_filters) {
 // Streams of a cycle's classes.  load[k] is class k's time alone (0: not in
 // the cycle); the longest class first, each to the stream with the least so
 // far.  Two classes on one stream run one after the other: with the class
-// number modulo 4 the two longest of a batch of 11 curves did: 129 ms for the
-// batch against 98 with this and the fits weighted below.
+// number modulo 4 two batches of 11 curves take 77.7 and 73.5 ms against 64.7 and
+// 59.8, and two sets of 8 served requests 54.7 and 51.1 against 45.1 and 43.3.
 void assign_streams(const double* load, int* stream) {
   std::vector<int> order;
   for (int k = 0; k < MAX_CLASSES; ++k)
@@ -1182,8 +1182,9 @@ int class_batch_update(ast_ctx* c, int k, const std::vector<DevJob*>& members) {
 // their filter capacity only share the launch of the larger one (which keeps
 // a fit's values as they are: the sums of filters a job does not have are not
 // used), while there are too many.  A class more than streams makes a cycle
-// up to twice as long: 8 served requests in 5 classes took 58 ms, in 4 they take
-// 44.
+// up to twice as long: two sets of 8 served requests in 5 classes and more take
+// 60.6 and 56.9 ms, in 4 they take 45.1 and 43.3 (two batches of 11 curves the
+// same either way).
 void merge_classes(std::vector<DevJob*>* members, double* load) {
   for (;;) {
     int n = 0, to = -1, from = -1;
@@ -2279,15 +2280,14 @@ static LaunchArgs chi2_args(const ast_ctx* c, const double* params, int n, doubl
 }
 
 // Up to here inputs and results of a call go through pinned memory that the
-// kernel reads and writes in place: one model of 57 points takes 76 us a call
-// (the kernel 60); before, with the kernel at 77, 84 us, and with three
-// allocations and four copies 129.
+// kernel reads and writes in place: one model of 57 points takes 74 us a call
+// (the kernel 59), with four copies from and to a kept block 106.
 constexpr size_t IN_PLACE_BYTES = (size_t)256 << 10;
 // With more than a wavefront for each SIMD a chi^2 batch is copied and
-// launched in two halves: 131072 models of 400 points 1610 -> 1305 us a call,
-// 81920 1428 -> 1210.  Up to there a half takes as long as the whole (65536
-// models 936 us, in halves 1152).  (Four quarters by asynchronous copies took
-// 2130 for the 131072: a pageable copy of 3 MB costs 400 us.)
+// launched in two halves: 131072 models of 400 points 1514 -> 1275 us a call,
+// 81920 1257 -> 1148, 262144 3094 -> 2487.  Up to there a half takes as long as
+// the whole (65536 models 821 us, in halves 1113).  Four quarters take 2025 us
+// for the 131072, whose quarters leave half the SIMDs idle, and 2273 for 262144.
 constexpr int SPLIT_MODELS = 65536;
 
 // chi^2 of n models in place (pinned memory `pin`).

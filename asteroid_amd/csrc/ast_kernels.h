@@ -868,7 +868,11 @@ __device__ inline void store_lane(const SlotBufs<CF>& B, size_t fit, size_t fo, 
 
 // One evaluation with LP lanes per model (chi2_model_rows), for the kernels
 // below: parameters at PRM[i * stride], delta_V to DV[m * dv_stride].  Out of
-// line, so that a kernel class has one copy of it for its kernels.
+// line, so that a kernel class has one copy of it for its kernels.  Being
+// called by fit_kernel too, the copies without a team are compiled for 128
+// registers; copies of their own budget for the other kernels measured the same
+// (256 to 16384 models, with and without torque and torque2: chi^2 between 3%
+// less and 2% more time, fits within 2%).
 template <class CF, int VC, int NF, bool MX, int LP, int ROLE = ROLE_ALL>
 __device__ __attribute__((noinline)) CF eval_rows(const double* PRM, size_t stride, CF* DV, size_t dv_stride,
                                                    const PointRec* pts_g, int n_data, int n_filters, int dof,
@@ -972,11 +976,14 @@ void fit_kernel(const GroupDesc<CF>* descs, SlotBufs<CF> B) {
     // enough of the group's fits have ended to leave a wavefront without one,
     // the others' points are dealt to the first lanes, whichever fit they
     // belong to (a fit's values do not depend on the lane), and the chi^2 goes
-    // back through LDS.  Fits that stop at an evaluation budget still end
-    // within 12 rounds of each other (a shrink is finished): 224 groups, two
-    // stages of 50 evaluations, 78 -> 72 ms; 2^18 fits of 100, mixed, 215 -> 209.
+    // back through LDS.  Fits that stop at an evaluation budget end within
+    // about N + 1 rounds of each other (12 with LS and torque: the last step's
+    // shrink is finished); those that converge or fail end earlier, and with
+    // refill each at its own time.  224 groups, two stages of 50 evaluations
+    // 74.4 -> 69.3 ms; 2^18 fits of 100, mixed, 212 -> 202; of 4800 the same.
     // With the chip's SIMDs not shared (groups of 65536 fits at most), few enough
-    // points take 4 or 16 lanes each (the two-stage search above: 72 -> 66 ms).
+    // points take 4 or 16 lanes each: the two-stage search 69.3 -> 64.4 ms, 260
+    // groups of 64 fits and 60 evaluations 41.7 -> 36.1.
     const bool spread = (size_t)gridDim.x * G <= 65536;
     const int lp = spread && pending * 16 <= G ? 16 : spread && pending * 4 <= G ? 4 : 1;
     const bool pack = pending <= G - 64 || lp > 1;
@@ -1031,8 +1038,8 @@ void fit_kernel(const GroupDesc<CF>* descs, SlotBufs<CF> B) {
 }
 
 // ---------------------------------------------------- several lanes per model
-// Registers for one or two waves per SIMD: these kernels run where the chip
-// is not full.
+// Registers for one or two waves per SIMD for what is inlined (the simplex's
+// set-up): these kernels run where the chip is not full.
 #define AST_ROWS_BOUNDS __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 2)))
 
 // chi2_batch_kernel with LP lanes per model, 64 / LP models per workgroup (of
@@ -1503,19 +1510,33 @@ struct LaunchArgs {
 // wavefronts (three with torque, of which the first is idle half the time)
 // find a SIMD each; the model cut in two parts (torque2) has no teams, its
 // step counts being the model's own.
-// Kernel time at 16 / 4 / 1 lanes without teams, LS + torque, 400 points over 3
-// days, FP64 -- chi^2: 64 models 279 / 363 / 530 us, 4096 346 / 376 / 533, 6144
-// 588 / 371 / 533, 16384 1132 / 423 / 533, 24576 - / 679 / 539; fits of 30
-// evaluations: 4096 15.3 / 17.9 / 38.4 ms, 16384 54.6 / 22.3 / 39.7, 24576
-// - / 37.3 / 39.8.
-// Teams of 16 / 4 lanes -- torque: chi^2 64 models 245 / 260 us, 1024 262 / 265,
-// 2048 - / 268, 4096 - / 279 (without 346), 6144 - / 345 (371), 12288 - / 397
-// (401); fits 1024 11.6 / 12.9 ms (13.0), 4096 - / 13.3 (15.3), 6144 - / 23.5
-// (18.6).  Without torque, where only the brightness is taken off: chi^2 1024
-// 292 / 306 us (301), 4096 - / 318 (345), 8192 - / 341 (405), 16384 - / 437
-// (442); fits 1024 12.2 / 13.9 ms (13.0), 8192 - / 16.1 (19.6), 12288 - / 26.2
-// (21.6), but re-optimised fits of 818 points on 3328 lanes 45.5 against 44.0,
-// since a wavefront then runs 16 simplexes' bookkeeping instead of 4.
+// Kernel time with 16-lane teams / 16 lanes / 4-lane teams / 4 lanes / one lane
+// (LS, 400 points over 3 days, FP64; the form taken in brackets):
+//   chi^2, torque, us        fits of 30 evaluations, torque, ms
+//     64 [244] 277 257 341 511    256 [11.1] 12.1 12.3 14.6 19.5
+//   1024 [261] 292 264 345 515   1024 [11.6] 12.9 12.7 15.9 20.1
+//   2048 342 307 [267] 346 515   2048 21.3 13.6 [12.8] 16.0 20.1
+//   4096 431 326 [272] 346 512   4096 41.0 16.1 [13.3] 16.1 20.1
+//   6144 775 549 332 [348] 515   6144 58.2 24.2 23.2 [18.9] 20.1
+//  12288 - 811 369 [365] 520    12288 - - 35.4 [21.8] 20.2
+//  16384 - 1037 599 [375] 524   16384 - - 46.3 [22.8] 20.3
+//  24576 - - 827 636 [538]      24576 - - 67.4 33.6 [20.6]
+//   chi^2, no torque, us     fits, no torque, ms
+//   1024 [207] 216 212 281 461   1024 8.1 [8.4] 9.1 11.6 16.2
+//   2048 244 229 [214] 287 462   2048 8.5 [8.9] 9.2 11.7 16.3
+//   4096 265 243 [215] 293 459   4096 16.0 [9.5] 9.5 12.0 16.2
+//   8192 695 409 [245] 296 464   8192 30.6 17.5 [10.3] 13.2 16.3
+//  12288 927 576 255 [302] 465  12288 - - 17.1 [14.1] 16.4
+//  16384 - 731 302 [309] 468    16384 - - 18.8 [14.9] 16.3
+//  24576 - - 551 491 [475]      24576 - - 26.3 23.1 [16.6]
+// The lines are the fits' with torque, and are taken for chi^2 too: its 4-lane
+// teams would still be 4% ahead at 6144 and 8192.  Without torque, where only
+// the brightness is taken off, chi^2 teams end with the fits' although they are
+// ahead up to 16384 (16% at 12288), and 16-lane teams are not built for the
+// fits: ahead by 4% up to 2048 only (a BC search by 4 to 6%).  From 12288 fits on
+// one lane is ahead in the table since its last fits share wavefronts, which is
+// much of 30 evaluations; of 200, fits with torque take 81 and 84 ms on 4 lanes
+// at 12288 and 16384, 111 and 112 on one, and 153 and 113 at 20480.
 struct RowShape {
   int lanes;
   bool team;
@@ -1529,8 +1550,13 @@ constexpr RowShape fit_shape(bool torque, bool torque2, int64_t n) {
   if (torque && !torque2) return chi2_shape(torque, torque2, n);
   return {n <= 4096 ? 16 : n <= 16384 ? 4 : 1, !torque2 && n > 4096 && n <= 8192};
 }
-constexpr int64_t ROWS_MAX = 16384;       // more models take a lane each
-constexpr int CURVE_ROWS_MAX = 4096;      // more model curves
+constexpr int64_t ROWS_MAX = 16384;  // more models take a lane each
+// More model curves take a lane each.  The line is where 4-lane teams with
+// torque still find a SIMD for each wavefront; curves of 2000 points take 1.29
+// ms up to there and 2.75 beyond (4-lane teams 1.65 for 4097, 1.71 for 8192, 1.85
+// for 12288 and 2.87 against 2.83 for 16384; without torque 1.24, 1.33, 1.68 and
+// 1.98 against 2.63 to 2.71), as before there were several lanes per model.
+constexpr int CURVE_ROWS_MAX = 4096;
 
 template <class CF, int VC, int NF, bool MX, int LP, bool TEAM>
 void launch_chi2_rows(const LaunchArgs& a) {

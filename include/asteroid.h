@@ -299,16 +299,17 @@ int ast_fetch_lanes(ast_ctx* ctx, double* f_last, int64_t* n_evals, int64_t* n_s
 
 /* The evaluator alone (chi2one, cuda.c:81-1011): chi^2 and the per-filter
  * delta_V of n parameter vectors (physical units, n*n_params doubles),
- * computed one model per GPU lane.  chi2 has n entries, dV n*n_filters. */
+ * computed one model per GPU lane, up to 16384 models by 4 or 16 lanes each
+ * (the same values).  chi2 has n entries, dV n*n_filters. */
 int ast_chi2_batch(ast_ctx* ctx, const double* params, int n, double* chi2, double* dV);
 
 /* ast_chi2_batch without any device allocation.  No counterpart in the
  * reference: it is for callers that cannot allocate device memory (code
  * under HIP graph capture, tight serving loops, harnesses that forbid
  * hipMalloc).  The models, chi^2 and delta_V are staged in a fixed device
- * array of the library (one per GPU, 6.4 MB, held until the process ends)
- * instead of buffers allocated per call; results are those of
- * ast_chi2_batch.  At most AST_NOALLOC_MAX_MODELS models per call (more is
+ * array of the library (one per GPU, 6.4 MB, held until the process ends), or,
+ * up to 256 KB, in the context's pinned memory (allocated with the context);
+ * results are those of ast_chi2_batch.  At most AST_NOALLOC_MAX_MODELS models per call (more is
  * AST_E_ARG).  All contexts on one GPU share that array: calls that overlap
  * on one GPU (from several threads or contexts) race and must be
  * serialised by the caller.  The context must have its model space and
@@ -335,7 +336,8 @@ int ast_copy_bandwidth(ast_ctx* ctx, int64_t bytes, int reps, double* bytes_per_
  * observations; its interior E,S come from `eph`, the 3-point ephemeris
  * (read_data.c:345; required for every variant).  Outputs, caller-owned:
  * t (n_plot grid times, may be NULL), vmod (n*n_plot, model k's curve at
- * vmod[k*n_plot ...]), chi2 (n), dV (n*n_filters).  One model per GPU lane. */
+ * vmod[k*n_plot ...]), chi2 (n), dV (n*n_filters).  Up to 4096 models by 4
+ * or 16 GPU lanes each, more by one (the same values). */
 int ast_model_curve(ast_ctx* ctx, const double* params, int n, const ast_ephem3* eph, int n_plot,
                     double* t, double* vmod, double* chi2, double* dV);
 
