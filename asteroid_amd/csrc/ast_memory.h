@@ -111,12 +111,13 @@ struct Memory {
 
  private:
   int device = -1;
+  // Never destroyed: a program may close its contexts as it exits.
   static std::mutex& all_mu() {
-    static std::mutex m;
+    static std::mutex& m = *new std::mutex;
     return m;
   }
   static std::vector<Memory*>& all() {  // the open ones
-    static std::vector<Memory*> v;
+    static std::vector<Memory*>& v = *new std::vector<Memory*>;
     return v;
   }
   // (with the lock) the oldest blocks first

@@ -51,6 +51,15 @@ static void keep(Memory& m, size_t n) {
   m.give(p, cap);
 }
 
+// Closed after main, by the destructor of an object older than the registry.
+struct Late {
+  Memory* m = nullptr;
+  ~Late() {
+    if (m) m->close();
+    delete m;
+  }
+} late;
+
 int main() {
   Memory a, b, c;
   a.open(0);
@@ -119,6 +128,8 @@ int main() {
   assert(used[0] == 0 && used[1] == 100 * MIB);
   c.close();
   assert(live.empty());
+  late.m = new Memory;
+  late.m->open(0);
   puts("memory ok");
 }
 """
